@@ -105,9 +105,15 @@ int fx_ctx_create(int device, uint64_t hbm_budget_bytes, fx_ctx** out) {
   size_t fr = 0, tot = 0;
   (void)hipMemGetInfo(&fr, &tot);
   c->budget = hbm_budget_bytes ? hbm_budget_bytes : static_cast<uint64_t>(fr / 10 * 9);
+  if (hipHostMalloc(&c->host_pinned, 4096, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
+    (void)hipStreamDestroy(c->stream);
+    delete c;
+    return fail(nullptr, FX_EDEVICE, "hipHostMalloc failed");
+  }
   if (hipMalloc(&c->scalars, 4096) != hipSuccess ||
       hipMalloc(&c->pimy_params, sizeof(fx::PimyParams) * fx::kMaxPointMaterials) != hipSuccess) {
     if (c->scalars) (void)hipFree(c->scalars);
+    (void)hipHostFree(c->host_pinned);
     (void)hipStreamDestroy(c->stream);
     delete c;
     return fail(nullptr, FX_EDEVICE, "hipMalloc failed");
@@ -116,6 +122,7 @@ int fx_ctx_create(int device, uint64_t hbm_budget_bytes, fx_ctx** out) {
     const std::string msg = c->error;
     (void)hipFree(c->scalars);
     (void)hipFree(c->pimy_params);
+    (void)hipHostFree(c->host_pinned);
     (void)hipStreamDestroy(c->stream);
     delete c;
     return fail(nullptr, rc, msg);
@@ -132,6 +139,7 @@ void fx_ctx_destroy(fx_ctx* ctx) {
   if (ctx->red) (void)hipFree(ctx->red);
   if (ctx->scalars) (void)hipFree(ctx->scalars);
   if (ctx->pimy_params) (void)hipFree(ctx->pimy_params);
+  if (ctx->host_pinned) (void)hipHostFree(ctx->host_pinned);
   (void)hipStreamSynchronize(ctx->own_stream);
   (void)hipStreamDestroy(ctx->own_stream);
   delete ctx;
@@ -265,7 +273,8 @@ void fx_batch_destroy(fx_batch* b) {
                   b->state_c, b->state_t, b->tangent, b->tangent32, b->slots, b->gather_start, b->gather_list, b->long_eqs, b->pimy_touched, b->dyn, b->gm,
                   b->cres, b->clist, b->ccount, b->nodal_m, b->nodal_am, b->nodal_m32, b->nodal_am32, b->eq_dir_dev,
                   b->words_ref, b->shared_word_ref, b->tied_word_ref, b->orphans_ref, b->ssp_elem, b->ssp_box,
-                  b->kx, b->ky, b->kz, b->cg_state, b->cg_red, b->internal_of_dev};
+                  b->kx, b->ky, b->kz, b->cg_state, b->cg_red, b->internal_of_dev,
+                  b->shared_at};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   ctx->used -= std::min<uint64_t>(ctx->used, b->device_bytes);
@@ -487,6 +496,22 @@ int fx_batch_create(fx_ctx* ctx, const fx_batch_desc* d, uint32_t flags, fx_batc
         ok(dev_zeros(ctx, b->partial64, static_cast<size_t>(std::max<int64_t>(lat.nslot, 1)) * 3, by)) &&
         ok(b->has_f32 ? dev_zeros(ctx, b->partial32, static_cast<size_t>(std::max<int64_t>(lat.nslot, 1)) * 3, by) : FX_OK) &&
         ok(dev_upload(ctx, b->perm, lat.perm.data(), lat.perm.size(), by));
+    // the shared equations' partials (hex8_sum_dot_kernel): the nodes' equations run on in order
+    {
+      std::vector<uint32_t> at;
+      for (size_t i = 0; i < lat.shared_word.size(); ++i) {
+        const uint32_t w = lat.shared_word[i], mt = lat.shared_meta[i];
+        for (uint32_t dd = 0, j = 0; dd < 3; ++dd) {
+          if (!((w >> 28) & (1u << dd))) continue;
+          const int64_t e = static_cast<int64_t>(w & 0x0fffffffu) + j++;
+          if (at.empty()) b->shared_eq0 = e;
+          at.push_back(3u * static_cast<uint32_t>(lat.shared_start[i]) + dd);
+          at.push_back(3u * (mt & 0xffffffu) | (mt >> 24) << 28);
+        }
+      }
+      b->shared_neq = static_cast<int64_t>(at.size() / 2);
+      if (!at.empty()) ok(dev_upload(ctx, b->shared_at, at.data(), at.size(), by));
+    }
     // the node words in the reference numbering, where each node's free DOFs have consecutive
     // reference equations (so a word's first equation and mask still name them)
     bool consecutive = true;

@@ -138,7 +138,7 @@ struct fx_ctx {
   double* red = nullptr;  // partial sums
   size_t red_cap = 0;
   void* scalars = nullptr;  // solver state block (device)
-  void* host_pinned = nullptr;
+  void* host_pinned = nullptr;  // 4 KB the device writes: a dot's result, a CG solve's progress
   void* pimy_params = nullptr;  // material-point driver: up to kMaxPointMaterials parameter sets
   bool use_graphs = false;      // CG iterations replayed from captured graphs (FX_OPT_GRAPHS)
   hipStream_t own_stream = nullptr;  // the stream the context created (stream is the caller's with FX_OPT_STREAM)
@@ -290,6 +290,10 @@ struct fx_batch {
   uint32_t* shared_word = nullptr;
   int32_t* shared_start = nullptr;
   uint32_t* shared_meta = nullptr;
+  // the shared nodes' equations [shared_eq0, shared_eq0 + shared_neq) (solver numbering): each one's
+  // first partial, then 3 * stride | tiles << 28
+  uint32_t* shared_at = nullptr;
+  int64_t shared_eq0 = 0, shared_neq = 0;
   double* partial64 = nullptr;        // [nslot * 3] per-tile sums at shared nodes
   float* partial32 = nullptr;
   int box_variant = 0;                // lattice kernel variant of the operator without mass terms (tuned)

@@ -48,7 +48,15 @@ __host__ __device__ inline void operator_factors(const DevParam& p, const fx_coe
 
 // ref = 1: x and y in the reference numbering (the batch's reference-numbering words)
 template <typename T, bool DIAG>
-int launch_box(fx_batch* b, const fx_coeffs& k, const T* x, T* y, int accumulate, const int32_t* done, int ref = 0);
+int launch_box(fx_batch* b, const fx_coeffs& k, const T* x, T* y, int accumulate, const int32_t* done, int ref = 0,
+               bool sums = true);
+// A lattice product y = A x with the chunk partials of x.y (VectorOps' order) formed by the kernel
+// that adds the shared nodes' partial sums (solver numbering); for batches box_sums_with_dot takes.
+inline bool box_sums_with_dot(const fx_batch* b) {
+  return b->lattice && !b->pimy && b->norphans == 0 && !b->nodal_m && !b->nodal_am;
+}
+template <typename T>
+int launch_box_dot(fx_batch* b, const fx_coeffs& k, const T* x, T* y, double* part, const int32_t* done);
 
 int operator_apply64(fx_batch* b, const fx_coeffs& k, const double* x, double* y, const int32_t* done = nullptr);
 int operator_apply32(fx_batch* b, const fx_coeffs& k, const float* x, float* y, const int32_t* done = nullptr);

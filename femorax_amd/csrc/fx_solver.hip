@@ -20,232 +20,293 @@
 
 #include "fx_internal.hpp"
 #include "fx_kernels.hpp"
+#include "fx_vecops.hpp"
 
 namespace fx {
 
-constexpr int kChunk = 2048;
-constexpr int kLanes = 64;
-
+// The CG's scalars on the device. A field is written by one kernel of an iteration only and read
+// by the others: update_dot_kernel writes it and rz, direction_kernel rz_next and the stop's
+// fields, so that every workgroup of a kernel derives the same step from the same values.
 struct CgState {
-  double rz, pap, alpha, beta, rr, tol, rhs_norm, init_res, final_res, scale;
-  int32_t it, done, converged, indefinite, max_it, pad;
+  double rz, rz_next, tol, rhs_norm, init_res, final_res;
+  int32_t it, done, converged, indefinite, max_it, zeros;
 };
 
-__device__ __forceinline__ double as_double(double v) { return v; }
-__device__ __forceinline__ double as_double(float v) { return static_cast<double>(v); }
+// The host's copy of a solve's progress, in pinned memory: the device writes `it` after each
+// iteration and, last of all, `done`, so the host neither copies nor synchronises to poll.
+struct CgMirror {
+  double rhs_norm, init_res, final_res;
+  int32_t it, converged, indefinite, zeros, done, pad;
+};
 
-// Partial sums per chunk of x.y (and, when y2 != null, of x2.y2) in VectorOps' lane order.
-template <typename T>
-__global__ __launch_bounds__(kLanes) void chunk_dot_kernel(int64_t n, const T* __restrict__ x, const T* __restrict__ y,
-                                                           const T* __restrict__ x2, const T* __restrict__ y2,
-                                                           double* __restrict__ partial, const int32_t* done) {
-  if (done && *done) return;
-  __shared__ double lane_sum[2][kLanes];
-  const int64_t c = blockIdx.x;
-  const int64_t begin = c * kChunk;
-  const int64_t len = (n - begin < kChunk) ? n - begin : kChunk;
-  const int l = threadIdx.x;
-  double s = 0.0, s2 = 0.0;
-  for (int64_t k = l; k < len; k += kLanes) {
-    s += as_double(x[begin + k]) * as_double(y[begin + k]);
-    if (y2) s2 += as_double(x2[begin + k]) * as_double(y2[begin + k]);
-  }
-  lane_sum[0][l] = s;
-  lane_sum[1][l] = s2;
-  __syncthreads();
-  if (l == 0) {
-    double t = 0.0, t2 = 0.0;
-    for (int j = 0; j < kLanes; ++j) t += lane_sum[0][j];
-    for (int j = 0; j < kLanes; ++j) t2 += lane_sum[1][j];
-    if (y2) {
-      partial[2 * c] = t;
-      partial[2 * c + 1] = t2;
-    } else {
-      partial[c] = t;
-    }
-  }
+__device__ inline void mirror_stop(CgMirror* m, const CgState* st, double final_res, int it, int converged) {
+  if (!m) return;
+  m->rhs_norm = st->rhs_norm;
+  m->init_res = st->init_res;
+  m->final_res = final_res;
+  m->converged = converged;
+  m->indefinite = st->indefinite;
+  m->zeros = st->zeros;
+  __hip_atomic_store(&m->it, it, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(&m->done, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-enum ReduceOp : int { kStore = 0, kRhsNorm, kInitRes, kRz0, kPap, kIter };
-
-// One chunk of a level, summed by one wave in VectorOps' order: lane l adds entries l, l + 64,
-// ... in turn, then lane 0 adds the 64 lane sums in lane order (through this wave's lane_sum
-// row in LDS: a wave's LDS accesses complete in program order). A full chunk issues each lane's
-// 32 loads together; a partial one (the last of a level, or a small vector) walks its entries.
-// Returns the total in lane 0.
-__device__ __forceinline__ double wave_chunk_sum(const double* src, int64_t stride, int64_t begin, int64_t len, int l,
-                                                 double* lane_sum) {
-  double s = 0.0;
-  if (len == kChunk) {
-    double v[kChunk / kLanes];
+// Partial sums per chunk of x.y in VectorOps' lane order (one workgroup per chunk, see
+// kVecThreads). 27,744 entries (14 chunks): 11.2 -> 3 us; 6.4 M entries: HBM-bound either way.
+template <typename T>
+__global__ __launch_bounds__(kVecThreads) void chunk_dot_kernel(int64_t n, const T* __restrict__ x,
+                                                                const T* __restrict__ y, double* __restrict__ partial,
+                                                                const int32_t* done) {
+  if (done && *done) return;
+  __shared__ T xs[kChunk], ys[kChunk];
+  __shared__ double row[kLanes];
+  const int64_t begin = static_cast<int64_t>(blockIdx.x) * kChunk;
+  const int len = static_cast<int>(n - begin < kChunk ? n - begin : kChunk);
+  const int t = threadIdx.x;
+  T xv[kPerThread], yv[kPerThread];
 #pragma unroll
-    for (int j = 0; j < kChunk / kLanes; ++j) v[j] = src[(begin + l + static_cast<int64_t>(j) * kLanes) * stride];
-#pragma unroll
-    for (int j = 0; j < kChunk / kLanes; ++j) s += v[j];
-  } else {
-    for (int64_t k = l; k < len; k += kLanes) s += src[(begin + k) * stride];
+  for (int j = 0; j < kPerThread; ++j) {
+    const int k = t + j * kVecThreads;
+    xv[j] = k < len ? x[begin + k] : T(0);
+    yv[j] = k < len ? y[begin + k] : T(0);
   }
-  lane_sum[l] = s;
-  __builtin_amdgcn_wave_barrier();
-  double t = 0.0;
-  if (l == 0)
-    for (int j = 0; j < kLanes; ++j) t += lane_sum[j];
-  __builtin_amdgcn_wave_barrier();
-  return t;
+#pragma unroll
+  for (int j = 0; j < kPerThread; ++j) {
+    xs[t + j * kVecThreads] = xv[j];
+    ys[t + j * kVecThreads] = yv[j];
+  }
+  __syncthreads();
+  if (t >= kLanes) return;
+  const double s = wave_staged_dot(xs, ys, len, t, row);
+  if (t == 0) partial[blockIdx.x] = s;
 }
 
 // Reduce `nv` (1 or 2) interleaved sequences of chunk partials level by level in one workgroup,
-// in VectorOps' order, then apply the solver step `op` to the totals. The first level's chunks
-// go to the workgroup's waves (red_threads: one wave per chunk, at most kRedWaves; their totals
-// in LDS); wave 0 sums those (one chunk: fewer than 2^31 entries have at most kRedTot first-level
-// chunks). The same bits as one wave walking the levels in turn.
+// in VectorOps' order, into out[v]. The first level's chunks go to the workgroup's waves
+// (red_threads: one wave per chunk, at most kRedWaves; their totals in LDS); wave 0 sums those
+// (one chunk: fewer than 2^31 entries have at most kRedTot first-level chunks). The same bits as
+// one wave walking the levels in turn.
 constexpr int kRedWaves = 8, kRedThreads = kRedWaves * kLanes, kRedTot = 512;
 static_assert(static_cast<int64_t>(kRedTot) * kChunk * kChunk >= (int64_t(1) << 31), "first-level totals of 2^31 entries");
-__host__ __device__ inline int64_t red_chunks(int64_t n) { return (n + kChunk - 1) / kChunk; }
 // the reduction's workgroup for n entries: a wave per first-level chunk of the n / 2048 partials
 inline dim3 red_threads(int64_t n) {
-  const int64_t c = red_chunks(red_chunks(n));
+  const int64_t c = chunks(chunks(n));
   return dim3(static_cast<unsigned>(kLanes * (c < 1 ? 1 : c > kRedWaves ? kRedWaves : c)));
 }
-__global__ __launch_bounds__(kRedThreads) void reduce_kernel(int64_t npart, int nv, double* __restrict__ partial,
-                                                             double* __restrict__ tmp, CgState* st, int op,
-                                                             double rtol, double atol, double* out) {
-  if (op == kPap || op == kIter)
-    if (st->done) return;
-  (void)tmp;
+__global__ __launch_bounds__(kRedThreads) void reduce_kernel(int64_t npart, int nv, const double* __restrict__ partial,
+                                                             const int32_t* done, double* out) {
+  if (done && *done) return;
   __shared__ double tot[2][kRedTot];
-  __shared__ double lane_sum[kRedWaves][kLanes];
+  __shared__ double row[kRedWaves][kLanes];
   const int l = threadIdx.x % kLanes, w = threadIdx.x / kLanes;
-  const int64_t nch = (npart + kChunk - 1) / kChunk;
+  const int64_t nch = chunks(npart);
   double total[2] = {0.0, 0.0};
   if (npart > 1) {
     for (int v = 0; v < nv; ++v)
       for (int64_t c = w; c < nch; c += static_cast<int64_t>(blockDim.x / kLanes)) {
         const int64_t begin = c * kChunk;
         const double t =
-            wave_chunk_sum(partial + v, nv, begin, npart - begin < kChunk ? npart - begin : kChunk, l, lane_sum[w]);
+            wave_chunk_sum(partial + v, nv, begin, npart - begin < kChunk ? npart - begin : kChunk, l, row[w]);
         if (l == 0) tot[v][c] = t;
       }
     __syncthreads();
     if (w == 0)
-      for (int v = 0; v < nv; ++v) total[v] = nch > 1 ? wave_chunk_sum(tot[v], 1, 0, nch, l, lane_sum[0]) : tot[v][0];
+      for (int v = 0; v < nv; ++v) total[v] = nch > 1 ? wave_chunk_sum(tot[v], 1, 0, nch, l, row[0]) : tot[v][0];
   } else {
     for (int v = 0; v < nv; ++v) total[v] = partial[v];
   }
   if (threadIdx.x != 0) return;
-  switch (op) {
-    case kStore:
-      out[0] = total[0];
-      break;
-    case kRhsNorm:
-      st->rhs_norm = sqrt(total[0]);
-      st->tol = fmax(rtol * st->rhs_norm, atol);
-      break;
-    case kInitRes: {
-      const double r = sqrt(total[0]);
-      st->init_res = st->final_res = r;
-      st->it = 0;
-      st->indefinite = 0;
-      st->converged = r <= st->tol;
-      st->done = st->converged || st->max_it <= 0;
-      break;
-    }
-    case kRz0:
-      st->rz = total[0];
-      break;
-    case kPap:
-      st->pap = total[0];
-      if (!(total[0] > 0.0)) {
-        st->indefinite = 1;
-        st->done = 1;
-      } else {
-        st->alpha = st->rz / total[0];
+  for (int v = 0; v < nv; ++v) out[v] = total[v];
+}
+
+// r = b - A x (ap holds A x); START: also z = inv r, p = z, and the chunk partials of r.r and r.z
+// (interleaved); else of r.r alone.
+template <typename T, bool START>
+__global__ __launch_bounds__(kVecThreads) void residual_kernel(int64_t n, const T* __restrict__ b,
+                                                               const T* __restrict__ ap, const T* __restrict__ inv,
+                                                               T* __restrict__ r, T* __restrict__ z, T* __restrict__ p,
+                                                               double* __restrict__ partial) {
+  __shared__ T rs[kChunk], zs[START ? kChunk : 1];
+  __shared__ double row[2][kLanes];
+  const int64_t begin = static_cast<int64_t>(blockIdx.x) * kChunk;
+  const int len = static_cast<int>(n - begin < kChunk ? n - begin : kChunk);
+  const int t = threadIdx.x;
+  T bv[kPerThread], av[kPerThread], iv[kPerThread];
+#pragma unroll
+  for (int j = 0; j < kPerThread; ++j) {
+    const int k = t + j * kVecThreads;
+    bv[j] = k < len ? b[begin + k] : T(0);
+    av[j] = k < len ? ap[begin + k] : T(0);
+    if constexpr (START) iv[j] = k < len ? inv[begin + k] : T(0);
+  }
+#pragma unroll
+  for (int j = 0; j < kPerThread; ++j) {
+    const int k = t + j * kVecThreads;
+    const T rj = bv[j] + T(-1) * av[j];
+    rs[k] = rj;
+    if (k < len) r[begin + k] = rj;
+    if constexpr (START) {
+      const T zj = iv[j] * rj;
+      zs[k] = zj;
+      if (k < len) {
+        z[begin + k] = zj;
+        p[begin + k] = zj;
       }
-      break;
-    case kIter: {
-      const double r = sqrt(total[0]);
-      st->it += 1;
-      st->final_res = r;
-      if (r <= st->tol) {
-        st->converged = 1;
-        st->done = 1;
-      } else {
-        st->beta = total[1] / st->rz;
-        st->rz = total[1];
-        if (st->it >= st->max_it) st->done = 1;
-      }
-      break;
     }
   }
-}
-
-template <typename T>
-__global__ void residual_kernel(int64_t n, const T* __restrict__ b, const T* __restrict__ ap, T* __restrict__ r) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < n) r[i] = b[i] + T(-1) * ap[i];
-}
-
-// z = inv r, p = z (first direction)
-template <typename T>
-__global__ void precond_first_kernel(int64_t n, const T* __restrict__ inv, const T* __restrict__ r, T* __restrict__ z,
-                                     T* __restrict__ p) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < n) {
-    const T zi = inv[i] * r[i];
-    z[i] = zi;
-    p[i] = zi;
-  }
-}
-
-// x += alpha p; r -= alpha ap; z = inv r   (cg.cpp:55-56, 64), skipped once done
-// p = z + beta p (cg.cpp:68)
-template <typename T>
-__global__ void direction_kernel(int64_t n, const CgState* st, const T* __restrict__ z, T* __restrict__ p) {
-  if (st->done) return;
-  const T beta = static_cast<T>(st->beta);
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = z[i] + beta * p[i];
-}
-
-// update_kernel followed by chunk_dot_kernel(r, r, r, z) in one pass: workgroup c updates x, r, z
-// on chunk c (lane l on entries l, l + 64, ...) and forms the chunk's lane sums of r.r and r.z
-// from the updated values in VectorOps' order, so x, r, z and the partials have the bits of the
-// two kernels.
-template <typename T>
-__global__ __launch_bounds__(kLanes) void update_dot_kernel(int64_t n, const CgState* st, T* __restrict__ x,
-                                                            T* __restrict__ r, T* __restrict__ z, const T* __restrict__ p,
-                                                            const T* __restrict__ ap, const T* __restrict__ inv,
-                                                            double* __restrict__ partial) {
-  if (st->done) return;
-  __shared__ double lane_sum[2][kLanes];
-  const T alpha = static_cast<T>(st->alpha);
-  const int64_t c = blockIdx.x;
-  const int64_t begin = c * kChunk;
-  const int64_t len = (n - begin < kChunk) ? n - begin : kChunk;
-  const int l = threadIdx.x;
-  double s = 0.0, s2 = 0.0;
-  for (int64_t k = l; k < len; k += kLanes) {
-    const int64_t i = begin + k;
-    x[i] += alpha * p[i];
-    const T ri = r[i] + (-alpha) * ap[i];
-    r[i] = ri;
-    const T zi = inv[i] * ri;
-    z[i] = zi;
-    s += as_double(ri) * as_double(ri);
-    s2 += as_double(ri) * as_double(zi);
-  }
-  lane_sum[0][l] = s;
-  lane_sum[1][l] = s2;
   __syncthreads();
-  if (l == 0) {
-    double t = 0.0, t2 = 0.0;
-    for (int j = 0; j < kLanes; ++j) t += lane_sum[0][j];
-    for (int j = 0; j < kLanes; ++j) t2 += lane_sum[1][j];
-    partial[2 * c] = t;
-    partial[2 * c + 1] = t2;
-  }
+  const int w = t / kLanes, l = t % kLanes;
+  if (w >= (START ? 2 : 1)) return;
+  double s;
+  if constexpr (START) s = wave_staged_dot(rs, w == 0 ? rs : zs, len, l, row[w]);
+  else s = wave_staged_dot(rs, rs, len, l, row[w]);
+  if (l == 0) partial[(START ? 2 : 1) * static_cast<int64_t>(blockIdx.x) + w] = s;
 }
 
+// The solve's state from ||b||, the first residual and r.z (cg.cpp:30-43): one workgroup.
+__global__ __launch_bounds__(kVecThreads) void cg_start_kernel(int64_t nb, const double* __restrict__ bpart, int64_t nr,
+                                                               const double* __restrict__ rpart, double rtol, double atol,
+                                                               int32_t max_it, const int32_t* zeros, CgState* st,
+                                                               CgMirror* mirror) {
+  __shared__ double row[3][kLanes];
+  __shared__ double tot[3];
+  const int w = threadIdx.x / kLanes, l = threadIdx.x % kLanes;
+  if (w < 3) {
+    const double s = w == 0 ? wave_total(bpart, 1, 0, nb, l, row[w]) : wave_total(rpart, 2, w - 1, nr, l, row[w]);
+    if (l == 0) tot[w] = s;
+  }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  st->rhs_norm = sqrt(tot[0]);
+  st->tol = fmax(rtol * st->rhs_norm, atol);
+  st->init_res = st->final_res = sqrt(tot[1]);
+  st->rz = st->rz_next = tot[2];
+  st->it = 0;
+  st->max_it = max_it;
+  st->indefinite = 0;
+  st->zeros = zeros ? *zeros : 0;
+  st->converged = st->init_res <= st->tol;
+  st->done = st->converged || max_it <= 0 || st->zeros > 0;
+  if (st->done) mirror_stop(mirror, st, st->final_res, 0, st->converged);
+}
+
+// alpha = r.z / p.Ap from the chunk partials of p.Ap; x += alpha p, r -= alpha Ap, z = inv r
+// (cg.cpp:48-64), and the chunk partials of r.r and r.z from the updated values. One workgroup
+// per chunk, its loads issued before the total of p.Ap is needed. 27,744 entries: 8.2 -> 4 us and
+// one launch less; HBM-bound from about a million entries.
+template <typename T>
+__global__ __launch_bounds__(kVecThreads) void update_dot_kernel(int64_t n, CgState* st, int64_t npap,
+                                                                 const double* __restrict__ pap, T* __restrict__ x,
+                                                                 T* __restrict__ r, T* __restrict__ z,
+                                                                 const T* __restrict__ p, const T* __restrict__ ap,
+                                                                 const T* __restrict__ inv, double* __restrict__ partial,
+                                                                 CgMirror* mirror) {
+  if (st->done) return;
+  __shared__ T rs[kChunk], zs[kChunk];
+  __shared__ double row[2][kLanes];
+  __shared__ double total;
+  const int64_t begin = static_cast<int64_t>(blockIdx.x) * kChunk;
+  const int len = static_cast<int>(n - begin < kChunk ? n - begin : kChunk);
+  const int t = threadIdx.x, w = t / kLanes, l = t % kLanes;
+  T xv[kPerThread], rv[kPerThread], pv[kPerThread], av[kPerThread], iv[kPerThread];
+#pragma unroll
+  for (int j = 0; j < kPerThread; ++j) {
+    const int k = t + j * kVecThreads;
+    const int64_t i = begin + (k < len ? k : 0);
+    xv[j] = x[i];
+    rv[j] = r[i];
+    pv[j] = p[i];
+    av[j] = ap[i];
+    iv[j] = inv[i];
+  }
+  if (w == 0) {
+    const double s = wave_total(pap, 1, 0, npap, l, row[0]);
+    if (l == 0) total = s;
+  }
+  __syncthreads();
+  if (!(total > 0.0)) {  // p.Ap <= 0: the operator is not positive definite (cg.cpp:49-53)
+    if (blockIdx.x == 0 && t == 0) {
+      st->indefinite = 1;
+      st->done = 1;
+      mirror_stop(mirror, st, st->final_res, st->it, 0);
+    }
+    return;
+  }
+  const double rz = st->rz_next;
+  const T alpha = static_cast<T>(rz / total);
+  if (blockIdx.x == 0 && t == 0) {
+    st->rz = rz;
+    st->it += 1;
+  }
+#pragma unroll
+  for (int j = 0; j < kPerThread; ++j) {
+    const int k = t + j * kVecThreads;
+    const T xj = xv[j] + alpha * pv[j];
+    const T rj = rv[j] + (-alpha) * av[j];
+    const T zj = iv[j] * rj;
+    rs[k] = rj;
+    zs[k] = zj;
+    if (k < len) {
+      x[begin + k] = xj;
+      r[begin + k] = rj;
+      z[begin + k] = zj;
+    }
+  }
+  __syncthreads();
+  if (w >= 2) return;
+  const double s = wave_staged_dot(rs, w == 0 ? rs : zs, len, l, row[w]);
+  if (l == 0) partial[2 * static_cast<int64_t>(blockIdx.x) + w] = s;
+}
+
+// The stop test on ||r|| (cg.cpp:60) and p = z + beta p (cg.cpp:68) from the chunk partials of r.r
+// and r.z: every workgroup takes the same decision; the first records it.
+template <typename T>
+__global__ __launch_bounds__(kVecThreads) void direction_kernel(int64_t n, CgState* st, int64_t npart,
+                                                                const double* __restrict__ part,
+                                                                const T* __restrict__ z, T* __restrict__ p,
+                                                                CgMirror* mirror) {
+  if (st->done) return;
+  __shared__ double row[2][kLanes];
+  __shared__ double tot[2];
+  const int64_t begin = static_cast<int64_t>(blockIdx.x) * kChunk;
+  const int len = static_cast<int>(n - begin < kChunk ? n - begin : kChunk);
+  const int t = threadIdx.x, w = t / kLanes, l = t % kLanes;
+  const int it = st->it, max_it = st->max_it;
+  const double rz = st->rz, tol = st->tol;
+  T zv[kPerThread], pv[kPerThread];
+#pragma unroll
+  for (int j = 0; j < kPerThread; ++j) {
+    const int k = t + j * kVecThreads;
+    const int64_t i = begin + (k < len ? k : 0);
+    zv[j] = z[i];
+    pv[j] = p[i];
+  }
+  if (w < 2) {
+    const double s = wave_total(part, 2, w, npart, l, row[w]);
+    if (l == 0) tot[w] = s;
+  }
+  __syncthreads();
+  const double rn = sqrt(tot[0]);
+  const bool converged = rn <= tol, stop = converged || it >= max_it;
+  if (blockIdx.x == 0 && t == 0) {
+    st->final_res = rn;
+    st->rz_next = tot[1];
+    if (converged) st->converged = 1;
+    if (stop) {
+      st->done = 1;
+      mirror_stop(mirror, st, rn, it, converged);
+    } else if (mirror) {
+      __hip_atomic_store(&mirror->it, it, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+  }
+  if (stop) return;
+  const T beta = static_cast<T>(tot[1] / rz);
+#pragma unroll
+  for (int j = 0; j < kPerThread; ++j) {
+    const int k = t + j * kVecThreads;
+    if (k < len) p[begin + k] = zv[j] + beta * pv[j];
+  }
+}
 
 template <typename T>
 __global__ void reciprocal_kernel(int64_t n, const double* __restrict__ d, T* __restrict__ inv, int32_t* zeros) {
@@ -289,11 +350,11 @@ int copy64(fx_ctx* ctx, int64_t n, const double* a, double* b) {
 namespace {
 
 inline dim3 grid_of(int64_t n, int bs = 256) { return dim3(static_cast<unsigned>((n + bs - 1) / bs)); }
-inline int64_t chunks(int64_t n) { return (n + kChunk - 1) / kChunk; }
+inline dim3 chunk_grid(int64_t n) { return dim3(static_cast<unsigned>(chunks(n))); }
 
-// Reduction scratch: [2 * chunks] partials + a level buffer.
+// Reduction scratch: the chunk partials of one dot, then of two, then their totals.
 int ensure_red(fx_ctx* ctx, int64_t n) {
-  const size_t need = static_cast<size_t>(2 * chunks(n) + 2 * (chunks(chunks(n)) + 2) + 16);
+  const size_t need = cg_red_doubles(n);
   if (ctx->red_cap >= need) return FX_OK;
   release_cg_graphs(ctx, nullptr);  // captured graphs read the old buffer
   if (ctx->red) (void)hipFree(ctx->red);
@@ -386,17 +447,14 @@ int dot64(fx_ctx* ctx, int64_t n, const double* x, const double* y, double* out)
     return FX_OK;
   }
   if (int rc = ensure_red(ctx, n)) return rc;
-  double* part = ctx->red;
-  double* tmp = ctx->red + 2 * chunks(n);
-  hipLaunchKernelGGL(chunk_dot_kernel<double>, dim3(static_cast<unsigned>(chunks(n))), dim3(kLanes), 0, ctx->stream,
-                     n, x, y, static_cast<const double*>(nullptr), static_cast<const double*>(nullptr), part,
+  double* dres = static_cast<double*>(ctx->host_pinned);  // the device writes the total to host memory
+  hipLaunchKernelGGL(chunk_dot_kernel<double>, chunk_grid(n), dim3(kVecThreads), 0, ctx->stream, n, x, y, ctx->red,
                      static_cast<const int32_t*>(nullptr));
-  double* dres = tmp + chunks(chunks(n)) + 8;
-  hipLaunchKernelGGL(reduce_kernel, dim3(1), red_threads(n), 0, ctx->stream, chunks(n), 1, part, tmp,
-                     static_cast<CgState*>(nullptr), static_cast<int>(kStore), 0.0, 0.0, dres);
+  hipLaunchKernelGGL(reduce_kernel, dim3(1), red_threads(n), 0, ctx->stream, chunks(n), 1, ctx->red,
+                     static_cast<const int32_t*>(nullptr), dres);
   FX_HIP(ctx, hipGetLastError());
-  FX_HIP(ctx, hipMemcpyAsync(out, dres, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
   FX_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  *out = *dres;
   return FX_OK;
 }
 
@@ -459,142 +517,222 @@ hipGraphExec_t cg_graph(fx_ctx* ctx, const CgGraphKey& key, Body body) {
   return exec;
 }
 
-// The CG setup on the device for vector type T: ||b||, r = b - A x, z = inv r, p = z, r.z; the
-// state block st and the reduction scratch red (2 chunks(n) + levels) are the solve's own.
-template <typename T, typename Apply>
-int cg_setup(fx_ctx* ctx, int64_t n, Apply apply, const T* inv, const T* b, T* x, T* r, T* z, T* p, T* ap,
-             CgState* st, double* red, double rtol, double atol, int max_it) {
+// A dot's chunk partials as the kernels that need their total take them: the partials themselves,
+// or past kInlineParts the total(s), reduced by a launch of their own (into tot).
+struct Parts {
+  int64_t n;
+  const double* p;
+};
+Parts total_of(fx_ctx* ctx, int64_t n, int nv, const double* part, double* tot, const int32_t* done) {
+  if (chunks(n) <= kInlineParts) return Parts{chunks(n), part};
+  hipLaunchKernelGGL(reduce_kernel, dim3(1), red_threads(n), 0, ctx->stream, chunks(n), nv, part, done, tot);
+  return Parts{1, tot};
+}
+
+// A CG solve's device arrays (solver numbering) and the operator they belong to.
+template <typename T>
+struct CgVectors {
+  const T *inv, *b;
+  T *x, *r, *z, *p, *ap;
+  CgState* st;
+  double* red;       // cg_red_doubles(n)
+  CgMirror* mirror;  // or null
+};
+
+// The CG setup on the device: ||b||, r = b - A x, z = inv r, p = z, r.z. zeros: the count of zero
+// diagonal entries (a solve that has any stops before its first iteration), or null.
+template <typename T, typename Op>
+int cg_setup(fx_ctx* ctx, int64_t n, const Op& op, const CgVectors<T>& v, double rtol, double atol, int max_it,
+             const int32_t* zeros) {
   hipStream_t s = ctx->stream;
-  double* part = red;
-  double* tmp = red + 2 * chunks(n);
-  const dim3 g = grid_of(n), cg_chunks(static_cast<unsigned>(chunks(n)));
-  CgState init{};
-  init.max_it = max_it;
-  FX_HIP(ctx, hipMemcpyAsync(st, &init, sizeof(CgState), hipMemcpyHostToDevice, s));
-  const T* nt = nullptr;
-  // ||b||
-  hipLaunchKernelGGL(chunk_dot_kernel<T>, cg_chunks, dim3(kLanes), 0, s, n, b, b, nt, nt, part,
-                     static_cast<const int32_t*>(nullptr));
-  hipLaunchKernelGGL(reduce_kernel, dim3(1), red_threads(n), 0, s, chunks(n), 1, part, tmp, st,
-                     static_cast<int>(kRhsNorm), rtol, atol, static_cast<double*>(nullptr));
-  // r = b - A x
-  if (int rc = apply(x, ap, static_cast<const int32_t*>(nullptr))) return rc;
-  hipLaunchKernelGGL(residual_kernel<T>, g, dim3(256), 0, s, n, b, ap, r);
-  hipLaunchKernelGGL(chunk_dot_kernel<T>, cg_chunks, dim3(kLanes), 0, s, n, r, r, nt, nt, part,
-                     static_cast<const int32_t*>(nullptr));
-  hipLaunchKernelGGL(reduce_kernel, dim3(1), red_threads(n), 0, s, chunks(n), 1, part, tmp, st,
-                     static_cast<int>(kInitRes), rtol, atol, static_cast<double*>(nullptr));
-  // z = inv r, p = z, rz = r.z
-  hipLaunchKernelGGL(precond_first_kernel<T>, g, dim3(256), 0, s, n, inv, r, z, p);
-  hipLaunchKernelGGL(chunk_dot_kernel<T>, cg_chunks, dim3(kLanes), 0, s, n, r, z, nt, nt, part,
-                     static_cast<const int32_t*>(nullptr));
-  hipLaunchKernelGGL(reduce_kernel, dim3(1), red_threads(n), 0, s, chunks(n), 1, part, tmp, st,
-                     static_cast<int>(kRz0), rtol, atol, static_cast<double*>(nullptr));
+  double *p1 = v.red, *p2 = v.red + chunks(n), *tot = v.red + 3 * chunks(n);
+  const int32_t* always = nullptr;
+  hipLaunchKernelGGL(chunk_dot_kernel<T>, chunk_grid(n), dim3(kVecThreads), 0, s, n, v.b, v.b, p1, always);
+  const Parts bb = total_of(ctx, n, 1, p1, tot, always);
+  if (int rc = op.apply(v.x, v.ap)) return rc;
+  hipLaunchKernelGGL((residual_kernel<T, true>), chunk_grid(n), dim3(kVecThreads), 0, s, n, v.b, v.ap, v.inv, v.r, v.z,
+                     v.p, p2);
+  const Parts rr = total_of(ctx, n, 2, p2, tot + 1, always);
+  hipLaunchKernelGGL(cg_start_kernel, dim3(1), dim3(kVecThreads), 0, s, bb.n, bb.p, rr.n, rr.p, rtol, atol, max_it,
+                     zeros, v.st, v.mirror);
   FX_HIP(ctx, hipGetLastError());
   return FX_OK;
 }
 
-// One CG iteration (cg.cpp:44-69): A p, p.Ap, the fused x, r, z update with r.r and r.z, the
-// direction; a no-op once the state's stop flag is set.
-template <typename T, typename Apply>
-int cg_iteration(fx_ctx* ctx, int64_t n, Apply apply, const T* inv, T* x, T* r, T* z, T* p, T* ap, CgState* st,
-                 double* red, double rtol, double atol) {
+// One CG iteration (cg.cpp:44-69): A p with p.Ap, the fused x, r, z update with r.r and r.z, the
+// stop test with the direction; a no-op once the state's stop flag is set.
+template <typename T, typename Op>
+int cg_iteration(fx_ctx* ctx, int64_t n, const Op& op, const CgVectors<T>& v) {
   hipStream_t s = ctx->stream;
-  double* part = red;
-  double* tmp = red + 2 * chunks(n);
-  const dim3 g = grid_of(n), cg_chunks(static_cast<unsigned>(chunks(n)));
-  const T* nt = nullptr;
-  const int32_t* done = &st->done;
-  if (int rc = apply(p, ap, done)) return rc;
-  hipLaunchKernelGGL(chunk_dot_kernel<T>, cg_chunks, dim3(kLanes), 0, s, n, p, ap, nt, nt, part, done);
-  hipLaunchKernelGGL(reduce_kernel, dim3(1), red_threads(n), 0, s, chunks(n), 1, part, tmp, st,
-                     static_cast<int>(kPap), rtol, atol, static_cast<double*>(nullptr));
-  hipLaunchKernelGGL(update_dot_kernel<T>, cg_chunks, dim3(kLanes), 0, s, n, st, x, r, z, p, ap, inv, part);
-  hipLaunchKernelGGL(reduce_kernel, dim3(1), red_threads(n), 0, s, chunks(n), 2, part, tmp, st,
-                     static_cast<int>(kIter), rtol, atol, static_cast<double*>(nullptr));
-  hipLaunchKernelGGL(direction_kernel<T>, g, dim3(256), 0, s, n, st, z, p);
+  double *p1 = v.red, *p2 = v.red + chunks(n), *tot = v.red + 3 * chunks(n);
+  const int32_t* done = &v.st->done;
+  if (int rc = op.apply_dot(v.p, v.ap, p1, done)) return rc;
+  const Parts pap = total_of(ctx, n, 1, p1, tot, done);
+  hipLaunchKernelGGL(update_dot_kernel<T>, chunk_grid(n), dim3(kVecThreads), 0, s, n, v.st, pap.n, pap.p, v.x, v.r, v.z,
+                     v.p, v.ap, v.inv, p2, v.mirror);
+  const Parts rr = total_of(ctx, n, 2, p2, tot + 1, done);
+  hipLaunchKernelGGL(direction_kernel<T>, chunk_grid(n), dim3(kVecThreads), 0, s, n, v.st, rr.n, rr.p, v.z, v.p,
+                     v.mirror);
   return FX_OK;
 }
 
+// K_eff of a batch for vector type T: y = A x, and A p with the chunk partials of p.Ap.
+template <typename T>
+struct BatchOp {
+  fx_batch* b;
+  fx_coeffs k;
+  int apply(const T* x, T* y) const {
+    if constexpr (sizeof(T) == 8) return operator_apply64(b, k, x, y, nullptr);
+    else return operator_apply32(b, k, x, y, nullptr);
+  }
+  int apply_dot(const T* p, T* ap, double* part, const int32_t* done) const {
+    if (box_sums_with_dot(b)) return launch_box_dot<T>(b, k, p, ap, part, done);
+    int rc;
+    if constexpr (sizeof(T) == 8) rc = operator_apply64(b, k, p, ap, done);
+    else rc = operator_apply32(b, k, p, ap, done);
+    if (rc) return rc;
+    hipLaunchKernelGGL(chunk_dot_kernel<T>, chunk_grid(b->neq), dim3(kVecThreads), 0, b->ctx->stream, b->neq, p, ap, part,
+                       done);
+    return FX_OK;
+  }
+};
+
 // The captured graph of a solve's iterations (null: graphs off, or the capture failed).
-template <typename T, typename Body>
-hipGraphExec_t cg_solve_graph(fx_ctx* ctx, int64_t n, const T* inv, const T* b, T* x, T* r, T* z, T* p, T* ap,
-                              CgState* st, double* red, double rtol, double atol, int max_it, const fx_batch* owner,
-                              const fx_coeffs* kc, Body body) {
-  if (!ctx->use_graphs || !owner || !kc || max_it <= 0) return nullptr;
+template <typename T>
+hipGraphExec_t cg_solve_graph(fx_ctx* ctx, int64_t n, const CgVectors<T>& v, double rtol, double atol, int max_it,
+                              const BatchOp<T>& op) {
+  if (!ctx->use_graphs || max_it <= 0) return nullptr;
+  const fx_batch* owner = op.b;
   CgGraphKey key{};
   key.owner = owner;
   key.n = n;
   key.tsize = static_cast<int32_t>(sizeof(T));
-  key.initial = kc->initial;
-  key.ks = kc->stiffness;
-  key.kd = kc->damping;
-  key.km = kc->mass;
+  key.initial = op.k.initial;
+  key.ks = op.k.stiffness;
+  key.kd = op.k.damping;
+  key.km = op.k.mass;
   key.rtol = rtol;
   key.atol = atol;
-  const void* ptrs[10] = {inv, b, x, r, z, p, ap, st, red, red + 2 * chunks(n)};
+  const void* ptrs[10] = {v.inv, v.b, v.x, v.r, v.z, v.p, v.ap, v.st, v.red, v.mirror};
   for (int i = 0; i < 10; ++i) key.ptr[i] = ptrs[i];
   key.state[0] = owner->state_c;
   key.state[1] = owner->state_t;
-  return cg_graph(ctx, key, body);
+  return cg_graph(ctx, key, [&]() -> int { return cg_iteration<T>(ctx, n, op, v); });
 }
 
-// The CG iteration on the device for vector type T. apply(x, y) computes y = A x for the
-// operator of `owner` with coefficients k. The iterations run in groups between host polls of
-// the device stop flag (4, 8, ..., 64 iterations); iterations after the stop are no-ops. With
-// graphs on, each group replays a captured graph of kGraphIters iterations (the same kernels
-// and arguments, so the same bits as launching them).
-template <typename T, typename Apply>
-int cg_device(fx_ctx* ctx, int64_t n, Apply apply, const T* inv, const T* b, T* x, T* r, T* z, T* p, T* ap,
-              CgState* st, double rtol, double atol, int max_it, CgState& host, const fx_batch* owner = nullptr,
-              const fx_coeffs* kc = nullptr) {
+// Iterations queued beyond the last one the device has reported: enough to hide the host's launch
+// times, and the only iterations that run as no-ops after the stop (four launches each; polling
+// by copies in groups of up to 64 iterations ran 30 of them on average).
+constexpr int kQueueAhead = 8;
+
+// The CG iterations on the device after cg_setup: the host launches them while it watches the
+// solve's mirror. With graphs on, each group replays a captured graph of kGraphIters iterations
+// (the same kernels and arguments, so the same bits as launching them).
+template <typename T>
+int cg_device(fx_ctx* ctx, int64_t n, const BatchOp<T>& op, const T* inv, const T* b, T* x, T* r, T* z, T* p, T* ap,
+              CgState* st, double rtol, double atol, int max_it, const int32_t* zeros, CgMirror& host) {
   if (int rc = ensure_red(ctx, n)) return rc;
-  double* red = ctx->red;
   hipStream_t s = ctx->stream;
-  if (int rc = cg_setup<T>(ctx, n, apply, inv, b, x, r, z, p, ap, st, red, rtol, atol, max_it)) return rc;
-  auto body = [&]() -> int { return cg_iteration<T>(ctx, n, apply, inv, x, r, z, p, ap, st, red, rtol, atol); };
-  hipGraphExec_t exec = cg_solve_graph<T>(ctx, n, inv, b, x, r, z, p, ap, st, red, rtol, atol, max_it, owner, kc, body);
-  int launched = 0, poll = 4;
-  for (;;) {
-    FX_HIP(ctx, hipMemcpyAsync(&host, st, sizeof(CgState), hipMemcpyDeviceToHost, s));
-    FX_HIP(ctx, hipStreamSynchronize(s));
-    if (host.done || launched >= max_it) break;
-    const int batch = std::min(poll, max_it - launched);
-    if (exec) {
-      const int graphs = (batch + kGraphIters - 1) / kGraphIters;
-      for (int i = 0; i < graphs; ++i) FX_HIP(ctx, hipGraphLaunch(exec, s));
-      launched += graphs * kGraphIters;
-    } else {
-      for (int i = 0; i < batch; ++i)
-        if (int rc = body()) return rc;
-      launched += batch;
+  // the mirror sits behind the dots' result in the context's pinned block
+  CgMirror* mirror = reinterpret_cast<CgMirror*>(static_cast<char*>(ctx->host_pinned) + 256);
+  __atomic_store_n(&mirror->it, 0, __ATOMIC_RELAXED);
+  __atomic_store_n(&mirror->done, 0, __ATOMIC_RELEASE);
+  const CgVectors<T> v{inv, b, x, r, z, p, ap, st, ctx->red, mirror};
+  if (int rc = cg_setup<T>(ctx, n, op, v, rtol, atol, max_it, zeros)) return rc;
+  hipGraphExec_t exec = cg_solve_graph<T>(ctx, n, v, rtol, atol, max_it, op);
+  const int group = exec ? kGraphIters : 1;
+  int launched = 0;
+  for (uint64_t spins = 0; !__atomic_load_n(&mirror->done, __ATOMIC_ACQUIRE);) {
+    if (launched < max_it && launched - __atomic_load_n(&mirror->it, __ATOMIC_RELAXED) < kQueueAhead + group - 1) {
+      if (exec) {
+        FX_HIP(ctx, hipGraphLaunch(exec, s));
+      } else {
+        if (int rc = cg_iteration<T>(ctx, n, op, v)) return rc;
+        FX_HIP(ctx, hipGetLastError());
+      }
+      launched += group;
+      spins = 0;
+      continue;
     }
-    FX_HIP(ctx, hipGetLastError());
-    poll = std::min(poll * 2, 64);
+    if (++spins % 4096 == 0) {  // the queued work has ended without a stop: a device error
+      const hipError_t q = hipStreamQuery(s);
+      if (q == hipErrorNotReady) continue;
+      FX_HIP(ctx, q);
+      if (__atomic_load_n(&mirror->done, __ATOMIC_ACQUIRE)) break;
+      if (launched >= max_it || __atomic_load_n(&mirror->it, __ATOMIC_RELAXED) < launched) {
+        ctx->error = "CG: the device did not report the queued iterations";
+        return FX_EDEVICE;
+      }
+    }
   }
+  host = *mirror;
   return FX_OK;
+}
+
+// The Jacobi preconditioner 1 / diag(K_eff), queued; the count of zero entries in *zeros (device).
+int jacobi_queue(fx_batch* b, const fx_coeffs& k, double* d, void* inv, bool f32, int32_t** zeros) {
+  fx_ctx* ctx = b->ctx;
+  if (int rc = operator_diagonal64(b, k, d)) return rc;
+  int32_t* z = reinterpret_cast<int32_t*>(ctx->scalars) + 64;
+  FX_HIP(ctx, hipMemsetAsync(z, 0, sizeof(int32_t), ctx->stream));
+  if (f32)
+    hipLaunchKernelGGL(reciprocal_kernel<float>, grid_of(b->neq), dim3(256), 0, ctx->stream, b->neq, d,
+                       static_cast<float*>(inv), z);
+  else
+    hipLaunchKernelGGL(reciprocal_kernel<double>, grid_of(b->neq), dim3(256), 0, ctx->stream, b->neq, d,
+                       static_cast<double*>(inv), z);
+  FX_HIP(ctx, hipGetLastError());
+  *zeros = z;
+  return FX_OK;
+}
+
+int zero_diagonal(fx_ctx* ctx, int32_t zeros) {
+  ctx->error = "Jacobi: " + std::to_string(zeros) + " zero diagonal entries";
+  return FX_EZERO;
 }
 
 int jacobi_inverse(fx_batch* b, const fx_coeffs& k, double* d, void* inv, bool f32) {
   fx_ctx* ctx = b->ctx;
-  if (int rc = operator_diagonal64(b, k, d)) return rc;
-  int32_t* zeros = reinterpret_cast<int32_t*>(ctx->scalars) + 64;
-  FX_HIP(ctx, hipMemsetAsync(zeros, 0, sizeof(int32_t), ctx->stream));
-  if (f32)
-    hipLaunchKernelGGL(reciprocal_kernel<float>, grid_of(b->neq), dim3(256), 0, ctx->stream, b->neq, d,
-                       static_cast<float*>(inv), zeros);
-  else
-    hipLaunchKernelGGL(reciprocal_kernel<double>, grid_of(b->neq), dim3(256), 0, ctx->stream, b->neq, d,
-                       static_cast<double*>(inv), zeros);
-  FX_HIP(ctx, hipGetLastError());
-  int32_t hz = 0;
+  int32_t *zeros = nullptr, hz = 0;
+  if (int rc = jacobi_queue(b, k, d, inv, f32, &zeros)) return rc;
   FX_HIP(ctx, hipMemcpyAsync(&hz, zeros, sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream));
   FX_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  if (hz > 0) {
-    ctx->error = "Jacobi: " + std::to_string(hz) + " zero diagonal entries";
-    return FX_EZERO;
-  }
+  return hz > 0 ? zero_diagonal(ctx, hz) : FX_OK;
+}
+
+// ||b - A x|| in FP64, queued; its chunk partials reduced into the context's pinned block, which
+// holds the square once the stream is idle.
+int queue_residual_norm(fx_batch* b, const fx_coeffs& k, const double* bi, const double* xi, double* ap, double* r) {
+  fx_ctx* ctx = b->ctx;
+  const int64_t n = b->neq;
+  if (int rc = ensure_red(ctx, n)) return rc;
+  if (int rc = operator_apply64(b, k, xi, ap)) return rc;
+  double* nul = nullptr;
+  hipLaunchKernelGGL((residual_kernel<double, false>), chunk_grid(n), dim3(kVecThreads), 0, ctx->stream, n, bi, ap,
+                     static_cast<const double*>(nullptr), r, nul, nul, ctx->red);
+  hipLaunchKernelGGL(reduce_kernel, dim3(1), red_threads(n), 0, ctx->stream, chunks(n), 1, ctx->red,
+                     static_cast<const int32_t*>(nullptr), static_cast<double*>(ctx->host_pinned));
+  FX_HIP(ctx, hipGetLastError());
   return FX_OK;
+}
+// A solve's end: the true residual, x back to the caller's numbering, both in place on return.
+int finish_solve(fx_batch* b, const fx_coeffs& k, const double* bi, const double* xi, double* ap, double* r, double* x,
+                 fx_solve_result& res) {
+  if (int rc = queue_residual_norm(b, k, bi, xi, ap, r)) return rc;
+  if (int rc = to_external<double>(b, xi, x)) return rc;
+  FX_HIP(b->ctx, hipStreamSynchronize(b->ctx->stream));
+  res.true_residual = std::sqrt(*static_cast<const double*>(b->ctx->host_pinned));
+  return FX_OK;
+}
+
+void cg_result(const CgMirror& h, fx_solve_result& res) {
+  res = fx_solve_result{};
+  res.converged = h.converged;
+  res.iterations = h.it;
+  res.indefinite = h.indefinite;
+  res.rhs_norm = h.rhs_norm;
+  res.initial_residual = h.init_res;
+  res.final_residual = h.final_res;
 }
 
 }  // namespace
@@ -609,48 +747,29 @@ int cg64_solver(fx_batch* b, const fx_coeffs& k, const fx_solve_options& o, cons
   fx_ctx* ctx = b->ctx;
   const int64_t n = b->neq;
   double *r = b->work, *z = r + n, *p = z + n, *ap = p + n, *inv = ap + n, *d = inv + n;
-  if (int rc = jacobi_inverse(b, k, d, inv, false)) return rc;
-  CgState* st = static_cast<CgState*>(ctx->scalars);
-  CgState h{};
-  auto apply = [&](const double* xx, double* yy, const int32_t* dn) { return operator_apply64(b, k, xx, yy, dn); };
-  if (int rc = cg_device<double>(ctx, n, apply, inv, bi, xi, r, z, p, ap, st, o.relative_tolerance,
-                                 o.absolute_tolerance, o.max_iterations, h, b, &k))
+  int32_t* zeros = nullptr;
+  if (int rc = jacobi_queue(b, k, d, inv, false, &zeros)) return rc;
+  CgMirror h{};
+  if (int rc = cg_device<double>(ctx, n, BatchOp<double>{b, k}, inv, bi, xi, r, z, p, ap,
+                                 static_cast<CgState*>(ctx->scalars), o.relative_tolerance, o.absolute_tolerance,
+                                 o.max_iterations, zeros, h))
     return rc;
-  res = fx_solve_result{};
-  res.converged = h.converged;
-  res.iterations = h.it;
-  res.indefinite = h.indefinite;
-  res.rhs_norm = h.rhs_norm;
-  res.initial_residual = h.init_res;
-  res.final_residual = h.final_res;
+  if (h.zeros > 0) return zero_diagonal(ctx, h.zeros);
+  cg_result(h, res);
   return FX_OK;
 }
 
-namespace {
-int cg64_once(fx_batch* b, const fx_coeffs& k, const fx_solve_options& o, const double* rhs, double* x,
-              fx_solve_result& res) {
-  fx_ctx* ctx = b->ctx;
+int cg64(fx_batch* b, const fx_coeffs& k, const fx_solve_options& o, const double* rhs, double* x,
+         fx_solve_result& res) {
   const int64_t n = b->neq;
   double *r = b->work, *ap = r + 3 * n, *bi = r + 6 * n, *xi = r + 7 * n;
   if (int rc = to_internal<double>(b, rhs, bi)) return rc;
   if (int rc = to_internal<double>(b, x, xi)) return rc;
   if (int rc = cg64_solver(b, k, o, bi, xi, res)) return rc;
-  // true residual ||b - A x||
-  if (int rc = operator_apply64(b, k, xi, ap)) return rc;
-  hipLaunchKernelGGL(residual_kernel<double>, grid_of(n), dim3(256), 0, ctx->stream, n, bi, ap, r);
-  double rr = 0;
-  if (int rc = dot64(ctx, n, r, r, &rr)) return rc;
-  res.true_residual = std::sqrt(rr);
-  return to_external<double>(b, xi, x);
-}
-}  // namespace
-
-int cg64(fx_batch* b, const fx_coeffs& k, const fx_solve_options& o, const double* rhs, double* x,
-         fx_solve_result& res) {
-  return cg64_once(b, k, o, rhs, x, res);
+  return finish_solve(b, k, bi, xi, ap, r, x, res);
 }
 
-size_t cg_red_doubles(int64_t n) { return static_cast<size_t>(2 * chunks(n) + 2 * (chunks(chunks(n)) + 2) + 16); }
+size_t cg_red_doubles(int64_t n) { return static_cast<size_t>(3 * chunks(n) + 16); }
 
 // Several FP64 CG solves advanced together on one stream (the serving loop's admission round): each
 // poll round launches every unfinished solve's next group of iterations (a captured graph per
@@ -663,10 +782,8 @@ int cg64_many(int32_t nb, fx_batch* const* bs, const fx_coeffs& k, const fx_solv
   fx_ctx* ctx = bs[0]->ctx;
   hipStream_t s = ctx->stream;
   struct Solve {
-    fx_batch* b;
-    double *r, *z, *p, *ap, *inv, *d, *bi, *xi;
-    CgState* st;
-    double* red;
+    CgVectors<double> v;
+    double *bi, *xi;
     hipGraphExec_t exec;
     int launched;
     bool active;
@@ -676,62 +793,35 @@ int cg64_many(int32_t nb, fx_batch* const* bs, const fx_coeffs& k, const fx_solv
   for (int32_t i = 0; i < nb; ++i) {
     fx_batch* b = bs[i];
     const int64_t n = b->neq;
-    Solve& v = sv[i];
-    v.b = b;
-    v.r = b->work;
-    v.z = v.r + n;
-    v.p = v.z + n;
-    v.ap = v.p + n;
-    v.inv = v.ap + n;
-    v.d = v.inv + n;
-    v.bi = v.r + 6 * n;
-    v.xi = v.r + 7 * n;
-    v.st = reinterpret_cast<CgState*>(b->cg_state);
-    v.red = b->cg_red;
-    v.launched = 0;
-    v.active = true;
-    if (int rc = to_internal<double>(b, rhs[i], v.bi)) return rc;
-    if (int rc = to_internal<double>(b, x[i], v.xi)) return rc;
-    if (int rc = jacobi_inverse(b, k, v.d, v.inv, false)) return rc;
-    auto apply = [b, &k](const double* xx, double* yy, const int32_t* dn) { return operator_apply64(b, k, xx, yy, dn); };
-    if (int rc = cg_setup<double>(ctx, n, apply, v.inv, v.bi, v.xi, v.r, v.z, v.p, v.ap, v.st, v.red,
-                                  o.relative_tolerance, o.absolute_tolerance, o.max_iterations))
+    double *r = b->work, *inv = r + 4 * n, *bi = r + 6 * n, *xi = r + 7 * n;
+    sv[i] = Solve{CgVectors<double>{inv, bi, xi, r, r + n, r + 2 * n, r + 3 * n, reinterpret_cast<CgState*>(b->cg_state),
+                                    b->cg_red, nullptr},
+                  bi, xi, nullptr, 0, true};
+    if (int rc = to_internal<double>(b, rhs[i], bi)) return rc;
+    if (int rc = to_internal<double>(b, x[i], xi)) return rc;
+    if (int rc = jacobi_inverse(b, k, r + 5 * n, inv, false)) return rc;
+    const BatchOp<double> op{b, k};
+    if (int rc = cg_setup<double>(ctx, n, op, sv[i].v, o.relative_tolerance, o.absolute_tolerance, o.max_iterations,
+                                  nullptr))
       return rc;
-    auto body = [&, b, n]() -> int {
-      return cg_iteration<double>(ctx, n, apply, v.inv, v.xi, v.r, v.z, v.p, v.ap, v.st, v.red, o.relative_tolerance,
-                                  o.absolute_tolerance);
-    };
-    v.exec = cg_solve_graph<double>(ctx, n, v.inv, v.bi, v.xi, v.r, v.z, v.p, v.ap, v.st, v.red, o.relative_tolerance,
-                                    o.absolute_tolerance, o.max_iterations, b, &k, body);
+    sv[i].exec = cg_solve_graph<double>(ctx, n, sv[i].v, o.relative_tolerance, o.absolute_tolerance, o.max_iterations,
+                                        op);
   }
   const int max_it = o.max_iterations;
   for (int poll = 4, left = nb; left > 0; poll = std::min(poll * 2, 64)) {
     for (int32_t i = 0; i < nb; ++i)
       if (sv[i].active)
-        FX_HIP(ctx, hipMemcpyAsync(&host[i], sv[i].st, sizeof(CgState), hipMemcpyDeviceToHost, s));
+        FX_HIP(ctx, hipMemcpyAsync(&host[i], sv[i].v.st, sizeof(CgState), hipMemcpyDeviceToHost, s));
     FX_HIP(ctx, hipStreamSynchronize(s));
     for (int32_t i = 0; i < nb; ++i) {
       Solve& v = sv[i];
       if (!v.active) continue;
+      fx_batch* b = bs[i];
       const CgState& h = host[i];
       if (h.done || v.launched >= max_it) {
-        // finished: cg64_solver's result, then cg64_once's true residual and permutation
-        fx_batch* b = v.b;
-        const int64_t n = b->neq;
-        fx_solve_result& rs = res[i];
-        rs = fx_solve_result{};
-        rs.converged = h.converged;
-        rs.iterations = h.it;
-        rs.indefinite = h.indefinite;
-        rs.rhs_norm = h.rhs_norm;
-        rs.initial_residual = h.init_res;
-        rs.final_residual = h.final_res;
-        if (int rc = operator_apply64(b, k, v.xi, v.ap)) return rc;
-        hipLaunchKernelGGL(residual_kernel<double>, grid_of(n), dim3(256), 0, s, n, v.bi, v.ap, v.r);
-        double rr = 0;
-        if (int rc = dot64(ctx, n, v.r, v.r, &rr)) return rc;
-        rs.true_residual = std::sqrt(rr);
-        if (int rc = to_external<double>(b, v.xi, x[i])) return rc;
+        // finished: cg64_solver's result, then cg64's true residual and permutation
+        cg_result(CgMirror{h.rhs_norm, h.init_res, h.final_res, h.it, h.converged, h.indefinite, 0, 1, 0}, res[i]);
+        if (int rc = finish_solve(b, k, v.bi, v.xi, v.v.ap, v.v.r, x[i], res[i])) return rc;
         v.active = false;
         --left;
         continue;
@@ -742,15 +832,8 @@ int cg64_many(int32_t nb, fx_batch* const* bs, const fx_coeffs& k, const fx_solv
         for (int g = 0; g < graphs; ++g) FX_HIP(ctx, hipGraphLaunch(v.exec, s));
         v.launched += graphs * kGraphIters;
       } else {
-        const int64_t n = v.b->neq;
-        fx_batch* b = v.b;
-        auto apply = [b, &k](const double* xx, double* yy, const int32_t* dn) {
-          return operator_apply64(b, k, xx, yy, dn);
-        };
         for (int it = 0; it < batch; ++it)
-          if (int rc = cg_iteration<double>(ctx, n, apply, v.inv, v.xi, v.r, v.z, v.p, v.ap, v.st, v.red,
-                                            o.relative_tolerance, o.absolute_tolerance))
-            return rc;
+          if (int rc = cg_iteration<double>(ctx, b->neq, BatchOp<double>{b, k}, v.v)) return rc;
         v.launched += batch;
       }
       FX_HIP(ctx, hipGetLastError());
@@ -763,18 +846,12 @@ int cg64_many(int32_t nb, fx_batch* const* bs, const fx_coeffs& k, const fx_solv
 // the solver-numbering solve, the true residual reported.
 int krylov64(fx_batch* b, int method, const fx_coeffs& k, const fx_solve_options& o, const double* rhs, double* x,
              fx_solve_result& res) {
-  fx_ctx* ctx = b->ctx;
   const int64_t n = b->neq;
   double *r = b->work, *ap = r + 3 * n, *bi = r + 6 * n, *xi = r + 7 * n;
   if (int rc = to_internal<double>(b, rhs, bi)) return rc;
   if (int rc = to_internal<double>(b, x, xi)) return rc;
   if (int rc = method == 1 ? gmres64_solver(b, k, o, bi, xi, res) : krylov64_solver(b, k, o, bi, xi, res)) return rc;
-  if (int rc = operator_apply64(b, k, xi, ap)) return rc;
-  hipLaunchKernelGGL(residual_kernel<double>, grid_of(n), dim3(256), 0, ctx->stream, n, bi, ap, r);
-  double rr = 0;
-  if (int rc = dot64(ctx, n, r, r, &rr)) return rc;
-  res.true_residual = std::sqrt(rr);
-  return to_external<double>(b, xi, x);
+  return finish_solve(b, k, bi, xi, ap, r, x, res);
 }
 
 int cg_mixed(fx_batch* b, const fx_coeffs& k, const fx_solve_options& o, double inner_rtol, const double* rhs,
@@ -784,7 +861,9 @@ int cg_mixed(fx_batch* b, const fx_coeffs& k, const fx_solve_options& o, double 
   if (int rc = to_internal<double>(b, rhs, bi)) return rc;
   if (int rc = to_internal<double>(b, x, xi)) return rc;
   if (int rc = cg_mixed_solver(b, k, o, inner_rtol, bi, xi, res)) return rc;
-  return to_external<double>(b, xi, x);
+  if (int rc = to_external<double>(b, xi, x)) return rc;
+  FX_HIP(b->ctx, hipStreamSynchronize(b->ctx->stream));
+  return FX_OK;
 }
 
 int cg_mixed_solver(fx_batch* b, const fx_coeffs& k, const fx_solve_options& o, double inner_rtol, const double* bi,
@@ -807,14 +886,11 @@ int cg_mixed_solver(fx_batch* b, const fx_coeffs& k, const fx_solve_options& o, 
   res = fx_solve_result{};
   res.rhs_norm = bnorm;
   int total_inner = 0;
-  auto apply32 = [&](const float* xx, float* yy, const int32_t* dn) { return operator_apply32(b, k, xx, yy, dn); };
   for (int outer = 0;; ++outer) {
     // r = b - A x in FP64
-    if (int rc = operator_apply64(b, k, xi, ap64)) return rc;
-    hipLaunchKernelGGL(residual_kernel<double>, grid_of(n), dim3(256), 0, s, n, bi, ap64, r64);
-    double rr = 0;
-    if (int rc = dot64(ctx, n, r64, r64, &rr)) return rc;
-    const double rn = std::sqrt(rr);
+    if (int rc = queue_residual_norm(b, k, bi, xi, ap64, r64)) return rc;
+    FX_HIP(ctx, hipStreamSynchronize(s));
+    const double rn = std::sqrt(*static_cast<const double*>(ctx->host_pinned));
     if (outer == 0) res.initial_residual = rn;
     res.final_residual = res.true_residual = rn;
     res.outer_iterations = outer;
@@ -826,9 +902,9 @@ int cg_mixed_solver(fx_batch* b, const fx_coeffs& k, const fx_solve_options& o, 
     // inner FP32 solve of A d = r / ||r||
     hipLaunchKernelGGL(to_f32_kernel, grid_of(n), dim3(256), 0, s, n, r64, rhs32, 1.0 / rn);
     hipLaunchKernelGGL(zero_kernel<float>, grid_of(n), dim3(256), 0, s, n, dx);
-    CgState h{};
-    if (int rc = cg_device<float>(ctx, n, apply32, inv, rhs32, dx, r, z, p, ap, st, inner_rtol, 0.0,
-                                  o.max_iterations - total_inner, h, b, &k))
+    CgMirror h{};
+    if (int rc = cg_device<float>(ctx, n, BatchOp<float>{b, k}, inv, rhs32, dx, r, z, p, ap, st, inner_rtol, 0.0,
+                                  o.max_iterations - total_inner, nullptr, h))
       return rc;
     total_inner += h.it;
     if (h.indefinite) res.indefinite = 1;
@@ -903,13 +979,10 @@ int dot64_static(fx_ctx* ctx, int64_t n, const double* x, const double* y, doubl
     FX_HIP(ctx, hipGetLastError());
     return FX_OK;
   }
-  double* part = base;
-  double* tmp = base + chunks(n);
-  hipLaunchKernelGGL(chunk_dot_kernel<double>, dim3(static_cast<unsigned>(chunks(n))), dim3(kLanes), 0, s, n, x, y,
-                     static_cast<const double*>(nullptr), static_cast<const double*>(nullptr), part,
-                     static_cast<const int32_t*>(nullptr));
-  hipLaunchKernelGGL(reduce_kernel, dim3(1), red_threads(n), 0, s, chunks(n), 1, part, tmp,
-                     static_cast<CgState*>(nullptr), static_cast<int>(kStore), 0.0, 0.0, out_dev);
+  hipLaunchKernelGGL(chunk_dot_kernel<double>, dim3(static_cast<unsigned>(chunks(n))), dim3(kVecThreads), 0, s, n, x, y,
+                     base, static_cast<const int32_t*>(nullptr));
+  hipLaunchKernelGGL(reduce_kernel, dim3(1), red_threads(n), 0, s, chunks(n), 1, base,
+                     static_cast<const int32_t*>(nullptr), out_dev);
   FX_HIP(ctx, hipGetLastError());
   return FX_OK;
 }
