@@ -185,15 +185,18 @@ class BlockWorker(threading.Thread):
         if ctx is not None:
             ctx.close()
 
-    def _resident(self, ctx, resident, n):
+    def _resident(self, ctx, resident, n, keep=()):
         """The resident batch of block size n (built and uploaded on first use, least recently
-        used ones evicted to stay within the worker's share of the budget)."""
+        used ones evicted to stay within the worker's share of the budget), or None where it
+        would take the place of one of the sizes in keep."""
         if n in resident:
             resident.move_to_end(n)
             return resident[n]
         model, mesh, rhs = self.problems.get(n)
         need = _block_bytes(mesh.neq, self.mixed)
         while resident and self.used + need > self.budget:  # admission within the block share
+            if next(iter(resident)) in keep:
+                return None
             _, (batch, b, x, nb) = resident.popitem(last=False)
             batch.close()
             b.free()
@@ -207,14 +210,24 @@ class BlockWorker(threading.Thread):
         return resident[n]
 
     def _solve_round(self, ctx, resident, rs):
-        got = [self._resident(ctx, resident, r.n) for r in rs]
-        for _, _, x, _ in got:
-            x.zero()
-        res = core.cg_many(ctx, [g[0] for g in got], [g[1] for g in got], [g[2] for g in got], rtol=self.rtol)
-        for r, g, rr in zip(rs, got, res):
-            r.result = dict(rr)
-            if self.keep_x:
-                r.result["x"] = g[2].get()
+        while rs:
+            # the blocks that are resident together, the rest after them
+            now, later, got = [], [], []
+            for r in rs:
+                g = self._resident(ctx, resident, r.n, keep=[q.n for q in now])
+                if g is None:
+                    later.append(r)
+                else:
+                    now.append(r)
+                    got.append(g)
+            for _, _, x, _ in got:
+                x.zero()
+            res = core.cg_many(ctx, [g[0] for g in got], [g[1] for g in got], [g[2] for g in got], rtol=self.rtol)
+            for r, g, rr in zip(now, got, res):
+                r.result = dict(rr)
+                if self.keep_x:
+                    r.result["x"] = g[2].get()
+            rs = later
 
     def _solve(self, ctx, resident, r):
         batch, b, x, _ = self._resident(ctx, resident, r.n)
