@@ -307,8 +307,15 @@ __device__ __forceinline__ uint32_t interior_word(int ib, int ln) {
   return (7u << 28) | static_cast<uint32_t>(ib + 3 * ((x - 1) + (kTileX - 1) * ((y - 1) + (kTileY - 1) * (z - 1))));
 }
 
-template <typename T, bool DIAG, int TZ>
-__device__ __forceinline__ void fetch_tile(const BoxArgs<T>& a, int tile, int t, TileFetch<T, TZ>& f) {
+template <typename T, int TZ>
+struct NoPair {  // fetch_tile's second vector: none
+  __device__ void operator()(int, uint32_t, uint32_t) const {}
+};
+
+// pair(r, mask, first equation): a second vector's values at the nodes of round r, fetched beside x
+template <typename T, bool DIAG, int TZ, typename Pair = NoPair<T, TZ>>
+__device__ __forceinline__ void fetch_tile(const BoxArgs<T>& a, int tile, int t, TileFetch<T, TZ>& f,
+                                           const Pair& pair = Pair{}) {
   using G = TileGeom<TZ>;
   const uint32_t* words = a.words + static_cast<size_t>(tile) * G::kNodes;
   const int32_t* slots = a.slots + static_cast<size_t>(tile) * G::kNodes;
@@ -340,6 +347,7 @@ __device__ __forceinline__ void fetch_tile(const BoxArgs<T>& a, int tile, int t,
         j += (mask >> d) & 1u;
       }
     }
+    pair(r, mask, w[r] & 0x0fffffffu);
     f.w[r] = (w[r] & 0x80000000u) ? ((w[r] & 0xf0000000u) | static_cast<uint32_t>(s[r])) : w[r];
   }
 }
@@ -358,9 +366,26 @@ struct NoHook {
 // node sums need no bounds. Node (x, y, z) of the tile sits at x + 9 (y + 9 z') in LDS, with
 // z' = z (RING = 0: every node plane of the tile held) or z mod RING (a ring of RING planes).
 // mid() runs after the barrier that ends the pass's reads of x, before its commits.
+// cf: the cell's factors read ahead (a uniform lattice's stdBrick cells), or null.
+template <typename T>
+struct CellFactors {
+  T lam, mu, mc;
+  bool lumped;
+};
+template <typename T>
+__device__ __forceinline__ CellFactors<T> cell_factors(const BoxArgs<T>& a, int pidx, double dvol) {
+  if (pidx == 0xffff) return CellFactors<T>{T(0), T(0), T(0), false};
+  const DevParam& p = a.params[pidx];
+  double fD, cM;
+  operator_factors(p, a.k, fD, cM);
+  return CellFactors<T>{static_cast<T>(fD * p.lam * dvol), static_cast<T>(fD * p.mu * dvol),
+                        static_cast<T>(cM * p.rho * dvol), p.mass_type != 0};
+}
+
 template <typename T, int MODE, int TZ, int RING = 0, typename Mid = NoHook>
 __device__ __forceinline__ void box_tile(const BoxArgs<T>& a, int pidx, const T* xs, const uint32_t* wsh, T* top,
-                                         int t, int pass, int tile, const Mid& mid = Mid{}) {
+                                         int t, int pass, int tile, const Mid& mid = Mid{},
+                                         const CellFactors<T>* cf = nullptr) {
   using G = TileGeom<TZ>;
   constexpr bool DIAG = MODE % 3 == 2;
   constexpr bool SSP = MODE >= 3 && MODE < 6;
@@ -375,7 +400,12 @@ __device__ __forceinline__ void box_tile(const BoxArgs<T>& a, int pidx, const T*
   for (int c = 0; c < 3; ++c)
 #pragma unroll
     for (int q = 0; q < 8; ++q) out[c][q] = T(0);
-  if (pidx != 0xffff) {
+  if (cf && pidx != 0xffff) {
+    int ln[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) ln[q] = (cx + (q & 1)) + NX * (cy + ((q >> 1) & 1)) + kPlane * lp(cz + (q >> 2));
+    box_apply<T, MODE % 3 == 1, LDS_NODES>(xs, ln, cf->lam, cf->mu, cf->mc, cf->lumped, a.K, out);
+  } else if (pidx != 0xffff) {
     const DevParam& p = a.params[pidx];
     double fD, cM;
     operator_factors(p, a.k, fD, cM);
@@ -556,6 +586,69 @@ __global__ __launch_bounds__(kTileThreads, WAVES > 0 ? WAVES : 1) void hex8_box_
   }
 }
 
+// A CG iteration's tile: the stop test, then the direction p = z + beta p_old formed as the tile's
+// nodes are fetched (both vectors gathered where the plain product gathers p), the tile's own
+// nodes' p stored, and the product of p. Every workgroup adds the chunk partials of r.r and r.z
+// (waves 0 and 1) while its gathers are in flight, and takes the same decision from them.
+template <typename T, int MODE, int TZ>
+__global__ __launch_bounds__(kTileThreads) void hex8_box_cg_kernel(BoxArgs<T> a, CgDirection<T> d) {
+  using G = TileGeom<TZ>;
+  __shared__ T xs[3 * G::kNodes];
+  __shared__ uint32_t wsh[G::kNodes];
+  __shared__ T top[3 * G::kRing * kPlane];
+  __shared__ double row[2][kLanes];
+  __shared__ double tot[2];
+  const int t = threadIdx.x, wave = t / kLanes, l = t % kLanes;
+  const int tile = blockIdx.x;
+  const int stopped = d.st->done, it = d.st->it, max_it = d.st->max_it;
+  const double rz = d.st->rz, tol = d.st->tol;
+  TileFetch<T, TZ> f;
+  T q[G::kRounds][3];
+  a.x = d.z;
+  fetch_tile<T, false, TZ>(a, tile, t, f, [&](int r, uint32_t mask, uint32_t eq) {
+    const T* src = d.p_old + eq;
+    int j = 0;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      q[r][c] = (mask & (1u << c)) ? src[j] : T(0);
+      j += (mask >> c) & 1u;
+    }
+  });
+  constexpr bool AHEAD = MODE < 3;  // the cells' factors read beside the gathers, not after them
+  CellFactors<T> cf[G::kPasses];
+  if constexpr (AHEAD)
+#pragma unroll
+    for (int pass = 0; pass < G::kPasses; ++pass) cf[pass] = cell_factors(a, f.pidx[pass], a.hx * a.hy * a.hz * 0.125);
+  if (wave < 2) {
+    const double s = wave_total(d.part, 2, wave, d.npart, l, row[wave]);
+    if (l == 0) tot[wave] = s;
+  }
+  if (stopped) return;
+  __syncthreads();
+  double beta;
+  if (!cg_decide(d.st, d.mirror, it, max_it, tol, rz, tot[0], tot[1], tile == 0 && t == 0, beta)) return;
+  const T bt = static_cast<T>(beta);
+#pragma unroll
+  for (int r = 0; r < G::kRounds; ++r) {
+    const int ln = t + r * kTileThreads;
+    if (ln < G::kNodes) {
+      const uint32_t own = (f.w[r] & 0x80000000u) ? 0u : f.w[r];  // a node only this tile touches
+      wsh[ln] = f.w[r];
+      int j = 0;
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        const T p = it > 0 ? f.v[r][c] + bt * q[r][c] : f.v[r][c];
+        xs[c * G::kNodes + ln] = p;
+        if (own & (1u << (28 + c))) d.p[(own & 0x0fffffffu) + j++] = p;
+      }
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int pass = 0; pass < G::kPasses; ++pass)
+    box_tile<T, MODE, TZ>(a, f.pidx[pass], xs, wsh, top, t, pass, tile, NoHook{}, AHEAD ? &cf[pass] : nullptr);
+}
+
 // Streamed tiles: the x and the words of only five node planes sit in LDS, in rings (node plane
 // z at ring plane z mod 5, ring index = tile node index mod 405). The first five planes are
 // fetched before the first pass; each later pass's four new planes are loaded while the pass
@@ -704,50 +797,83 @@ __global__ __launch_bounds__(256) void hex8_shared_sum_kernel(const uint32_t* __
     if (mask & (1u << d)) y[base + j++] = acc[d];
 }
 
-// The same sums for the solvers' A p, in the pass that forms p.Ap: workgroup c takes the entries of
-// chunk c of VectorOps' order; an entry of the shared nodes' equations [e0, e0 + ne) is summed
-// from its tiles' partials (the order above, so the same bits) and stored, the others (the tiles'
-// own nodes; the tied sets, already summed) are read. at[2 e], at[2 e + 1]: a shared equation's
-// first partial, and 3 * (stride) | tiles << 28. One launch and one pass over y less than the
-// sums and the dot apart; 27,744 entries: 2.7 + 11.2 -> 3.5 us.
+// The same sums for a CG iteration's A p, in the pass that forms p.Ap: workgroup c takes the entries
+// of chunk c of VectorOps' order. The tiles' own equations [0, own) are read, p and y; past them
+// the direction is formed here, and y at a shared equation [e0, e0 + ne) is summed from its tiles'
+// partials (the order above, so the same bits) and stored (the tied sets are summed before).
+// at[2 e], at[2 e + 1]: a shared equation's first partial, and 3 * stride | tiles << 28. One
+// launch and one pass over y less than the sums and the dot apart.
 template <typename T>
-__global__ __launch_bounds__(kVecThreads) void hex8_sum_dot_kernel(int64_t n, int64_t e0, int64_t ne,
+__global__ __launch_bounds__(kVecThreads) void hex8_sum_dot_kernel(int64_t n, int64_t own, int64_t e0, int64_t ne,
                                                                    const uint32_t* __restrict__ at,
-                                                                   const T* __restrict__ partial,
-                                                                   const T* __restrict__ x, T* __restrict__ y,
-                                                                   double* __restrict__ part, const int32_t* done) {
-  if (done && *done) return;
+                                                                   const T* __restrict__ partial, T* __restrict__ y,
+                                                                   double* __restrict__ part, CgDirection<T> d) {
   __shared__ T xs[kChunk], ys[kChunk];
   __shared__ double row[kLanes];
   const int64_t begin = static_cast<int64_t>(blockIdx.x) * kChunk;
   const int len = static_cast<int>(n - begin < kChunk ? n - begin : kChunk);
   const int t = threadIdx.x;
+  const int stopped = d.st->done, it = d.st->it;
+  const T beta = static_cast<T>(d.st->beta);
   T xv[kPerThread], yv[kPerThread];
-  const bool sums = begin + len > e0 && begin < e0 + ne;
-  uint2 m[kPerThread];
-#pragma unroll
-  for (int j = 0; j < kPerThread; ++j) {
-    const int k = t + j * kVecThreads;
-    const int64_t i = begin + k, e = i - e0;
-    const bool mine = k < len && sums && e >= 0 && e < ne;
-    xv[j] = k < len ? x[i] : T(0);
-    yv[j] = k < len && !mine ? y[i] : T(0);
-    m[j] = mine ? reinterpret_cast<const uint2*>(at)[e] : uint2{0u, 0u};
-  }
-  if (sums) {
+  const bool past = begin + len > own;
+  // unconditional loads (an entry past the end reads the chunk's first), so that all are in flight
+  if (!past) {
 #pragma unroll
     for (int j = 0; j < kPerThread; ++j) {
-      const int tiles = static_cast<int>(m[j].y >> 28);
-      if (tiles == 0) continue;
-      const T* p = partial + m[j].x;
-      const size_t stride = m[j].y & 0x0fffffffu;
-      T v[8];
+      const int k = t + j * kVecThreads;
+      const int64_t i = begin + (k < len ? k : 0);
+      xv[j] = d.p[i];
+      yv[j] = y[i];
+    }
+    if (stopped) return;
+  } else {
+    const T* pp = d.z ? d.p_old : d.p;
+    const T* pz = d.z ? d.z : d.p;
+    T zv[kPerThread];
+    uint2 m[kPerThread];
 #pragma unroll
-      for (int q = 0; q < 8; ++q) v[q] = q < tiles ? p[q * stride] : T(0);
-      T acc = v[0];
+    for (int j = 0; j < kPerThread; ++j) {
+      const int k = t + j * kVecThreads;
+      const int64_t i = begin + (k < len ? k : 0), e = i - e0;
+      const bool sum = k < len && e >= 0 && e < ne;
+      m[j] = reinterpret_cast<const uint2*>(at)[sum ? e : 0];
+      if (!sum) m[j] = uint2{0u, 0u};
+      xv[j] = (i < own ? d.p : pp)[i];
+      zv[j] = pz[i];
+      yv[j] = y[i];
+    }
+    if (stopped) return;
 #pragma unroll
-      for (int q = 1; q < 8; ++q)
-        if (q < tiles) acc += v[q];
+    for (int j = 0; j < kPerThread; ++j) {
+      const int k = t + j * kVecThreads;
+      const int64_t i = begin + k;
+      if (k < len && i >= own && d.z) {
+        xv[j] = it == 0 ? zv[j] : zv[j] + beta * xv[j];
+        d.p[i] = xv[j];
+      }
+    }
+    // two tiles at almost every shared node (a face): their partials for all entries together,
+    // the further ones of edges and corners after them
+    T v0[kPerThread], v1[kPerThread];
+#pragma unroll
+    for (int j = 0; j < kPerThread; ++j) {
+      v0[j] = partial[m[j].x];
+      v1[j] = partial[m[j].x + (m[j].y & 0x0fffffffu)];
+    }
+#pragma unroll
+    for (int j = 0; j < kPerThread; ++j) {
+      const uint32_t tiles = m[j].y >> 28, stride = m[j].y & 0x0fffffffu;
+      if (tiles == 0u) continue;
+      T acc = v0[j] + v1[j];
+      if (tiles > 2u) {
+        T v[6];
+#pragma unroll
+        for (uint32_t q = 2; q < 8; ++q) v[q - 2] = q < tiles ? partial[m[j].x + q * stride] : T(0);
+#pragma unroll
+        for (uint32_t q = 2; q < 8; ++q)
+          if (q < tiles) acc += v[q - 2];
+      }
       yv[j] = acc;
       y[begin + t + j * kVecThreads] = acc;
     }
@@ -814,6 +940,59 @@ int resident_tiles(fx_ctx* ctx, const void* kernel) {
   }
   return cache[key] = per_cu * ncu;
 }
+
+// Up to this many tiles (one launch's worth of resident workgroups) the words of a tile's interior
+// nodes are loaded, not computed from the header's base: the header is one more round of memory
+// latency before the gathers, and the bytes it saves do not matter there.
+constexpr int kFewTiles = 1024;
+
+template <typename T>
+BoxArgs<T> box_args(fx_batch* b, const fx_coeffs& k, const T* x, T* y, int accumulate, const int32_t* done, int ref) {
+  BoxArgs<T> a{};
+  a.tiles = b->tiles;
+  a.words = ref ? b->words_ref : b->words;
+  a.slots = b->tile_slots;
+  a.use_interior = ref || b->ntiles <= kFewTiles ? 0 : 1;
+  a.cell_param = b->cell_param;
+  a.params = b->params;
+  a.k = k;
+  a.hx = b->hx;
+  a.hy = b->hy;
+  a.hz = b->hz;
+  const double kap[3] = {0.25 / b->hx, 0.25 / b->hy, 0.25 / b->hz};
+  for (int d = 0; d < 3; ++d) {
+    a.K.kap[d] = static_cast<T>(kap[d]);
+    a.K.w0[d] = static_cast<T>(8.0 * kap[d]);
+    a.K.w1[d] = static_cast<T>(8.0 / 3.0 * kap[d]);
+    a.K.kk[d] = static_cast<T>(8.0 / 9.0 * kap[d] * kap[d]);
+  }
+  a.K.kks = static_cast<T>(8.0 / 9.0 * (kap[0] * kap[0] + kap[1] * kap[1] + kap[2] * kap[2]));
+  a.x = x;
+  a.y = y;
+  if constexpr (sizeof(T) == 8) {
+    a.partial = b->partial64;
+  } else {
+    a.partial = b->partial32;
+  }
+  a.ntiles = b->ntiles;
+  a.accumulate = accumulate;
+  a.done = done;
+  a.ssp = b->ssp_box;
+  a.kx = b->kx;
+  a.ky = b->ky;
+  a.kz = b->kz;
+  return a;
+}
+
+// whether some parameter set has a mass factor cM' = cM + cC alphaM
+bool has_mass(const fx_batch* b, const fx_coeffs& k) {
+  for (const DevParam& p : b->host_params) {
+    double fD, cM;
+    operator_factors(p, k, fD, cM);
+    if (cM != 0.0) return true;
+  }
+  return false;
+}
 }  // namespace
 
 template <typename T, bool DIAG>
@@ -823,13 +1002,7 @@ int launch_box(fx_batch* b, const fx_coeffs& k, const T* x, T* y, int accumulate
     b->ctx->error = "operator: no reference-numbering words for this batch";
     return FX_EINVAL;
   }
-  // the mass-free kernel unless some parameter set has a mass factor cM' = cM + cC alphaM
-  bool mass = false;
-  for (const DevParam& p : b->host_params) {
-    double fD, cM;
-    operator_factors(p, k, fD, cM);
-    mass |= cM != 0.0;
-  }
+  const bool mass = has_mass(b, k);  // else the mass-free kernel
   // variant bits 0-1: the register budget of the mass-free kernel (the compiler's choice, or at
   // least 5, 7, 8 waves per SIMD: 84, 72, 64 VGPRs in FP64, the last two with a few spills; the
   // mass and diagonal kernels keep the compiler's choice); bit 2: persistent workgroups with
@@ -884,39 +1057,7 @@ int launch_box(fx_batch* b, const fx_coeffs& k, const T* x, T* y, int accumulate
     const int resident = resident_tiles(b->ctx, reinterpret_cast<const void*>(kernel));
     if (resident > 0 && resident < grid) grid = resident >= 8 ? resident / 8 * 8 : resident;
   }
-  BoxArgs<T> a{};
-  a.tiles = b->tiles;
-  a.words = ref ? b->words_ref : b->words;
-  a.slots = b->tile_slots;
-  a.use_interior = ref ? 0 : 1;
-  a.cell_param = b->cell_param;
-  a.params = b->params;
-  a.k = k;
-  a.hx = b->hx;
-  a.hy = b->hy;
-  a.hz = b->hz;
-  const double kap[3] = {0.25 / b->hx, 0.25 / b->hy, 0.25 / b->hz};
-  for (int d = 0; d < 3; ++d) {
-    a.K.kap[d] = static_cast<T>(kap[d]);
-    a.K.w0[d] = static_cast<T>(8.0 * kap[d]);
-    a.K.w1[d] = static_cast<T>(8.0 / 3.0 * kap[d]);
-    a.K.kk[d] = static_cast<T>(8.0 / 9.0 * kap[d] * kap[d]);
-  }
-  a.K.kks = static_cast<T>(8.0 / 9.0 * (kap[0] * kap[0] + kap[1] * kap[1] + kap[2] * kap[2]));
-  a.x = x;
-  a.y = y;
-  if constexpr (sizeof(T) == 8) {
-    a.partial = b->partial64;
-  } else {
-    a.partial = b->partial32;
-  }
-  a.ntiles = b->ntiles;
-  a.accumulate = accumulate;
-  a.done = done;
-  a.ssp = b->ssp_box;
-  a.kx = b->kx;
-  a.ky = b->ky;
-  a.kz = b->kz;
+  BoxArgs<T> a = box_args<T>(b, k, x, y, accumulate, done, ref);
   if (!a.partial) {
     b->ctx->error = "operator: no partial-sum buffer for this precision";
     return FX_EINVAL;
@@ -937,18 +1078,44 @@ template int launch_box<double, false>(fx_batch*, const fx_coeffs&, const double
 template int launch_box<double, true>(fx_batch*, const fx_coeffs&, const double*, double*, int, const int32_t*, int, bool);
 template int launch_box<float, false>(fx_batch*, const fx_coeffs&, const float*, float*, int, const int32_t*, int, bool);
 
+bool box_sums_with_dot(const fx_batch* b) {
+  return b->lattice && !b->pimy && b->norphans == 0 && !b->nodal_m && !b->nodal_am;
+}
+bool box_forms_direction(const fx_batch* b) {
+  return box_sums_with_dot(b) && b->tile_z != 16 && chunks(b->neq) <= kInlineParts;
+}
+
 template <typename T>
-int launch_box_dot(fx_batch* b, const fx_coeffs& k, const T* x, T* y, double* part, const int32_t* done) {
-  if (int rc = launch_box<T, false>(b, k, x, y, 0, done, 0, false)) return rc;
-  const T* partial;
-  if constexpr (sizeof(T) == 8) partial = b->partial64;
-  else partial = b->partial32;
-  hipLaunchKernelGGL(hex8_sum_dot_kernel<T>, dim3(static_cast<unsigned>(chunks(b->neq))), dim3(kVecThreads), 0,
-                     b->ctx->stream, b->neq, b->shared_eq0, b->shared_neq, b->shared_at, partial, x, y, part, done);
+int launch_box_cg(fx_batch* b, const fx_coeffs& k, const CgDirection<T>& d, T* y, double* part) {
+  using Kernel = void (*)(BoxArgs<T>, CgDirection<T>);
+#define FX_BOX_CG(TZ)                                                                                    \
+  {{hex8_box_cg_kernel<T, 0, TZ>, hex8_box_cg_kernel<T, 1, TZ>}, {hex8_box_cg_kernel<T, 3, TZ>, hex8_box_cg_kernel<T, 4, TZ>}, \
+   {hex8_box_cg_kernel<T, 6, TZ>, hex8_box_cg_kernel<T, 7, TZ>}}
+  static const Kernel table4[3][2] = FX_BOX_CG(4);
+  static const Kernel table8[3][2] = FX_BOX_CG(8);
+#undef FX_BOX_CG
+  const Kernel kernel = (b->tile_z == 8 ? table8 : table4)[b->ssp ? 1 : b->rect ? 2 : 0][has_mass(b, k) ? 1 : 0];
+  hipStream_t st = b->ctx->stream;
+  const int32_t* done = &d.st->done;
+  const BoxArgs<T> a = box_args<T>(b, k, static_cast<const T*>(nullptr), y, 0, done, 0);
+  if (!a.partial) {
+    b->ctx->error = "operator: no partial-sum buffer for this precision";
+    return FX_EINVAL;
+  }
+  if (d.z) {
+    hipLaunchKernelGGL(kernel, dim3(b->ntiles), dim3(kTileThreads), 0, st, a, d);
+    if (b->ntied > 0)
+      hipLaunchKernelGGL(hex8_tied_sum_kernel<T>, dim3((b->ntied + 3) / 4), dim3(256), 0, st, b->tied_word,
+                         b->tied_start, a.partial, y, b->ntied, 0, done);
+  } else if (int rc = launch_box<T, false>(b, k, d.p, y, 0, done, 0, false)) {
+    return rc;
+  }
+  hipLaunchKernelGGL(hex8_sum_dot_kernel<T>, dim3(static_cast<unsigned>(chunks(b->neq))), dim3(kVecThreads), 0, st,
+                     b->neq, b->own_neq, b->shared_eq0, b->shared_neq, b->shared_at, a.partial, y, part, d);
   FX_HIP(b->ctx, hipGetLastError());
   return FX_OK;
 }
-template int launch_box_dot<double>(fx_batch*, const fx_coeffs&, const double*, double*, double*, const int32_t*);
-template int launch_box_dot<float>(fx_batch*, const fx_coeffs&, const float*, float*, double*, const int32_t*);
+template int launch_box_cg<double>(fx_batch*, const fx_coeffs&, const CgDirection<double>&, double*, double*);
+template int launch_box_cg<float>(fx_batch*, const fx_coeffs&, const CgDirection<float>&, float*, double*);
 
 }  // namespace fx

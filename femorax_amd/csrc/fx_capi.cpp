@@ -510,7 +510,13 @@ int fx_batch_create(fx_ctx* ctx, const fx_batch_desc* d, uint32_t flags, fx_batc
         }
       }
       b->shared_neq = static_cast<int64_t>(at.size() / 2);
-      if (!at.empty()) ok(dev_upload(ctx, b->shared_at, at.data(), at.size(), by));
+      for (const uint32_t w : lat.words) {
+        const uint32_t mask = (w >> 28) & 7u;
+        if (mask && !(w & 0x80000000u))
+          b->own_neq = std::max<int64_t>(b->own_neq, static_cast<int64_t>(w & 0x0fffffffu) + __builtin_popcount(mask));
+      }
+      if (at.empty()) at.assign(2, 0u);  // read, not used
+      ok(dev_upload(ctx, b->shared_at, at.data(), at.size(), by));
     }
     // the node words in the reference numbering, where each node's free DOFs have consecutive
     // reference equations (so a word's first equation and mask still name them)

@@ -294,6 +294,7 @@ struct fx_batch {
   // first partial, then 3 * stride | tiles << 28
   uint32_t* shared_at = nullptr;
   int64_t shared_eq0 = 0, shared_neq = 0;
+  int64_t own_neq = 0;  // the equations of the nodes only one tile touches: [0, own_neq)
   double* partial64 = nullptr;        // [nslot * 3] per-tile sums at shared nodes
   float* partial32 = nullptr;
   int box_variant = 0;                // lattice kernel variant of the operator without mass terms (tuned)

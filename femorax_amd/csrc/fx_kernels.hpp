@@ -50,13 +50,20 @@ __host__ __device__ inline void operator_factors(const DevParam& p, const fx_coe
 template <typename T, bool DIAG>
 int launch_box(fx_batch* b, const fx_coeffs& k, const T* x, T* y, int accumulate, const int32_t* done, int ref = 0,
                bool sums = true);
-// A lattice product y = A x with the chunk partials of x.y (VectorOps' order) formed by the kernel
-// that adds the shared nodes' partial sums (solver numbering); for batches box_sums_with_dot takes.
-inline bool box_sums_with_dot(const fx_batch* b) {
-  return b->lattice && !b->pimy && b->norphans == 0 && !b->nodal_m && !b->nodal_am;
-}
+// A CG iteration's lattice product y = A p with the chunk partials of p.y (VectorOps' order), in a
+// tile launch and one that adds the shared nodes' partial sums (solver numbering); and in front
+// of it, where d.z is given, the stop test and the direction p = z + beta p_old, formed as the
+// tiles fetch it. box_sums_with_dot: the batches it takes (the product is the elements' alone).
+// box_forms_direction: those whose direction it forms: 4- and 8-deep tiles, few enough equations
+// that every tile adds up r.r and r.z itself. At 13,872 equations that saves a launch (3.7 us of
+// 24 us an iteration); at 6.4 M the second gather costs more than the pass it saves (75 + 32
+// against 21 + 52 + 28 us).
 template <typename T>
-int launch_box_dot(fx_batch* b, const fx_coeffs& k, const T* x, T* y, double* part, const int32_t* done);
+struct CgDirection;
+bool box_sums_with_dot(const fx_batch* b);
+bool box_forms_direction(const fx_batch* b);
+template <typename T>
+int launch_box_cg(fx_batch* b, const fx_coeffs& k, const CgDirection<T>& d, T* y, double* part);
 
 int operator_apply64(fx_batch* b, const fx_coeffs& k, const double* x, double* y, const int32_t* done = nullptr);
 int operator_apply32(fx_batch* b, const fx_coeffs& k, const float* x, float* y, const int32_t* done = nullptr);

@@ -24,42 +24,15 @@
 
 namespace fx {
 
-// The CG's scalars on the device. A field is written by one kernel of an iteration only and read
-// by the others: update_dot_kernel writes it and rz, direction_kernel rz_next and the stop's
-// fields, so that every workgroup of a kernel derives the same step from the same values.
-struct CgState {
-  double rz, rz_next, tol, rhs_norm, init_res, final_res;
-  int32_t it, done, converged, indefinite, max_it, zeros;
-};
-
-// The host's copy of a solve's progress, in pinned memory: the device writes `it` after each
-// iteration and, last of all, `done`, so the host neither copies nor synchronises to poll.
-struct CgMirror {
-  double rhs_norm, init_res, final_res;
-  int32_t it, converged, indefinite, zeros, done, pad;
-};
-
-__device__ inline void mirror_stop(CgMirror* m, const CgState* st, double final_res, int it, int converged) {
-  if (!m) return;
-  m->rhs_norm = st->rhs_norm;
-  m->init_res = st->init_res;
-  m->final_res = final_res;
-  m->converged = converged;
-  m->indefinite = st->indefinite;
-  m->zeros = st->zeros;
-  __hip_atomic_store(&m->it, it, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-  __hip_atomic_store(&m->done, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
 // Partial sums per chunk of x.y in VectorOps' lane order (one workgroup per chunk, see
 // kVecThreads). 27,744 entries (14 chunks): 11.2 -> 3 us; 6.4 M entries: HBM-bound either way.
 template <typename T>
 __global__ __launch_bounds__(kVecThreads) void chunk_dot_kernel(int64_t n, const T* __restrict__ x,
                                                                 const T* __restrict__ y, double* __restrict__ partial,
                                                                 const int32_t* done) {
-  if (done && *done) return;
   __shared__ T xs[kChunk], ys[kChunk];
   __shared__ double row[kLanes];
+  const int stopped = done ? *done : 0;
   const int64_t begin = static_cast<int64_t>(blockIdx.x) * kChunk;
   const int len = static_cast<int>(n - begin < kChunk ? n - begin : kChunk);
   const int t = threadIdx.x;
@@ -67,9 +40,11 @@ __global__ __launch_bounds__(kVecThreads) void chunk_dot_kernel(int64_t n, const
 #pragma unroll
   for (int j = 0; j < kPerThread; ++j) {
     const int k = t + j * kVecThreads;
-    xv[j] = k < len ? x[begin + k] : T(0);
-    yv[j] = k < len ? y[begin + k] : T(0);
+    const int64_t i = begin + (k < len ? k : 0);  // unconditional, so that all are in flight
+    xv[j] = x[i];
+    yv[j] = y[i];
   }
+  if (stopped) return;
 #pragma unroll
   for (int j = 0; j < kPerThread; ++j) {
     xs[t + j * kVecThreads] = xv[j];
@@ -135,9 +110,10 @@ __global__ __launch_bounds__(kVecThreads) void residual_kernel(int64_t n, const 
 #pragma unroll
   for (int j = 0; j < kPerThread; ++j) {
     const int k = t + j * kVecThreads;
-    bv[j] = k < len ? b[begin + k] : T(0);
-    av[j] = k < len ? ap[begin + k] : T(0);
-    if constexpr (START) iv[j] = k < len ? inv[begin + k] : T(0);
+    const int64_t i = begin + (k < len ? k : 0);
+    bv[j] = b[i];
+    av[j] = ap[i];
+    if constexpr (START) iv[j] = inv[i];
   }
 #pragma unroll
   for (int j = 0; j < kPerThread; ++j) {
@@ -181,6 +157,7 @@ __global__ __launch_bounds__(kVecThreads) void cg_start_kernel(int64_t nb, const
   st->tol = fmax(rtol * st->rhs_norm, atol);
   st->init_res = st->final_res = sqrt(tot[1]);
   st->rz = st->rz_next = tot[2];
+  st->beta = 0.0;
   st->it = 0;
   st->max_it = max_it;
   st->indefinite = 0;
@@ -201,10 +178,11 @@ __global__ __launch_bounds__(kVecThreads) void update_dot_kernel(int64_t n, CgSt
                                                                  const T* __restrict__ p, const T* __restrict__ ap,
                                                                  const T* __restrict__ inv, double* __restrict__ partial,
                                                                  CgMirror* mirror) {
-  if (st->done) return;
   __shared__ T rs[kChunk], zs[kChunk];
   __shared__ double row[2][kLanes];
   __shared__ double total;
+  const int stopped = st->done;
+  const double rz = st->rz_next;
   const int64_t begin = static_cast<int64_t>(blockIdx.x) * kChunk;
   const int len = static_cast<int>(n - begin < kChunk ? n - begin : kChunk);
   const int t = threadIdx.x, w = t / kLanes, l = t % kLanes;
@@ -223,6 +201,7 @@ __global__ __launch_bounds__(kVecThreads) void update_dot_kernel(int64_t n, CgSt
     const double s = wave_total(pap, 1, 0, npap, l, row[0]);
     if (l == 0) total = s;
   }
+  if (stopped) return;
   __syncthreads();
   if (!(total > 0.0)) {  // p.Ap <= 0: the operator is not positive definite (cg.cpp:49-53)
     if (blockIdx.x == 0 && t == 0) {
@@ -232,7 +211,6 @@ __global__ __launch_bounds__(kVecThreads) void update_dot_kernel(int64_t n, CgSt
     }
     return;
   }
-  const double rz = st->rz_next;
   const T alpha = static_cast<T>(rz / total);
   if (blockIdx.x == 0 && t == 0) {
     st->rz = rz;
@@ -259,52 +237,37 @@ __global__ __launch_bounds__(kVecThreads) void update_dot_kernel(int64_t n, CgSt
 }
 
 // The stop test on ||r|| (cg.cpp:60) and p = z + beta p (cg.cpp:68) from the chunk partials of r.r
-// and r.z: every workgroup takes the same decision; the first records it.
+// and r.z, for products that take p as it is (launch_box_cg's form it themselves). The loads are
+// issued before the stop flag is read: one round of memory latency, not two.
 template <typename T>
-__global__ __launch_bounds__(kVecThreads) void direction_kernel(int64_t n, CgState* st, int64_t npart,
-                                                                const double* __restrict__ part,
-                                                                const T* __restrict__ z, T* __restrict__ p,
-                                                                CgMirror* mirror) {
-  if (st->done) return;
+__global__ __launch_bounds__(kVecThreads) void direction_kernel(int64_t n, CgDirection<T> d) {
   __shared__ double row[2][kLanes];
   __shared__ double tot[2];
   const int64_t begin = static_cast<int64_t>(blockIdx.x) * kChunk;
   const int len = static_cast<int>(n - begin < kChunk ? n - begin : kChunk);
   const int t = threadIdx.x, w = t / kLanes, l = t % kLanes;
-  const int it = st->it, max_it = st->max_it;
-  const double rz = st->rz, tol = st->tol;
+  const int stopped = d.st->done, it = d.st->it, max_it = d.st->max_it;
+  const double rz = d.st->rz, tol = d.st->tol;
   T zv[kPerThread], pv[kPerThread];
 #pragma unroll
   for (int j = 0; j < kPerThread; ++j) {
     const int k = t + j * kVecThreads;
     const int64_t i = begin + (k < len ? k : 0);
-    zv[j] = z[i];
-    pv[j] = p[i];
+    zv[j] = d.z[i];
+    pv[j] = d.p_old[i];
   }
   if (w < 2) {
-    const double s = wave_total(part, 2, w, npart, l, row[w]);
+    const double s = wave_total(d.part, 2, w, d.npart, l, row[w]);
     if (l == 0) tot[w] = s;
   }
+  if (stopped) return;
   __syncthreads();
-  const double rn = sqrt(tot[0]);
-  const bool converged = rn <= tol, stop = converged || it >= max_it;
-  if (blockIdx.x == 0 && t == 0) {
-    st->final_res = rn;
-    st->rz_next = tot[1];
-    if (converged) st->converged = 1;
-    if (stop) {
-      st->done = 1;
-      mirror_stop(mirror, st, rn, it, converged);
-    } else if (mirror) {
-      __hip_atomic_store(&mirror->it, it, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
-  }
-  if (stop) return;
-  const T beta = static_cast<T>(tot[1] / rz);
+  double beta;
+  if (!cg_decide(d.st, d.mirror, it, max_it, tol, rz, tot[0], tot[1], blockIdx.x == 0 && t == 0, beta)) return;
 #pragma unroll
   for (int j = 0; j < kPerThread; ++j) {
     const int k = t + j * kVecThreads;
-    if (k < len) p[begin + k] = zv[j] + beta * pv[j];
+    if (k < len) d.p[begin + k] = zv[j] + static_cast<T>(beta) * pv[j];
   }
 }
 
@@ -481,7 +444,7 @@ struct CgGraphKey {
   int64_t n;
   int32_t tsize, initial;
   double ks, kd, km, rtol, atol;
-  const void* ptr[10];
+  const void* ptr[11];
   // the batch arrays the operator kernels read whose pointers change between calls: the
   // committed and trial histories swap on every commit (the committed tangent is formed from
   // the committed history), so each parity of the swap has its own graph
@@ -504,7 +467,7 @@ hipGraphExec_t cg_graph(fx_ctx* ctx, const CgGraphKey& key, Body body) {
   hipStream_t s = ctx->stream;
   if (hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) != hipSuccess) return nullptr;
   int rc = FX_OK;
-  for (int i = 0; i < kGraphIters && rc == FX_OK; ++i) rc = body();
+  for (int i = 0; i < kGraphIters && rc == FX_OK; ++i) rc = body(i);
   hipGraph_t graph = nullptr;
   const hipError_t ec = hipStreamEndCapture(s, &graph);
   hipGraphExec_t exec = nullptr;
@@ -533,7 +496,7 @@ Parts total_of(fx_ctx* ctx, int64_t n, int nv, const double* part, double* tot, 
 template <typename T>
 struct CgVectors {
   const T *inv, *b;
-  T *x, *r, *z, *p, *ap;
+  T *x, *r, *z, *p, *p2, *ap;  // p2: the direction's second buffer (products that form it)
   CgState* st;
   double* red;       // cg_red_doubles(n)
   CgMirror* mirror;  // or null
@@ -559,20 +522,34 @@ int cg_setup(fx_ctx* ctx, int64_t n, const Op& op, const CgVectors<T>& v, double
   return FX_OK;
 }
 
-// One CG iteration (cg.cpp:44-69): A p with p.Ap, the fused x, r, z update with r.r and r.z, the
-// stop test with the direction; a no-op once the state's stop flag is set.
+// One CG iteration (cg.cpp:44-69): A p with p.Ap, then the x, r, z update with r.r and r.z; a no-op
+// once the state's stop flag is set. The stop test and the next direction follow the update
+// (direction_kernel), or lead the next iteration's product where the operator forms its direction
+// itself: iteration i then writes p into buffer i mod 2. last: the stop test also runs by itself
+// (no iteration follows, or not before the host has looked).
 template <typename T, typename Op>
-int cg_iteration(fx_ctx* ctx, int64_t n, const Op& op, const CgVectors<T>& v) {
+int cg_iteration(fx_ctx* ctx, int64_t n, const Op& op, const CgVectors<T>& v, int i, bool last) {
   hipStream_t s = ctx->stream;
   double *p1 = v.red, *p2 = v.red + chunks(n), *tot = v.red + 3 * chunks(n);
   const int32_t* done = &v.st->done;
-  if (int rc = op.apply_dot(v.p, v.ap, p1, done)) return rc;
+  const bool own = op.own_direction();
+  T* p = own && (i & 1) ? v.p2 : v.p;
+  if (own) {
+    const CgDirection<T> d{v.st, v.mirror, chunks(n), p2, v.z, (i & 1) ? v.p : v.p2, p};
+    if (int rc = op.apply_dot(d, v.ap, p1)) return rc;
+  } else if (int rc = op.apply_dot(p, v.ap, p1, v.st)) {
+    return rc;
+  }
   const Parts pap = total_of(ctx, n, 1, p1, tot, done);
   hipLaunchKernelGGL(update_dot_kernel<T>, chunk_grid(n), dim3(kVecThreads), 0, s, n, v.st, pap.n, pap.p, v.x, v.r, v.z,
-                     v.p, v.ap, v.inv, p2, v.mirror);
+                     p, v.ap, v.inv, p2, v.mirror);
   const Parts rr = total_of(ctx, n, 2, p2, tot + 1, done);
-  hipLaunchKernelGGL(direction_kernel<T>, chunk_grid(n), dim3(kVecThreads), 0, s, n, v.st, rr.n, rr.p, v.z, v.p,
-                     v.mirror);
+  if (!own)
+    hipLaunchKernelGGL(direction_kernel<T>, chunk_grid(n), dim3(kVecThreads), 0, s, n,
+                       CgDirection<T>{v.st, v.mirror, rr.n, rr.p, v.z, p, p});
+  else if (last)  // the decision alone: no entry of p
+    hipLaunchKernelGGL(direction_kernel<T>, dim3(1), dim3(kVecThreads), 0, s, static_cast<int64_t>(0),
+                       CgDirection<T>{v.st, v.mirror, rr.n, rr.p, v.z, p, p});
   return FX_OK;
 }
 
@@ -585,8 +562,11 @@ struct BatchOp {
     if constexpr (sizeof(T) == 8) return operator_apply64(b, k, x, y, nullptr);
     else return operator_apply32(b, k, x, y, nullptr);
   }
-  int apply_dot(const T* p, T* ap, double* part, const int32_t* done) const {
-    if (box_sums_with_dot(b)) return launch_box_dot<T>(b, k, p, ap, part, done);
+  bool own_direction() const { return box_forms_direction(b); }
+  int apply_dot(const CgDirection<T>& d, T* ap, double* part) const { return launch_box_cg<T>(b, k, d, ap, part); }
+  int apply_dot(T* p, T* ap, double* part, CgState* st) const {
+    if (box_sums_with_dot(b)) return apply_dot(CgDirection<T>{st, nullptr, 0, nullptr, nullptr, nullptr, p}, ap, part);
+    const int32_t* done = &st->done;
     int rc;
     if constexpr (sizeof(T) == 8) rc = operator_apply64(b, k, p, ap, done);
     else rc = operator_apply32(b, k, p, ap, done);
@@ -613,11 +593,11 @@ hipGraphExec_t cg_solve_graph(fx_ctx* ctx, int64_t n, const CgVectors<T>& v, dou
   key.km = op.k.mass;
   key.rtol = rtol;
   key.atol = atol;
-  const void* ptrs[10] = {v.inv, v.b, v.x, v.r, v.z, v.p, v.ap, v.st, v.red, v.mirror};
-  for (int i = 0; i < 10; ++i) key.ptr[i] = ptrs[i];
+  const void* ptrs[11] = {v.inv, v.b, v.x, v.r, v.z, v.p, v.p2, v.ap, v.st, v.red, v.mirror};
+  for (int i = 0; i < 11; ++i) key.ptr[i] = ptrs[i];
   key.state[0] = owner->state_c;
   key.state[1] = owner->state_t;
-  return cg_graph(ctx, key, [&]() -> int { return cg_iteration<T>(ctx, n, op, v); });
+  return cg_graph(ctx, key, [&](int i) -> int { return cg_iteration<T>(ctx, n, op, v, i, i + 1 == kGraphIters); });
 }
 
 // Iterations queued beyond the last one the device has reported: enough to hide the host's launch
@@ -629,15 +609,15 @@ constexpr int kQueueAhead = 8;
 // solve's mirror. With graphs on, each group replays a captured graph of kGraphIters iterations
 // (the same kernels and arguments, so the same bits as launching them).
 template <typename T>
-int cg_device(fx_ctx* ctx, int64_t n, const BatchOp<T>& op, const T* inv, const T* b, T* x, T* r, T* z, T* p, T* ap,
-              CgState* st, double rtol, double atol, int max_it, const int32_t* zeros, CgMirror& host) {
+int cg_device(fx_ctx* ctx, int64_t n, const BatchOp<T>& op, const T* inv, const T* b, T* x, T* r, T* z, T* p, T* p2,
+              T* ap, CgState* st, double rtol, double atol, int max_it, const int32_t* zeros, CgMirror& host) {
   if (int rc = ensure_red(ctx, n)) return rc;
   hipStream_t s = ctx->stream;
   // the mirror sits behind the dots' result in the context's pinned block
   CgMirror* mirror = reinterpret_cast<CgMirror*>(static_cast<char*>(ctx->host_pinned) + 256);
   __atomic_store_n(&mirror->it, 0, __ATOMIC_RELAXED);
   __atomic_store_n(&mirror->done, 0, __ATOMIC_RELEASE);
-  const CgVectors<T> v{inv, b, x, r, z, p, ap, st, ctx->red, mirror};
+  const CgVectors<T> v{inv, b, x, r, z, p, p2, ap, st, ctx->red, mirror};
   if (int rc = cg_setup<T>(ctx, n, op, v, rtol, atol, max_it, zeros)) return rc;
   hipGraphExec_t exec = cg_solve_graph<T>(ctx, n, v, rtol, atol, max_it, op);
   const int group = exec ? kGraphIters : 1;
@@ -647,7 +627,7 @@ int cg_device(fx_ctx* ctx, int64_t n, const BatchOp<T>& op, const T* inv, const 
       if (exec) {
         FX_HIP(ctx, hipGraphLaunch(exec, s));
       } else {
-        if (int rc = cg_iteration<T>(ctx, n, op, v)) return rc;
+        if (int rc = cg_iteration<T>(ctx, n, op, v, launched, launched + 1 == max_it)) return rc;
         FX_HIP(ctx, hipGetLastError());
       }
       launched += group;
@@ -750,7 +730,7 @@ int cg64_solver(fx_batch* b, const fx_coeffs& k, const fx_solve_options& o, cons
   int32_t* zeros = nullptr;
   if (int rc = jacobi_queue(b, k, d, inv, false, &zeros)) return rc;
   CgMirror h{};
-  if (int rc = cg_device<double>(ctx, n, BatchOp<double>{b, k}, inv, bi, xi, r, z, p, ap,
+  if (int rc = cg_device<double>(ctx, n, BatchOp<double>{b, k}, inv, bi, xi, r, z, p, d, ap,
                                  static_cast<CgState*>(ctx->scalars), o.relative_tolerance, o.absolute_tolerance,
                                  o.max_iterations, zeros, h))
     return rc;
@@ -794,7 +774,7 @@ int cg64_many(int32_t nb, fx_batch* const* bs, const fx_coeffs& k, const fx_solv
     fx_batch* b = bs[i];
     const int64_t n = b->neq;
     double *r = b->work, *inv = r + 4 * n, *bi = r + 6 * n, *xi = r + 7 * n;
-    sv[i] = Solve{CgVectors<double>{inv, bi, xi, r, r + n, r + 2 * n, r + 3 * n, reinterpret_cast<CgState*>(b->cg_state),
+    sv[i] = Solve{CgVectors<double>{inv, bi, xi, r, r + n, r + 2 * n, r + 5 * n, r + 3 * n, reinterpret_cast<CgState*>(b->cg_state),
                                     b->cg_red, nullptr},
                   bi, xi, nullptr, 0, true};
     if (int rc = to_internal<double>(b, rhs[i], bi)) return rc;
@@ -833,7 +813,8 @@ int cg64_many(int32_t nb, fx_batch* const* bs, const fx_coeffs& k, const fx_solv
         v.launched += graphs * kGraphIters;
       } else {
         for (int it = 0; it < batch; ++it)
-          if (int rc = cg_iteration<double>(ctx, b->neq, BatchOp<double>{b, k}, v.v)) return rc;
+          if (int rc = cg_iteration<double>(ctx, b->neq, BatchOp<double>{b, k}, v.v, v.launched + it, it + 1 == batch))
+            return rc;
         v.launched += batch;
       }
       FX_HIP(ctx, hipGetLastError());
@@ -875,7 +856,8 @@ int cg_mixed_solver(fx_batch* b, const fx_coeffs& k, const fx_solve_options& o, 
   }
   const int64_t n = b->neq;
   double *r64 = b->work, *ap64 = r64 + 3 * n, *d64 = r64 + 5 * n;
-  float *inv = b->work32, *r = inv + n, *z = r + n, *p = z + n, *ap = p + n, *dx = ap + n, *rhs32 = dx + n;
+  float *inv = b->work32, *r = inv + n, *z = r + n, *p = z + n, *ap = p + n, *dx = ap + n, *rhs32 = dx + n,
+        *p2 = rhs32 + n;
   if (int rc = jacobi_inverse(b, k, d64, inv, true)) return rc;
   CgState* st = static_cast<CgState*>(ctx->scalars);
   hipStream_t s = ctx->stream;
@@ -903,7 +885,7 @@ int cg_mixed_solver(fx_batch* b, const fx_coeffs& k, const fx_solve_options& o, 
     hipLaunchKernelGGL(to_f32_kernel, grid_of(n), dim3(256), 0, s, n, r64, rhs32, 1.0 / rn);
     hipLaunchKernelGGL(zero_kernel<float>, grid_of(n), dim3(256), 0, s, n, dx);
     CgMirror h{};
-    if (int rc = cg_device<float>(ctx, n, BatchOp<float>{b, k}, inv, rhs32, dx, r, z, p, ap, st, inner_rtol, 0.0,
+    if (int rc = cg_device<float>(ctx, n, BatchOp<float>{b, k}, inv, rhs32, dx, r, z, p, p2, ap, st, inner_rtol, 0.0,
                                   o.max_iterations - total_inner, nullptr, h))
       return rc;
     total_inner += h.it;

@@ -1,4 +1,4 @@
-// Device pieces of VectorOps' dot order (vector_ops.cpp:19-64) shared by the Krylov kernels:
+// Device pieces of the Krylov kernels: the CG's state and VectorOps' dot order (vector_ops.cpp:19-64):
 // chunks of 2048 entries, lane l of 64 summing entries l, l + 64, ... of its chunk, the lane sums
 // added in lane order, chunk sums reduced level by level the same way.
 #pragma once
@@ -34,8 +34,12 @@ __device__ __forceinline__ double lane_order_sum(double s, int l, int lanes, dou
   __builtin_amdgcn_wave_barrier();
   double t = 0.0;
   if (lanes == kLanes) {
-#pragma unroll 16
-    for (int j = 0; j < kLanes; ++j) t += row[j];
+    // every read issued ahead of the 64 dependent adds
+    double v[kLanes];
+#pragma unroll
+    for (int j = 0; j < kLanes; ++j) v[j] = row[j];
+#pragma unroll
+    for (int j = 0; j < kLanes; ++j) t += v[j];
   } else {
     for (int j = 0; j < lanes; ++j) t += row[j];
   }
@@ -67,17 +71,88 @@ __device__ __forceinline__ double wave_total(const double* part, int nv, int v, 
   return wave_chunk_sum(part + v, nv, 0, npart, l, row);
 }
 
-// The dot of a staged chunk x.y (LDS, entries 0..len) by one wave, in VectorOps' order.
+// The dot of a staged chunk x.y (LDS, kChunk entries of which len count) by one wave, in
+// VectorOps' order.
 template <typename T>
 __device__ __forceinline__ double wave_staged_dot(const T* x, const T* y, int len, int l, double* row) {
   double s = 0.0;
-  if (len == kChunk) {
+  for (int k0 = 0; k0 < len; k0 += 16 * kLanes) {
+    T xv[16], yv[16];
 #pragma unroll
-    for (int j = 0; j < kChunk / kLanes; ++j) s += as_double(x[l + j * kLanes]) * as_double(y[l + j * kLanes]);
-  } else {
-    for (int k = l; k < len; k += kLanes) s += as_double(x[k]) * as_double(y[k]);
+    for (int j = 0; j < 16; ++j) {
+      xv[j] = x[k0 + l + j * kLanes];
+      yv[j] = y[k0 + l + j * kLanes];
+    }
+#pragma unroll
+    for (int j = 0; j < 16; ++j)
+      if (k0 + l + j * kLanes < len) s += as_double(xv[j]) * as_double(yv[j]);
   }
   return lane_order_sum(s, l, len < kLanes ? len : kLanes, row);
 }
+
+// The CG's scalars on the device. A field is written by one kernel of an iteration only and read
+// by the others: update_dot_kernel writes it and rz, the kernel that forms the direction
+// (cg_decide) rz_next, beta and the stop's fields, so that every workgroup of a kernel derives
+// the same step from the same values.
+struct CgState {
+  double rz, rz_next, beta, tol, rhs_norm, init_res, final_res;
+  int32_t it, done, converged, indefinite, max_it, zeros;
+};
+
+// The host's copy of a solve's progress, in pinned memory: the device writes `it` after each
+// iteration and, last of all, `done`, so the host neither copies nor synchronises to poll.
+struct CgMirror {
+  double rhs_norm, init_res, final_res;
+  int32_t it, converged, indefinite, zeros, done, pad;
+};
+
+__device__ inline void mirror_stop(CgMirror* m, const CgState* st, double final_res, int it, int converged) {
+  if (!m) return;
+  m->rhs_norm = st->rhs_norm;
+  m->init_res = st->init_res;
+  m->final_res = final_res;
+  m->converged = converged;
+  m->indefinite = st->indefinite;
+  m->zeros = st->zeros;
+  __hip_atomic_store(&m->it, it, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(&m->done, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// What every workgroup of the kernel that forms the direction decides from the totals of r.r and r.z
+// (cg.cpp:60-68): false once the solve stops, else the direction is z + beta p (it > 0) or z. The
+// kernel's first thread (first) records it.
+__device__ inline bool cg_decide(CgState* st, CgMirror* mirror, int it, int max_it, double tol, double rz, double rr,
+                                 double rz_next, bool first, double& beta) {
+  beta = 0.0;
+  if (it == 0) return true;  // cg_start_kernel has decided
+  const double rn = sqrt(rr);
+  const bool converged = rn <= tol, stop = converged || it >= max_it;
+  beta = rz_next / rz;
+  if (first) {
+    st->final_res = rn;
+    st->rz_next = rz_next;
+    st->beta = beta;
+    if (converged) st->converged = 1;
+    if (stop) {
+      st->done = 1;
+      mirror_stop(mirror, st, rn, it, converged);
+    } else if (mirror) {
+      __hip_atomic_store(&mirror->it, it, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+  }
+  return !stop;
+}
+
+// The CG vectors of a product that forms its own direction p = z + beta p_old (launch_box_cg), and
+// the chunk partials of r.r and r.z (or, n = 1, their totals).
+template <typename T>
+struct CgDirection {
+  CgState* st;
+  CgMirror* mirror;
+  int64_t npart;
+  const double* part;
+  const T *z, *p_old;
+  T* p;
+};
 
 }  // namespace fx
