@@ -753,14 +753,9 @@ __global__ __launch_bounds__(kTileThreads, WAVES > 0 ? WAVES : 1) void hex8_stre
 // tile, so the threads of a wave read each block contiguously. The shared nodes' equations are
 // consecutive in the internal numbering, in the same order.
 template <typename T>
-__global__ __launch_bounds__(256) void hex8_shared_sum_kernel(const uint32_t* __restrict__ word,
-                                                              const int32_t* __restrict__ start,
-                                                              const uint32_t* __restrict__ meta,
-                                                              const T* __restrict__ partial, T* __restrict__ y,
-                                                              int n, int accumulate, const int32_t* done) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  if (done && *done) return;
+__device__ __forceinline__ void shared_sum(int i, const uint32_t* __restrict__ word, const int32_t* __restrict__ start,
+                                           const uint32_t* __restrict__ meta, const T* __restrict__ partial,
+                                           T* __restrict__ y, int accumulate) {
   const uint32_t w = word[i];
   const uint32_t mask = (w >> 28) & 7u;
   const int base = static_cast<int>(w & 0x0fffffffu);
@@ -795,6 +790,18 @@ __global__ __launch_bounds__(256) void hex8_shared_sum_kernel(const uint32_t* __
 #pragma unroll
   for (int d = 0; d < 3; ++d)
     if (mask & (1u << d)) y[base + j++] = acc[d];
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void hex8_shared_sum_kernel(const uint32_t* __restrict__ word,
+                                                              const int32_t* __restrict__ start,
+                                                              const uint32_t* __restrict__ meta,
+                                                              const T* __restrict__ partial, T* __restrict__ y,
+                                                              int n, int accumulate, const int32_t* done) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  if (done && *done) return;
+  shared_sum(i, word, start, meta, partial, y, accumulate);
 }
 
 // The same sums for a CG iteration's A p, in the pass that forms p.Ap: workgroup c takes the entries
@@ -893,14 +900,9 @@ __global__ __launch_bounds__(kVecThreads) void hex8_sum_dot_kernel(int64_t n, in
 // column): the partial sums of every tile at every node of the set, one wave per set, the lanes
 // striding over the set's slots, then a butterfly over the lanes (a fixed order).
 template <typename T>
-__global__ __launch_bounds__(256) void hex8_tied_sum_kernel(const uint32_t* __restrict__ word,
-                                                            const int32_t* __restrict__ start,
-                                                            const T* __restrict__ partial, T* __restrict__ y, int n,
-                                                            int accumulate, const int32_t* done) {
-  const int u = static_cast<int>(blockIdx.x) * 4 + static_cast<int>(threadIdx.x) / 64;  // one set per wave
+__device__ __forceinline__ void tied_sum(int u, const uint32_t* __restrict__ word, const int32_t* __restrict__ start,
+                                         const T* __restrict__ partial, T* __restrict__ y, int accumulate) {
   const int lane = threadIdx.x % 64;
-  if (u >= n) return;  // the whole wave
-  if (done && *done) return;
   const int s0 = start[u], s1 = start[u + 1];
   T acc[3] = {T(0), T(0), T(0)};
   for (int s = s0 + lane; s < s1; s += 64)
@@ -920,6 +922,28 @@ __global__ __launch_bounds__(256) void hex8_tied_sum_kernel(const uint32_t* __re
     if (!(mask & (1u << d))) continue;
     T* dst = y + base + j++;
     *dst = accumulate ? *dst + acc[d] : acc[d];
+  }
+}
+
+// The tied sets (one wave each, four a workgroup) and, in the workgroups after the first
+// tied_blocks, the shared nodes: one launch for both, whose reads do not wait for each other
+// (40^3 column: 3.4 + 4.7 us in two launches).
+template <typename T>
+__global__ __launch_bounds__(256) void hex8_sums_kernel(const uint32_t* __restrict__ tied_word,
+                                                        const int32_t* __restrict__ tied_start, int ntied,
+                                                        const uint32_t* __restrict__ word,
+                                                        const int32_t* __restrict__ start,
+                                                        const uint32_t* __restrict__ meta, int nshared,
+                                                        const T* __restrict__ partial, T* __restrict__ y, int accumulate,
+                                                        const int32_t* done) {
+  if (done && *done) return;
+  const int tied_blocks = (ntied + 3) / 4, b = static_cast<int>(blockIdx.x);
+  if (b < tied_blocks) {
+    const int u = b * 4 + static_cast<int>(threadIdx.x) / 64;
+    if (u < ntied) tied_sum(u, tied_word, tied_start, partial, y, accumulate);
+  } else {
+    const int i = (b - tied_blocks) * 256 + static_cast<int>(threadIdx.x);
+    if (i < nshared) shared_sum(i, word, start, meta, partial, y, accumulate);
   }
 }
 
@@ -1063,13 +1087,16 @@ int launch_box(fx_batch* b, const fx_coeffs& k, const T* x, T* y, int accumulate
     return FX_EINVAL;
   }
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(kTileThreads), 0, b->ctx->stream, a);
-  if (b->nshared > 0 && sums)
-    hipLaunchKernelGGL(hex8_shared_sum_kernel<T>, dim3((b->nshared + 255) / 256), dim3(256), 0, b->ctx->stream,
-                       ref ? b->shared_word_ref : b->shared_word, b->shared_start, b->shared_meta, a.partial, y,
-                       b->nshared, accumulate, done);
+  const int nsh = sums ? b->nshared : 0;
   if (b->ntied > 0)
-    hipLaunchKernelGGL(hex8_tied_sum_kernel<T>, dim3((b->ntied + 3) / 4), dim3(256), 0, b->ctx->stream,
-                       ref ? b->tied_word_ref : b->tied_word, b->tied_start, a.partial, y, b->ntied, accumulate, done);
+    hipLaunchKernelGGL(hex8_sums_kernel<T>, dim3((b->ntied + 3) / 4 + (nsh + 255) / 256), dim3(256), 0, b->ctx->stream,
+                       ref ? b->tied_word_ref : b->tied_word, b->tied_start, b->ntied,
+                       ref ? b->shared_word_ref : b->shared_word, b->shared_start, b->shared_meta, nsh, a.partial, y,
+                       accumulate, done);
+  else if (nsh > 0)
+    hipLaunchKernelGGL(hex8_shared_sum_kernel<T>, dim3((nsh + 255) / 256), dim3(256), 0, b->ctx->stream,
+                       ref ? b->shared_word_ref : b->shared_word, b->shared_start, b->shared_meta, a.partial, y, nsh,
+                       accumulate, done);
   FX_HIP(b->ctx, hipGetLastError());
   return FX_OK;
 }
@@ -1105,8 +1132,8 @@ int launch_box_cg(fx_batch* b, const fx_coeffs& k, const CgDirection<T>& d, T* y
   if (d.z) {
     hipLaunchKernelGGL(kernel, dim3(b->ntiles), dim3(kTileThreads), 0, st, a, d);
     if (b->ntied > 0)
-      hipLaunchKernelGGL(hex8_tied_sum_kernel<T>, dim3((b->ntied + 3) / 4), dim3(256), 0, st, b->tied_word,
-                         b->tied_start, a.partial, y, b->ntied, 0, done);
+      hipLaunchKernelGGL(hex8_sums_kernel<T>, dim3((b->ntied + 3) / 4), dim3(256), 0, st, b->tied_word, b->tied_start,
+                         b->ntied, b->shared_word, b->shared_start, b->shared_meta, 0, a.partial, y, 0, done);
   } else if (int rc = launch_box<T, false>(b, k, d.p, y, 0, done, 0, false)) {
     return rc;
   }

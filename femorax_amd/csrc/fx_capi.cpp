@@ -105,7 +105,7 @@ int fx_ctx_create(int device, uint64_t hbm_budget_bytes, fx_ctx** out) {
   size_t fr = 0, tot = 0;
   (void)hipMemGetInfo(&fr, &tot);
   c->budget = hbm_budget_bytes ? hbm_budget_bytes : static_cast<uint64_t>(fr / 10 * 9);
-  if (hipHostMalloc(&c->host_pinned, 4096, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
+  if (hipHostMalloc(&c->host_pinned, kPinnedBytes, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
     (void)hipStreamDestroy(c->stream);
     delete c;
     return fail(nullptr, FX_EDEVICE, "hipHostMalloc failed");

@@ -119,6 +119,8 @@ void build_contraction(int32_t nnode, int32_t neq, const int32_t* node_eq, Contr
 
 }  // namespace fx
 
+constexpr size_t kPinnedBytes = 16384;
+
 // A captured run of CG iterations (cg_device): the key holds everything the kernels' arguments
 // depend on, owner the batch whose arrays they read (its graphs go when the batch goes).
 struct fx_cg_graph {
@@ -138,7 +140,9 @@ struct fx_ctx {
   double* red = nullptr;  // partial sums
   size_t red_cap = 0;
   void* scalars = nullptr;  // solver state block (device)
-  void* host_pinned = nullptr;  // 4 KB the device writes: a dot's result, a CG solve's progress
+  // kPinnedBytes the device writes: a dot's result (0), a CG solve's progress (256), GMRES' Hessenberg
+  // columns (512)
+  void* host_pinned = nullptr;
   void* pimy_params = nullptr;  // material-point driver: up to kMaxPointMaterials parameter sets
   bool use_graphs = false;      // CG iterations replayed from captured graphs (FX_OPT_GRAPHS)
   hipStream_t own_stream = nullptr;  // the stream the context created (stream is the caller's with FX_OPT_STREAM)
@@ -194,12 +198,12 @@ namespace fx {
 constexpr int kMaxPointLoads = 32;
 constexpr int kMaxPointMaterials = 8;
 constexpr int kGmresRestart = 30;  // GMRES(30) (gmres.hpp default restart)
-// doubles of the GMRES workspace (FX_BATCH_GMRES): V (m + 1 columns), Z (m), the initial guess,
-// the combine coefficients, and the block dots' chunk partials and level buffers
+// doubles of the GMRES workspace (FX_BATCH_GMRES): V (m + 1 columns), Z (m + 1), the initial guess,
+// the combine coefficients, the two passes' chunk partials of m + 1 dots and their totals
 inline size_t gmres_workspace(int64_t n) {
-  const int64_t ch = (n + 2047) / 2048, lvl = 2 * ((ch + 2047) / 2048 + 2);
-  return static_cast<size_t>(2 * kGmresRestart + 3) * static_cast<size_t>(n > 0 ? n : 1) + kGmresRestart + 1 +
-         static_cast<size_t>(kGmresRestart + 1) * static_cast<size_t>(ch + lvl + 1);
+  const int64_t ch = (n + 2047) / 2048;
+  return static_cast<size_t>(2 * kGmresRestart + 3) * static_cast<size_t>(n > 0 ? n : 1) +
+         static_cast<size_t>(kGmresRestart + 1) * static_cast<size_t>(2 * ch + 4);
 }
 struct PimyParams;
 // PressureIndependMultiYield (fx_pimy_host.cpp, fx_pimy.hip)
@@ -349,7 +353,7 @@ struct fx_batch {
   int32_t nlong = 0;
   std::vector<int8_t> eq_dir;
   int8_t* eq_dir_dev = nullptr;  // the same on the device, solver numbering (explicit ground loads)
-  // GMRES workspace (FX_BATCH_GMRES): V [(m + 1) n], Z [m n], coefficients [m + 1], CG start [n]
+  // GMRES workspace (FX_BATCH_GMRES, gmres_workspace)
   double* gm = nullptr;
   // nodal masses of the model (fx_batch_set_nodal_mass), solver numbering; the elements' own
   // lumped masses (host, solver numbering) that the lumped arrays add them to

@@ -105,3 +105,31 @@ def test_stop_is_seen_without_iterations_to_spare(ctx):
     dx.zero()
     assert batch.cg(db, dx, rtol=1e-10)["iterations"] == r["iterations"]
     batch.close()
+
+
+@pytest.mark.parametrize("name", ["one_element", "chunk_plus", "tied", "general", "rows_of_tiles"])
+def test_gmres_steps_match_oracle(ctx, name):
+    """The Arnoldi steps kept on the device: the first steps, a whole cycle, one step past it, and a
+    stop inside a cycle with steps still queued (the same counts and residuals as the oracle's
+    host loop, whose dots have the same order). Two Gram-Schmidt passes keep the basis orthogonal
+    to rounding, so x moves by about the condition number of the projected system times 1e-16."""
+    model = CASES[name]()
+    pm = core.Mesh(model)
+    params = pm.params_for(model)
+    batch = core.Batch(ctx, pm, params, gmres=True)
+    om, op = fxo.OracleMesh(model), fxo.elastic_params(params)
+    b = meshes.random_vector(pm.neq, 5)
+    db, dx = core.DeviceArray.from_host(ctx, b), core.DeviceArray(ctx, pm.neq)
+    for its in (1, 2, 30, 31, 37):
+        if its > pm.neq:
+            continue
+        dx.zero()
+        r = batch.gmres(db, dx, rtol=1e-12, max_it=its)
+        xo, ro = om.gmres(op, b, rtol=1e-12, max_it=its)
+        assert r["iterations"] == ro["iterations"] and r["converged"] == ro["converged"]
+        assert np.max(np.abs(dx.get() - xo)) <= 1e-9 * np.max(np.abs(xo)), (name, its)
+    dx.zero()
+    r = batch.gmres(db, dx, rtol=0.3)
+    _, ro = om.gmres(op, b, rtol=0.3)
+    assert r["converged"] and r["iterations"] == ro["iterations"]
+    batch.close()
