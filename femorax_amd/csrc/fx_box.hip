@@ -25,6 +25,7 @@
 
 #include "fx_internal.hpp"
 #include "fx_kernels.hpp"
+#include "fx_step_device.hpp"
 #include "fx_vecops.hpp"
 
 namespace fx {
@@ -130,16 +131,10 @@ __device__ __forceinline__ void box_constant_strain(const T (&b)[3][8], T lam, T
   }
 }
 
-template <typename T, bool MASS, int NODES>
-__device__ __forceinline__ void box_apply(const T* xs, const int (&ln)[8], T lam, T mu, T mc, bool lumped,
-                                          const BoxConst<T>& K, T (&y)[3][8]) {
-  T b[3][8];
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-#pragma unroll
-    for (int q = 0; q < 8; ++q) b[c][q] = xs[c * NODES + ln[q]];
-    hadamard8(b[c]);
-  }
+// The stiffness's modal gradient y from the modal values b = H v.
+template <typename T>
+__device__ __forceinline__ void box_stiffness_modes(const T (&b)[3][8], T lam, T mu, const BoxConst<T>& K,
+                                                    T (&y)[3][8]) {
   const T m2 = mu + mu;
   box_constant_strain(b, lam, mu, K, y);
   // the bilinear modes that vary along p: rows d1, d2 (the other axes) of the gradient's p-linear
@@ -177,16 +172,37 @@ __device__ __forceinline__ void box_apply(const T* xs, const int (&ln)[8], T lam
   }
 #pragma unroll
   for (int c = 0; c < 3; ++c) y[c][0] = T(0);
-  if (MASS && !lumped) {
-    // consistent mass: g[c][m] += mc / (8 3^|m|) b[c][m]
+}
+
+// Consistent mass: g[c][m] += mc / (8 3^|m|) b[c][m]
+template <typename T>
+__device__ __forceinline__ void box_mass_modes(const T (&b)[3][8], T mc, T (&y)[3][8]) {
 #pragma unroll
-    for (int m = 0; m < 8; ++m) {
-      const int w = (m & 1) + ((m >> 1) & 1) + ((m >> 2) & 1);
-      const T f = mc * T(w == 0 ? 1.0 / 8.0 : w == 1 ? 1.0 / 24.0 : w == 2 ? 1.0 / 72.0 : 1.0 / 216.0);
+  for (int m = 0; m < 8; ++m) {
+    const int w = (m & 1) + ((m >> 1) & 1) + ((m >> 2) & 1);
+    const T f = mc * T(w == 0 ? 1.0 / 8.0 : w == 1 ? 1.0 / 24.0 : w == 2 ? 1.0 / 72.0 : 1.0 / 216.0);
 #pragma unroll
-      for (int c = 0; c < 3; ++c) y[c][m] += f * b[c][m];
-    }
+    for (int c = 0; c < 3; ++c) y[c][m] += f * b[c][m];
   }
+}
+
+template <typename T, int NODES>
+__device__ __forceinline__ void box_modes(const T* xs, const int (&ln)[8], T (&b)[3][8]) {
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) b[c][q] = xs[c * NODES + ln[q]];
+    hadamard8(b[c]);
+  }
+}
+
+template <typename T, bool MASS, int NODES>
+__device__ __forceinline__ void box_apply(const T* xs, const int (&ln)[8], T lam, T mu, T mc, bool lumped,
+                                          const BoxConst<T>& K, T (&y)[3][8]) {
+  T b[3][8];
+  box_modes<T, NODES>(xs, ln, b);
+  box_stiffness_modes(b, lam, mu, K, y);
+  if (MASS && !lumped) box_mass_modes(b, mc, y);
 #pragma unroll
   for (int c = 0; c < 3; ++c) hadamard8_transposed(y[c]);
   if (MASS && lumped) {
@@ -356,6 +372,89 @@ struct NoHook {
   __device__ void operator()() const {}
 };
 
+// A rectilinear lattice's cell: its sizes and modal constants from its plane intervals.
+template <typename T>
+__device__ __forceinline__ void cell_geometry(const BoxArgs<T>& a, int tile, int cx, int cy, int cz, double (&hc)[3],
+                                              BoxConst<T>& Kc) {
+  const TileHeader& th = a.tiles[tile];
+  const double* kh[3] = {a.kx + 2 * (th.ox + cx), a.ky + 2 * (th.oy + cy), a.kz + 2 * (th.oz + cz)};
+  double ks = 0.0;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    const double kap = kh[d][0];
+    hc[d] = kh[d][1];
+    Kc.kap[d] = static_cast<T>(kap);
+    Kc.w0[d] = static_cast<T>(8.0 * kap);
+    Kc.w1[d] = static_cast<T>(8.0 / 3.0 * kap);
+    Kc.kk[d] = static_cast<T>(8.0 / 9.0 * kap * kap);
+    ks += kap * kap;
+  }
+  Kc.kks = static_cast<T>(8.0 / 9.0 * ks);
+}
+
+// The node sums of one pass's cell results and their commits (commit(ln, val[3]): tile node ln's
+// sum over the tile). mid() runs after the barrier that ends the pass's reads of x, before the
+// commits.
+template <typename T, int TZ, int RING, typename Mid, typename Commit>
+__device__ __forceinline__ void box_sum_commit(const T (&out)[3][8], T* top, int t, int pass, const Mid& mid,
+                                               const Commit& commit) {
+  using G = TileGeom<TZ>;
+  constexpr int NX = kTileX + 1;
+  auto lp = [](int z) { return RING ? z % RING : z; };
+  const int cx = t % kTileX, cy = (t / kTileX) % kTileY;
+  const int cz = __builtin_amdgcn_readfirstlane(t / (kTileX * kTileY)) + 4 * pass;  // one plane per wave
+  // in-plane sums, x first then y: the cell's corners a (cx, cy), b (cx+1, cy), c (cx, cy+1),
+  // d (cx+1, cy+1) of its bottom (k = 0) or top (k = 1) face. Row sums p = a + b(t-1) at node
+  // (cx, cy) and q = c + d(t-1) at (cx, cy+1); then node (cx, cy) gets m = p + q(t-8), node
+  // (cx+1, cy) e = b + d(t-8). A missing neighbour (cx = 0 or cy = 0) enters with factor 0 (a
+  // fused multiply-add by 1 is the plain sum). The last column and row of cells also keep e, q
+  // and d for the x = 8 column, y = 8 row and their corner. Top-face sums go to the LDS ring
+  // (the plane above reads them), bottom-face sums stay in registers.
+  const T fx = cx > 0 ? T(1) : T(0), fy = cy > 0 ? T(1) : T(0);
+  const bool xe = cx == kTileX - 1, ye = cy == kTileY - 1;
+  const int pi[4] = {cx + NX * cy, (cx + 1) + NX * cy, cx + NX * (cy + 1), (cx + 1) + NX * (cy + 1)};
+  const bool has[4] = {true, xe, ye, xe && ye};
+  auto slot = [&](int c, int plane) { return (c * G::kRing + plane % G::kRing) * kPlane; };
+  T F0[3][4];  // bottom face: [component][main, x edge, y edge, corner]
+#pragma unroll
+  for (int k = 1; k >= 0; --k)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const T oa = out[c][4 * k], ob = out[c][1 + 4 * k], oc = out[c][2 + 4 * k], od = out[c][3 + 4 * k];
+      const T p = fma_t(lane_up1(ob), fx, oa);
+      const T q = fma_t(lane_up1(od), fx, oc);
+      const T m = fma_t(shfl_up(q, kTileX), fy, p);
+      const T e = fma_t(shfl_up(od, kTileX), fy, ob);
+      const T f[4] = {m, e, q, od};
+      if (k == 1) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (has[r]) top[slot(c, cz) + pi[r]] = f[r];
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) F0[c][r] = f[r];
+      }
+    }
+  __syncthreads();
+  mid();
+  // commit: plane z = cz (bottom face + the plane below's top face), and for the last plane of
+  // cells also plane z = TZ (its own top face)
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    if (!has[r]) continue;
+    T val[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) val[c] = cz > 0 ? F0[c][r] + top[slot(c, cz - 1) + pi[r]] : F0[c][r];
+    commit(pi[r] + kPlane * lp(cz), val);
+    if (cz == TZ - 1) {
+      T up[3];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) up[c] = top[slot(c, cz) + pi[r]];
+      commit(pi[r] + kPlane * lp(cz + 1), up);
+    }
+  }
+}
+
 // One pass of a tile: cell (cx, cy, cz = wave + 4 pass). MODE: 0 apply without mass terms, 1
 // apply with mass terms, 2 diagonal; 3, 4, 5 the same for SSPbrick cells; 6, 7, 8 the same on a
 // rectilinear lattice (each cell's spacings from the tile's origin). The cell's results are
@@ -365,7 +464,6 @@ struct NoHook {
 // (zero results) and a node past it has no word (nothing fetched, nothing committed), so the
 // node sums need no bounds. Node (x, y, z) of the tile sits at x + 9 (y + 9 z') in LDS, with
 // z' = z (RING = 0: every node plane of the tile held) or z mod RING (a ring of RING planes).
-// mid() runs after the barrier that ends the pass's reads of x, before its commits.
 // cf: the cell's factors read ahead (a uniform lattice's stdBrick cells), or null.
 template <typename T>
 struct CellFactors {
@@ -413,22 +511,7 @@ __device__ __forceinline__ void box_tile(const BoxArgs<T>& a, int pidx, const T*
     // the cell's plane intervals
     double hc[3] = {a.hx, a.hy, a.hz};
     BoxConst<T> Kc = a.K;
-    if constexpr (RECT) {
-      const TileHeader& th = a.tiles[tile];
-      const double* kh[3] = {a.kx + 2 * (th.ox + cx), a.ky + 2 * (th.oy + cy), a.kz + 2 * (th.oz + cz)};
-      double ks = 0.0;
-#pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        const double kap = kh[d][0];
-        hc[d] = kh[d][1];
-        Kc.kap[d] = static_cast<T>(kap);
-        Kc.w0[d] = static_cast<T>(8.0 * kap);
-        Kc.w1[d] = static_cast<T>(8.0 / 3.0 * kap);
-        Kc.kk[d] = static_cast<T>(8.0 / 9.0 * kap * kap);
-        ks += kap * kap;
-      }
-      Kc.kks = static_cast<T>(8.0 / 9.0 * ks);
-    }
+    if constexpr (RECT) cell_geometry(a, tile, cx, cy, cz, hc, Kc);
     const double dvol = hc[0] * hc[1] * hc[2] * 0.125;
     if constexpr (DIAG && SSP) {
       // diag(K_e) per corner, kept per parameter set, and the lumped mass
@@ -472,42 +555,6 @@ __device__ __forceinline__ void box_tile(const BoxArgs<T>& a, int pidx, const T*
                                                p.mass_type != 0, Kc, out);
     }
   }
-  // in-plane sums, x first then y: the cell's corners a (cx, cy), b (cx+1, cy), c (cx, cy+1),
-  // d (cx+1, cy+1) of its bottom (k = 0) or top (k = 1) face. Row sums p = a + b(t-1) at node
-  // (cx, cy) and q = c + d(t-1) at (cx, cy+1); then node (cx, cy) gets m = p + q(t-8), node
-  // (cx+1, cy) e = b + d(t-8). A missing neighbour (cx = 0 or cy = 0) enters with factor 0 (a
-  // fused multiply-add by 1 is the plain sum). The last column and row of cells also keep e, q
-  // and d for the x = 8 column, y = 8 row and their corner. Top-face sums go to the LDS ring
-  // (the plane above reads them), bottom-face sums stay in registers.
-  const T fx = cx > 0 ? T(1) : T(0), fy = cy > 0 ? T(1) : T(0);
-  const bool xe = cx == kTileX - 1, ye = cy == kTileY - 1;
-  const int pi[4] = {cx + NX * cy, (cx + 1) + NX * cy, cx + NX * (cy + 1), (cx + 1) + NX * (cy + 1)};
-  const bool has[4] = {true, xe, ye, xe && ye};
-  auto slot = [&](int c, int plane) { return (c * G::kRing + plane % G::kRing) * kPlane; };
-  T F0[3][4];  // bottom face: [component][main, x edge, y edge, corner]
-#pragma unroll
-  for (int k = 1; k >= 0; --k)
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      const T oa = out[c][4 * k], ob = out[c][1 + 4 * k], oc = out[c][2 + 4 * k], od = out[c][3 + 4 * k];
-      const T p = fma_t(lane_up1(ob), fx, oa);
-      const T q = fma_t(lane_up1(od), fx, oc);
-      const T m = fma_t(shfl_up(q, kTileX), fy, p);
-      const T e = fma_t(shfl_up(od, kTileX), fy, ob);
-      const T f[4] = {m, e, q, od};
-      if (k == 1) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (has[r]) top[slot(c, cz) + pi[r]] = f[r];
-      } else {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) F0[c][r] = f[r];
-      }
-    }
-  __syncthreads();
-  mid();
-  // commit: plane z = cz (bottom face + the plane below's top face), and for the last plane of
-  // cells also plane z = TZ (its own top face)
   auto commit = [&](int ln, const T (&val)[3]) {
     const uint32_t w = wsh[ln];
     const uint32_t idx = w & 0x0fffffffu;
@@ -532,20 +579,7 @@ __device__ __forceinline__ void box_tile(const BoxArgs<T>& a, int pidx, const T*
       }
     }
   };
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    if (!has[r]) continue;
-    T val[3];
-#pragma unroll
-    for (int c = 0; c < 3; ++c) val[c] = cz > 0 ? F0[c][r] + top[slot(c, cz - 1) + pi[r]] : F0[c][r];
-    commit(pi[r] + kPlane * lp(cz), val);
-    if (cz == TZ - 1) {
-      T up[3];
-#pragma unroll
-      for (int c = 0; c < 3; ++c) up[c] = top[slot(c, cz) + pi[r]];
-      commit(pi[r] + kPlane * lp(cz + 1), up);
-    }
-  }
+  box_sum_commit<T, TZ, RING>(out, top, t, pass, mid, commit);
 }
 
 // One workgroup per tile (PERSIST: each workgroup walks tiles blockIdx.x, + gridDim.x, ...
@@ -647,6 +681,124 @@ __global__ __launch_bounds__(kTileThreads) void hex8_box_cg_kernel(BoxArgs<T> a,
 #pragma unroll
   for (int pass = 0; pass < G::kPasses; ++pass)
     box_tile<T, MODE, TZ>(a, f.pidx[pass], xs, wsh, top, t, pass, tile, NoHook{}, AHEAD ? &cf[pass] : nullptr);
+}
+
+// The elements' internal force K u + C v - F_body in one tile pass (std_brick.hpp:493-543): the
+// stiffness acts on u + beta v (beta = betaK + betaKinit + betaKcomm of the cell's parameter set,
+// elastic: every stiffness term has the tangent D), the alphaM mass on v, and a cell's body force
+// is b V / 8 at each corner, so neither C v, its sum with K u nor F_body is a pass of its own.
+// PAIR: with velocities v (times vscale); else K u - F_body. STEP: an equation whose force is
+// complete here (a node only this tile touches) takes the CentralDifference update on the spot,
+// so the force is never stored: U(n+1) over U(n-1), which no other tile reads at such a node.
+template <int MODE, int TZ, bool PAIR, bool STEP>
+__global__ __launch_bounds__(kTileThreads) void hex8_box_force_kernel(BoxArgs<double> a, const double* v, double vscale,
+                                                                      CdStep g) {
+  using G = TileGeom<TZ>;
+  constexpr bool RECT = MODE >= 6;
+  constexpr int NX = kTileX + 1;
+  __shared__ double xs[3 * G::kNodes];
+  __shared__ double vs[PAIR ? 3 * G::kNodes : 1];
+  __shared__ uint32_t wsh[G::kNodes];
+  __shared__ double top[3 * G::kRing * kPlane];
+  const int t = threadIdx.x, tile = blockIdx.x;
+  TileFetch<double, TZ> f;
+  double q[G::kRounds][3];
+  fetch_tile<double, false, TZ>(a, tile, t, f, [&](int r, uint32_t mask, uint32_t eq) {
+    if constexpr (PAIR) {
+      const double* src = v + eq;
+      int j = 0;
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        q[r][c] = (mask & (1u << c)) ? src[j] : 0.0;
+        j += (mask >> c) & 1u;
+      }
+    }
+  });
+#pragma unroll
+  for (int r = 0; r < G::kRounds; ++r) {
+    const int ln = t + r * kTileThreads;
+    if (ln < G::kNodes) {
+      wsh[ln] = f.w[r];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        xs[c * G::kNodes + ln] = f.v[r][c];
+        if constexpr (PAIR) vs[c * G::kNodes + ln] = q[r][c];
+      }
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int pass = 0; pass < G::kPasses; ++pass) {
+    const int cx = t % kTileX, cy = (t / kTileX) % kTileY;
+    const int cz = __builtin_amdgcn_readfirstlane(t / (kTileX * kTileY)) + 4 * pass;
+    double out[3][8];
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+      for (int k = 0; k < 8; ++k) out[c][k] = 0.0;
+    const int pidx = f.pidx[pass];
+    if (pidx != 0xffff) {
+      const DevParam& p = a.params[pidx];
+      double hc[3] = {a.hx, a.hy, a.hz};
+      BoxConst<double> Kc = a.K;
+      if constexpr (RECT) cell_geometry(a, tile, cx, cy, cz, hc, Kc);
+      const double dvol = hc[0] * hc[1] * hc[2] * 0.125;
+      int ln[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) ln[k] = (cx + (k & 1)) + NX * (cy + ((k >> 1) & 1)) + kPlane * (cz + (k >> 2));
+      if constexpr (PAIR) {
+        const double beta = vscale * (p.betaK + p.betaKinit + p.betaKcomm), mc = vscale * p.alphaM * p.rho * dvol;
+        double b[3][8], bv[3][8];
+        box_modes<double, G::kNodes>(vs, ln, bv);
+        box_modes<double, G::kNodes>(xs, ln, b);
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+          for (int k = 0; k < 8; ++k) b[c][k] += beta * bv[c][k];
+        box_stiffness_modes(b, p.lam * dvol, p.mu * dvol, Kc, out);
+        if (p.mass_type == 0) box_mass_modes(bv, mc, out);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) hadamard8_transposed(out[c]);
+        if (p.mass_type != 0)
+#pragma unroll
+          for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int k = 0; k < 8; ++k) out[c][k] += mc * vs[c * G::kNodes + ln[k]];
+      } else {
+        box_apply<double, false, G::kNodes>(xs, ln, p.lam * dvol, p.mu * dvol, 0.0, false, Kc, out);
+      }
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        const double bc = p.b[c] * dvol;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) out[c][k] -= bc;
+      }
+    }
+    box_sum_commit<double, TZ, 0>(out, top, t, pass, NoHook{}, [&](int ln, const double (&val)[3]) {
+      const uint32_t w = wsh[ln];
+      const uint32_t idx = w & 0x0fffffffu;
+      if (w & 0x80000000u) {
+        double* dst = a.partial + static_cast<size_t>(idx) * 3;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) dst[d] = val[d];
+        return;
+      }
+      int j = 0;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        if (!(w & (1u << (28 + d)))) continue;
+        const uint32_t e = idx + j++;
+        if constexpr (STEP) {
+          double um;
+          if constexpr (PAIR) um = vs[d * G::kNodes + ln];
+          else um = g.um[e];
+          g.um[e] = cd_next(g, e, val[d], xs[d * G::kNodes + ln], um);
+        } else {
+          a.y[e] = val[d];
+        }
+      }
+    });
+  }
 }
 
 // Streamed tiles: the x and the words of only five node planes sit in LDS, in rings (node plane
@@ -752,10 +904,11 @@ __global__ __launch_bounds__(kTileThreads, WAVES > 0 ? WAVES : 1) void hex8_stre
 // thread per shared node; a group of nodes with the same tiles keeps one block of slots per
 // tile, so the threads of a wave read each block contiguously. The shared nodes' equations are
 // consecutive in the internal numbering, in the same order.
-template <typename T>
+// add: values the sum starts from (y += the sum), or null; store(equation, sum)
+template <typename T, typename Store>
 __device__ __forceinline__ void shared_sum(int i, const uint32_t* __restrict__ word, const int32_t* __restrict__ start,
                                            const uint32_t* __restrict__ meta, const T* __restrict__ partial,
-                                           T* __restrict__ y, int accumulate) {
+                                           const T* add, const Store& store) {
   const uint32_t w = word[i];
   const uint32_t mask = (w >> 28) & 7u;
   const int base = static_cast<int>(w & 0x0fffffffu);
@@ -769,7 +922,7 @@ __device__ __forceinline__ void shared_sum(int i, const uint32_t* __restrict__ w
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
       acc[d] = p[d];
-      if (accumulate && (mask & (1u << d))) acc[d] = y[base + j] + acc[d];
+      if (add && (mask & (1u << d))) acc[d] = add[base + j] + acc[d];
       j += (mask >> d) & 1u;
     }
   }
@@ -789,7 +942,7 @@ __device__ __forceinline__ void shared_sum(int i, const uint32_t* __restrict__ w
   int j = 0;
 #pragma unroll
   for (int d = 0; d < 3; ++d)
-    if (mask & (1u << d)) y[base + j++] = acc[d];
+    if (mask & (1u << d)) store(base + j++, acc[d]);
 }
 
 template <typename T>
@@ -801,7 +954,8 @@ __global__ __launch_bounds__(256) void hex8_shared_sum_kernel(const uint32_t* __
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   if (done && *done) return;
-  shared_sum(i, word, start, meta, partial, y, accumulate);
+  shared_sum(i, word, start, meta, partial, accumulate ? y : static_cast<const T*>(nullptr),
+             [&](int64_t e, T f) { y[e] = f; });
 }
 
 // The same sums for a CG iteration's A p, in the pass that forms p.Ap: workgroup c takes the entries
@@ -899,9 +1053,9 @@ __global__ __launch_bounds__(kVecThreads) void hex8_sum_dot_kernel(int64_t n, in
 // y at tied equation sets (nodes that hold the same equations: the laminar ties of a soil
 // column): the partial sums of every tile at every node of the set, one wave per set, the lanes
 // striding over the set's slots, then a butterfly over the lanes (a fixed order).
-template <typename T>
+template <typename T, typename Store>
 __device__ __forceinline__ void tied_sum(int u, const uint32_t* __restrict__ word, const int32_t* __restrict__ start,
-                                         const T* __restrict__ partial, T* __restrict__ y, int accumulate) {
+                                         const T* __restrict__ partial, const Store& store) {
   const int lane = threadIdx.x % 64;
   const int s0 = start[u], s1 = start[u + 1];
   T acc[3] = {T(0), T(0), T(0)};
@@ -920,8 +1074,7 @@ __device__ __forceinline__ void tied_sum(int u, const uint32_t* __restrict__ wor
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
     if (!(mask & (1u << d))) continue;
-    T* dst = y + base + j++;
-    *dst = accumulate ? *dst + acc[d] : acc[d];
+    store(base + j++, acc[d]);
   }
 }
 
@@ -940,10 +1093,33 @@ __global__ __launch_bounds__(256) void hex8_sums_kernel(const uint32_t* __restri
   const int tied_blocks = (ntied + 3) / 4, b = static_cast<int>(blockIdx.x);
   if (b < tied_blocks) {
     const int u = b * 4 + static_cast<int>(threadIdx.x) / 64;
-    if (u < ntied) tied_sum(u, tied_word, tied_start, partial, y, accumulate);
+    if (u < ntied)
+      tied_sum(u, tied_word, tied_start, partial, [&](int64_t e, T f) { y[e] = accumulate ? y[e] + f : f; });
   } else {
     const int i = (b - tied_blocks) * 256 + static_cast<int>(threadIdx.x);
-    if (i < nshared) shared_sum(i, word, start, meta, partial, y, accumulate);
+    if (i < nshared)
+      shared_sum(i, word, start, meta, partial, accumulate ? y : static_cast<const T*>(nullptr),
+                 [&](int64_t e, T f) { y[e] = f; });
+  }
+}
+
+// The shared and tied equations of a CentralDifference step (hex8_box_force_kernel<STEP>): their
+// force summed as above and updated on the spot.
+__global__ __launch_bounds__(256) void hex8_step_sums_kernel(const uint32_t* __restrict__ tied_word,
+                                                             const int32_t* __restrict__ tied_start, int ntied,
+                                                             const uint32_t* __restrict__ word,
+                                                             const int32_t* __restrict__ start,
+                                                             const uint32_t* __restrict__ meta, int nshared,
+                                                             const double* __restrict__ partial,
+                                                             const double* __restrict__ u, CdStep g) {
+  const int tied_blocks = (ntied + 3) / 4, b = static_cast<int>(blockIdx.x);
+  auto update = [&](int64_t e, double f) { g.um[e] = cd_next(g, e, f, u[e], g.um[e]); };
+  if (b < tied_blocks) {
+    const int n = b * 4 + static_cast<int>(threadIdx.x) / 64;
+    if (n < ntied) tied_sum(n, tied_word, tied_start, partial, update);
+  } else {
+    const int i = (b - tied_blocks) * 256 + static_cast<int>(threadIdx.x);
+    if (i < nshared) shared_sum(i, word, start, meta, partial, static_cast<const double*>(nullptr), update);
   }
 }
 
@@ -1104,6 +1280,36 @@ int launch_box(fx_batch* b, const fx_coeffs& k, const T* x, T* y, int accumulate
 template int launch_box<double, false>(fx_batch*, const fx_coeffs&, const double*, double*, int, const int32_t*, int, bool);
 template int launch_box<double, true>(fx_batch*, const fx_coeffs&, const double*, double*, int, const int32_t*, int, bool);
 template int launch_box<float, false>(fx_batch*, const fx_coeffs&, const float*, float*, int, const int32_t*, int, bool);
+
+bool box_forms_force(const fx_batch* b) {
+  return b->lattice && !b->pimy && !b->ssp && b->tile_z != 16 && b->norphans == 0;
+}
+
+int launch_box_force(fx_batch* b, const double* u, const double* v, double vscale, double* f, int ref,
+                     const CdStep* step) {
+  using Kernel = void (*)(BoxArgs<double>, const double*, double, CdStep);
+#define FX_BOX_FORCE(M, TZ)                                                                     \
+  {{hex8_box_force_kernel<M, TZ, false, false>, hex8_box_force_kernel<M, TZ, false, true>},      \
+   {hex8_box_force_kernel<M, TZ, true, false>, hex8_box_force_kernel<M, TZ, true, true>}}
+  static const Kernel table[2][2][2][2] = {{FX_BOX_FORCE(0, 4), FX_BOX_FORCE(0, 8)},
+                                           {FX_BOX_FORCE(6, 4), FX_BOX_FORCE(6, 8)}};
+#undef FX_BOX_FORCE
+  const BoxArgs<double> a = box_args<double>(b, fx_coeffs{1.0, 0.0, 0.0, 0}, u, f, 0, nullptr, ref);
+  hipStream_t st = b->ctx->stream;
+  const Kernel kernel = table[b->rect ? 1 : 0][b->tile_z == 8 ? 1 : 0][v ? 1 : 0][step ? 1 : 0];
+  hipLaunchKernelGGL(kernel, dim3(b->ntiles), dim3(kTileThreads), 0, st, a, v, vscale, step ? *step : CdStep{});
+  const uint32_t *tw = ref ? b->tied_word_ref : b->tied_word, *sw = ref ? b->shared_word_ref : b->shared_word;
+  const dim3 grid((b->ntied + 3) / 4 + (b->nshared + 255) / 256);
+  const int32_t* always = nullptr;
+  if (grid.x > 0 && step)
+    hipLaunchKernelGGL(hex8_step_sums_kernel, grid, dim3(256), 0, st, tw, b->tied_start, b->ntied, sw, b->shared_start,
+                       b->shared_meta, b->nshared, b->partial64, u, *step);
+  else if (grid.x > 0)
+    hipLaunchKernelGGL(hex8_sums_kernel<double>, grid, dim3(256), 0, st, tw, b->tied_start, b->ntied, sw,
+                       b->shared_start, b->shared_meta, b->nshared, b->partial64, f, 0, always);
+  FX_HIP(b->ctx, hipGetLastError());
+  return FX_OK;
+}
 
 bool box_sums_with_dot(const fx_batch* b) {
   return b->lattice && !b->pimy && b->norphans == 0 && !b->nodal_m && !b->nodal_am;

@@ -1147,7 +1147,12 @@ int fx_force(fx_batch* b, const double* u, const double* v, double* f) {
   FX_HIP(b->ctx, hipSetDevice(b->ctx->device));
   const size_t n = static_cast<size_t>(b->neq);
   double* W = b->work;
-  if (b->internal) {
+  // a lattice's force on the caller's vectors in place (f apart from u and v)
+  auto apart = [&](const double* x) { return !x || x + n <= f || f + n <= x; };
+  if (fx::box_forms_force(b) && b->words_ref && !b->nodal_am && apart(u) && apart(v)) {
+    const double* vd = v && fx::elements_damp(b) ? v : nullptr;
+    if (int rc = fx::launch_box_force(b, u, vd, 1.0, f, 1, nullptr)) return rc;
+  } else if (b->internal) {
     if (int rc = fx::to_internal<double>(b, u, W)) return rc;
     if (v)
       if (int rc = fx::to_internal<double>(b, v, W + n)) return rc;

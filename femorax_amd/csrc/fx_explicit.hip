@@ -19,6 +19,7 @@
 
 #include "fx_internal.hpp"
 #include "fx_kernels.hpp"
+#include "fx_step_device.hpp"
 
 namespace fx {
 
@@ -58,29 +59,15 @@ __global__ void point_load_kernel(PointLoads p, double* f) {
 
 struct CdArgs {
   int32_t n;
-  double c2, c3, dt;
+  double dt;
   const double* f;     // K u (+ loads folded in)
   const double* fd;    // C v_e of the elements, or null
   const double* body;  // F_body, or null
-  const double* m;
-  const double* am;    // lumped alphaM mass, or null
-  const double* dash;  // dampers outside the elements, or null
   const double* u;     // U(n)
-  double* um;          // in: U(n-1); out: U(n+1)
   double* v;
   double* a;
-  const int8_t* dir;   // the DOF direction of each equation
-  int32_t gdir;        // the excitation's direction, or -1
-  double ag;           // its acceleration at this step's load time
+  CdStep s;
 };
-
-// The effective ground-motion load on equation q (ground_load, explicit_analysis.cpp:48-58):
-// -m(q) a_g when q acts in the excitation's direction.
-__device__ inline double ground_load(const CdArgs& g, int32_t q, double mq) {
-  double r = 0.0;
-  if (g.gdir >= 0 && g.dir[q] == g.gdir) r -= mq * g.ag;
-  return r;
-}
 
 // RECORD: also the recorded velocity and acceleration. They feed no later displacement (the
 // dampers act at the garbage velocity), so the loop writes them only in its last two steps: the
@@ -89,27 +76,17 @@ template <bool RECORD>
 __global__ __launch_bounds__(kThreads) void cd_update_kernel(CdArgs g) {
   const int32_t q = blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= g.n) return;
-  const double uq = g.u[q], umq = g.um[q], mq = g.m[q];
+  const double uq = g.u[q], umq = g.s.um[q];
   double fq = g.f[q];
   if (g.fd) fq += g.fd[q];
   if (g.body) fq -= g.body[q];
-  double cq = 0.0;
-  if (g.am) cq += g.am[q];
-  if (g.dash) {
-    const double dq = g.dash[q];
-    fq += dq * (umq * -g.c2);  // the damper's force at the garbage velocity
-    cq += dq;
-  }
-  const double ag = uq * (-2.0 * g.c3) + umq * g.c3;
-  const double R = -fq - mq * ag + ground_load(g, q, mq);
-  const double A = mq * g.c3 + cq * g.c2;
-  const double U = R / A;
-  g.um[q] = U;
+  const double U = cd_next(g.s, q, fq, uq, umq);
+  g.s.um[q] = U;
   if constexpr (RECORD) {
     double Udot = U * 3.0;
     Udot += uq * -4.0;
     Udot += umq;
-    Udot *= g.c2;
+    Udot *= g.s.c2;
     const double Udotdot = (Udot - g.v[q]) / g.dt;
     g.v[q] = Udot;
     g.a[q] = Udotdot;
@@ -132,17 +109,19 @@ __global__ __launch_bounds__(kThreads) void ed_predict_kernel(int32_t n, double 
 __global__ __launch_bounds__(kThreads) void ed_correct_kernel(CdArgs g) {
   const int32_t q = blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= g.n) return;
-  const double mq = g.m[q];
+  const double mq = g.s.m[q], vh = g.s.um[q];
   double fq = g.f[q];
   if (g.fd) fq += g.fd[q];
   if (g.body) fq -= g.body[q];
-  if (g.dash) fq += g.dash[q] * g.um[q];
-  const double R = -fq + ground_load(g, q, mq);
+  if (g.s.dash) fq += g.s.dash[q] * vh;
+  const double R = -fq + ground_load(g.s.dir, g.s.gdir, g.s.ag, q, mq);
   const double a_new = R / mq;
   const double t = 3.0 * a_new + g.a[q];
-  g.v[q] = g.um[q] + t * (g.dt * 0.125);
+  g.v[q] = vh + t * (g.dt * 0.125);
   g.a[q] = a_new;
 }
+
+}  // namespace
 
 bool elements_damp(const fx_batch* b) {
   for (const DevParam& p : b->host_params)
@@ -150,11 +129,11 @@ bool elements_damp(const fx_batch* b) {
   return false;
 }
 
-}  // namespace
-
 int force64(fx_batch* b, const double* u, const double* v, double* f, double* scratch) {
   if (b->pimy) {  // the return map (and the damping force at v)
     if (int rc = pimy_force64(b, u, v, f, false)) return rc;
+  } else if (box_forms_force(b)) {
+    if (int rc = launch_box_force(b, u, v && elements_damp(b) ? v : nullptr, 1.0, f, 0, nullptr)) return rc;
   } else {
     const int32_t n = b->neq;
     if (int rc = elements_apply64(b, fx_coeffs{1.0, 0.0, 0.0, 0}, u, f)) return rc;
@@ -219,17 +198,17 @@ int cd_run(fx_batch* b, const fx_cd_desc& d, double* u, double* um, double* v, d
   for (int j = 0; j < d.nload; ++j) pl.eq[j] = b->internal ? b->internal_of[d.load_eq[j]] : d.load_eq[j];
   CdArgs g{};
   g.n = n;
-  g.c2 = c2;
-  g.c3 = c3;
   g.dt = d.dt;
   g.f = f;
   g.fd = damp ? fd : nullptr;
   g.body = b->pimy ? nullptr : b->body;  // the return-map force carries the body force
-  g.m = b->lumped_m;
-  g.am = b->lumped_am;
-  g.dash = dash;
-  g.dir = b->eq_dir_dev;
-  g.gdir = d.ground_dir;
+  g.s.c2 = c2;
+  g.s.c3 = c3;
+  g.s.m = b->lumped_m;
+  g.s.am = b->lumped_am;
+  g.s.dash = dash;
+  g.s.dir = b->eq_dir_dev;
+  g.s.gdir = d.ground_dir;
   // node recorders after every step (explicit_analysis.cpp:724-731): u and the recorded v, a
   const bool rec = recorder_active(d.recorder), rec_rates = recorder_reads_rates(d.recorder);
   const int32_t* rmap = nullptr;
@@ -240,7 +219,7 @@ int cd_run(fx_batch* b, const fx_cd_desc& d, double* u, double* um, double* v, d
     for (int32_t k = 0; k < d.nsteps; ++k) {
       hipLaunchKernelGGL(ed_predict_kernel, dim3(blocks_for(n)), dim3(kThreads), 0, ctx->stream, n, d.dt, U, VH, Acc);
       time += d.dt;
-      g.ag = ground_at(k, time);
+      g.s.ag = ground_at(k, time);
       if (damp)
         if (int rc = operator_apply64(b, fx_coeffs{0.0, 1.0, 0.0, 0}, VH, fd)) return rc;
       if (b->pimy) {
@@ -255,7 +234,7 @@ int cd_run(fx_batch* b, const fx_cd_desc& d, double* u, double* um, double* v, d
         hipLaunchKernelGGL(point_load_kernel, dim3(1), dim3(64), 0, ctx->stream, pl, f);
       }
       g.u = U;
-      g.um = VH;
+      g.s.um = VH;
       g.v = V;
       g.a = Acc;
       hipLaunchKernelGGL(ed_correct_kernel, dim3(blocks_for(n)), dim3(kThreads), 0, ctx->stream, g);
@@ -264,9 +243,26 @@ int cd_run(fx_batch* b, const fx_cd_desc& d, double* u, double* um, double* v, d
         if (int rc = recorder_record(d.recorder, time, n, U, V, Acc, rmap)) return rc;
     }
   }
+  // a lattice step without recorded rates in two launches, the update run where each equation's
+  // force is complete (4 M elements, dashpots: 64 B of vectors per equation and step become 48)
+  const bool fused = !ed && box_forms_force(b) && !b->nodal_am && pl.n <= kStepLoads;
   for (int32_t k = 0; !ed && k < d.nsteps; ++k) {
-    g.ag = ground_at(k, time);
+    g.s.ag = ground_at(k, time);
     time += d.dt;
+    if (fused && !rec_rates && k < d.nsteps - 2) {
+      CdStep s = g.s;
+      s.um = Um;
+      s.nload = pl.n;
+      for (int j = 0; j < pl.n; ++j) {
+        s.load_eq[j] = pl.eq[j];
+        s.load[j] = d.load_hist[static_cast<size_t>(k) * pl.n + j];
+      }
+      if (int rc = launch_box_force(b, U, damp ? Um : nullptr, -c2, nullptr, 0, &s)) return rc;
+      std::swap(U, Um);
+      if (rec)
+        if (int rc = recorder_record(d.recorder, time, n, U, V, Acc, rmap)) return rc;
+      continue;
+    }
     if (edamp)
       hipLaunchKernelGGL(scale_kernel, dim3(blocks_for(n)), dim3(kThreads), 0, ctx->stream, n, -c2, Um, ve);
     if (damp)
@@ -283,7 +279,7 @@ int cd_run(fx_batch* b, const fx_cd_desc& d, double* u, double* um, double* v, d
       hipLaunchKernelGGL(point_load_kernel, dim3(1), dim3(64), 0, ctx->stream, pl, f);
     }
     g.u = U;
-    g.um = Um;
+    g.s.um = Um;
     g.v = V;
     g.a = Acc;
     // a record of v or a needs this step's (and so the step before's v): the full update every

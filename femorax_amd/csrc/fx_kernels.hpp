@@ -50,6 +50,17 @@ __host__ __device__ inline void operator_factors(const DevParam& p, const fx_coe
 template <typename T, bool DIAG>
 int launch_box(fx_batch* b, const fx_coeffs& k, const T* x, T* y, int accumulate, const int32_t* done, int ref = 0,
                bool sums = true);
+// The elements' force f = K u + C (vscale v) - F_body of a lattice batch (v null: no damping force)
+// in a tile launch and one that adds the shared and tied sums; ref: reference numbering. step: no
+// f; every equation takes the CentralDifference update where its force is complete (solver
+// numbering). box_forms_force: the batches it takes.
+struct CdStep;
+bool box_forms_force(const fx_batch* b);
+int launch_box_force(fx_batch* b, const double* u, const double* v, double vscale, double* f, int ref,
+                     const CdStep* step);
+// Whether some parameter set has Rayleigh damping (fx_explicit.hip).
+bool elements_damp(const fx_batch* b);
+
 // A CG iteration's lattice product y = A p with the chunk partials of p.y (VectorOps' order), in a
 // tile launch and one that adds the shared nodes' partial sums (solver numbering); and in front
 // of it, where d.z is given, the stop test and the direction p = z + beta p_old, formed as the
