@@ -792,7 +792,7 @@ __global__ __launch_bounds__(kTileThreads) void hex8_box_force_kernel(BoxArgs<do
           double um;
           if constexpr (PAIR) um = vs[d * G::kNodes + ln];
           else um = g.um[e];
-          g.um[e] = cd_next(g, e, val[d], xs[d * G::kNodes + ln], um);
+          cd_store(g, e, val[d], xs[d * G::kNodes + ln], um);
         } else {
           a.y[e] = val[d];
         }
@@ -1113,7 +1113,7 @@ __global__ __launch_bounds__(256) void hex8_step_sums_kernel(const uint32_t* __r
                                                              const double* __restrict__ partial,
                                                              const double* __restrict__ u, CdStep g) {
   const int tied_blocks = (ntied + 3) / 4, b = static_cast<int>(blockIdx.x);
-  auto update = [&](int64_t e, double f) { g.um[e] = cd_next(g, e, f, u[e], g.um[e]); };
+  auto update = [&](int64_t e, double f) { cd_store(g, e, f, u[e], g.um[e]); };
   if (b < tied_blocks) {
     const int n = b * 4 + static_cast<int>(threadIdx.x) / 64;
     if (n < ntied) tied_sum(n, tied_word, tied_start, partial, update);

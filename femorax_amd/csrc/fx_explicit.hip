@@ -69,28 +69,13 @@ struct CdArgs {
   CdStep s;
 };
 
-// RECORD: also the recorded velocity and acceleration. They feed no later displacement (the
-// dampers act at the garbage velocity), so the loop writes them only in its last two steps: the
-// last step's acceleration needs the velocity of the step before.
-template <bool RECORD>
 __global__ __launch_bounds__(kThreads) void cd_update_kernel(CdArgs g) {
   const int32_t q = blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= g.n) return;
-  const double uq = g.u[q], umq = g.s.um[q];
   double fq = g.f[q];
   if (g.fd) fq += g.fd[q];
   if (g.body) fq -= g.body[q];
-  const double U = cd_next(g.s, q, fq, uq, umq);
-  g.s.um[q] = U;
-  if constexpr (RECORD) {
-    double Udot = U * 3.0;
-    Udot += uq * -4.0;
-    Udot += umq;
-    Udot *= g.s.c2;
-    const double Udotdot = (Udot - g.v[q]) / g.dt;
-    g.v[q] = Udot;
-    g.a[q] = Udotdot;
-  }
+  cd_store(g.s, q, fq, g.u[q], g.s.um[q]);
 }
 
 // ExplicitDifference newStep (ed_predict, explicit_analysis.cpp:60-68): vh += dt a; u += dt vh.
@@ -165,14 +150,8 @@ int cd_run(fx_batch* b, const fx_cd_desc& d, double* u, double* um, double* v, d
     Um = W + N;
     V = W + 2 * N;
     Acc = W + 3 * N;
-    if (int rc = to_internal<double>(b, u, U)) return rc;
-    if (int rc = to_internal<double>(b, um, Um)) return rc;
-    if (int rc = to_internal<double>(b, v, V)) return rc;
-    if (int rc = to_internal<double>(b, a, Acc)) return rc;
-    if (d.dash) {
-      dash = W + 6 * N;
-      if (int rc = to_internal<double>(b, d.dash, dash)) return rc;
-    }
+    if (d.dash) dash = W + 6 * N;
+    if (int rc = to_internal_all(b, VectorPairs{{{u, U}, {um, Um}, {v, V}, {a, Acc}, {d.dash, d.dash ? dash : nullptr}}})) return rc;
   }
   double* f = W + 4 * N;
   double* ve = W + 5 * N;
@@ -204,6 +183,7 @@ int cd_run(fx_batch* b, const fx_cd_desc& d, double* u, double* um, double* v, d
   g.body = b->pimy ? nullptr : b->body;  // the return-map force carries the body force
   g.s.c2 = c2;
   g.s.c3 = c3;
+  g.s.dt = d.dt;
   g.s.m = b->lumped_m;
   g.s.am = b->lumped_am;
   g.s.dash = dash;
@@ -243,15 +223,20 @@ int cd_run(fx_batch* b, const fx_cd_desc& d, double* u, double* um, double* v, d
         if (int rc = recorder_record(d.recorder, time, n, U, V, Acc, rmap)) return rc;
     }
   }
-  // a lattice step without recorded rates in two launches, the update run where each equation's
-  // force is complete (4 M elements, dashpots: 64 B of vectors per equation and step become 48)
+  // a lattice step in two launches, the update run where each equation's force is complete (with
+  // dashpots 64 B of vectors per equation and step become 48)
   const bool fused = !ed && box_forms_force(b) && !b->nodal_am && pl.n <= kStepLoads;
   for (int32_t k = 0; !ed && k < d.nsteps; ++k) {
     g.s.ag = ground_at(k, time);
     time += d.dt;
-    if (fused && !rec_rates && k < d.nsteps - 2) {
+    // the recorded v and a only where a record reads them (of this step, so of every step) and in
+    // the last two steps: the last step's acceleration needs the velocity of the step before
+    const bool rates = rec_rates || k >= d.nsteps - 2;
+    g.s.um = Um;
+    g.s.v = rates ? V : nullptr;
+    g.s.a = rates ? Acc : nullptr;
+    if (fused) {
       CdStep s = g.s;
-      s.um = Um;
       s.nload = pl.n;
       for (int j = 0; j < pl.n; ++j) {
         s.load_eq[j] = pl.eq[j];
@@ -279,15 +264,7 @@ int cd_run(fx_batch* b, const fx_cd_desc& d, double* u, double* um, double* v, d
       hipLaunchKernelGGL(point_load_kernel, dim3(1), dim3(64), 0, ctx->stream, pl, f);
     }
     g.u = U;
-    g.s.um = Um;
-    g.v = V;
-    g.a = Acc;
-    // a record of v or a needs this step's (and so the step before's v): the full update every
-    // step, as the reference's cd_solve always does
-    if (rec_rates || k >= d.nsteps - 2)
-      hipLaunchKernelGGL(cd_update_kernel<true>, dim3(blocks_for(n)), dim3(kThreads), 0, ctx->stream, g);
-    else
-      hipLaunchKernelGGL(cd_update_kernel<false>, dim3(blocks_for(n)), dim3(kThreads), 0, ctx->stream, g);
+    hipLaunchKernelGGL(cd_update_kernel, dim3(blocks_for(n)), dim3(kThreads), 0, ctx->stream, g);
     std::swap(U, Um);  // U(n+1) sits in the old U(n-1) buffer
     if (b->pimy) std::swap(b->state_c, b->state_t);  // commit_state: the trial history becomes committed
     if (rec)
@@ -296,10 +273,7 @@ int cd_run(fx_batch* b, const fx_cd_desc& d, double* u, double* um, double* v, d
   FX_HIP(ctx, hipGetLastError());
   // back to the caller's buffers: u = U(n+1), um = U(n)
   if (b->internal) {
-    if (int rc = to_external<double>(b, U, u)) return rc;
-    if (int rc = to_external<double>(b, Um, um)) return rc;
-    if (int rc = to_external<double>(b, V, v)) return rc;
-    if (int rc = to_external<double>(b, Acc, a)) return rc;
+    if (int rc = to_external_all(b, VectorPairs{{{U, u}, {Um, um}, {V, v}, {Acc, a}}})) return rc;
   } else if (!ed && U != u) {  // an odd number of steps: the roles are swapped
     if (int rc = copy64(ctx, n, U, ve)) return rc;
     if (int rc = copy64(ctx, n, Um, U)) return rc;

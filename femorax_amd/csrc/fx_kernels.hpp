@@ -103,6 +103,17 @@ int to_internal(fx_batch* b, const T* ext, T* in);
 template <typename T>
 int to_external(fx_batch* b, const T* in, T* ext);
 
+// Up to five vectors permuted in one pass (the permutation read once); pairs with a null are skipped.
+struct VectorPair {
+  const double* src = nullptr;
+  double* dst = nullptr;
+};
+struct VectorPairs {
+  VectorPair p[5];
+};
+int to_internal_all(fx_batch* b, const VectorPairs& v);
+int to_external_all(fx_batch* b, const VectorPairs& v);
+
 // Solver-side launchers (fx_solver.hip).
 int copy64(fx_ctx* ctx, int64_t n, const double* a, double* b);
 int dot64(fx_ctx* ctx, int64_t n, const double* x, const double* y, double* out);

@@ -733,6 +733,27 @@ int to_external(fx_batch* b, const T* in, T* ext) {
   FX_HIP(b->ctx, hipGetLastError());
   return FX_OK;
 }
+__global__ void perm_all_kernel(int32_t n, const int32_t* __restrict__ perm, VectorPairs v, int inward) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int q = perm[i], from = inward ? q : i, to = inward ? i : q;
+  double x[5];
+#pragma unroll
+  for (int k = 0; k < 5; ++k)
+    if (v.p[k].dst) x[k] = v.p[k].src[from];
+#pragma unroll
+  for (int k = 0; k < 5; ++k)
+    if (v.p[k].dst) v.p[k].dst[to] = x[k];
+}
+int perm_all(fx_batch* b, const VectorPairs& v, int inward) {
+  if (b->neq == 0) return FX_OK;
+  hipLaunchKernelGGL(perm_all_kernel, dim3((b->neq + 255) / 256), dim3(256), 0, b->ctx->stream, b->neq, b->perm, v,
+                     inward);
+  FX_HIP(b->ctx, hipGetLastError());
+  return FX_OK;
+}
+int to_internal_all(fx_batch* b, const VectorPairs& v) { return perm_all(b, v, 1); }
+int to_external_all(fx_batch* b, const VectorPairs& v) { return perm_all(b, v, 0); }
 template int to_internal<double>(fx_batch*, const double*, double*);
 template int to_internal<float>(fx_batch*, const float*, float*);
 template int to_external<double>(fx_batch*, const double*, double*);

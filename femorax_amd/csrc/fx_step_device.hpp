@@ -20,6 +20,9 @@ struct CdStep {
   const int8_t* dir;   // the DOF direction of each equation
   int32_t gdir;        // the excitation's direction, or -1
   double ag;           // its acceleration at this step's load time
+  double* v;           // the recorded velocity and acceleration (in: v of the step before), or null
+  double* a;
+  double dt;
   int32_t nload;       // point loads P(q): f(q) -= P
   int32_t load_eq[kStepLoads];
   double load[kStepLoads];
@@ -51,6 +54,21 @@ __device__ inline double cd_next(const CdStep& g, int64_t q, double fq, double u
   const double R = -fq - mq * ag + ground_load(g.dir, g.gdir, g.ag, q, mq);
   const double A = mq * g.c3 + cq * g.c2;
   return R / A;
+}
+
+// The equation's step stored: U(n+1) over U(n-1), and the recorded rates where they are asked for
+// (they feed no later displacement: the dampers act at the garbage velocity).
+__device__ inline void cd_store(const CdStep& g, int64_t q, double fq, double uq, double umq) {
+  const double U = cd_next(g, q, fq, uq, umq);
+  g.um[q] = U;
+  if (!g.v) return;
+  double Udot = U * 3.0;
+  Udot += uq * -4.0;
+  Udot += umq;
+  Udot *= g.c2;
+  const double Udotdot = (Udot - g.v[q]) / g.dt;
+  g.v[q] = Udot;
+  g.a[q] = Udotdot;
 }
 
 }  // namespace fx
