@@ -217,8 +217,8 @@ __device__ __forceinline__ double gauss_N(int gp, int k) {
 // The internal force: the update at u at every point (STORE also keeps the tangents; REPLAY takes
 // each point's stress and tangent from the compacted pass instead of updating; DAMP adds the
 // Rayleigh damping force at the velocities a.v, std_brick.hpp:409-464). One thread per point.
-// A point leaves in LDS its node forces (and damping terms) and its dvol, 25 (49) values: the
-// element's first lane forms the body terms itself. The registers are held to 256, two waves per
+// A point leaves in LDS its node forces (and damping terms) and its dvol, 25 (49) values; the
+// element's eight lanes then sum a node each and form its body terms. The registers are held to 256, two waves per
 // SIMD (the return map's history loads then overlap another wave's arithmetic): the element's
 // geometry is formed again after the return map instead of held through it, the tangent kept as
 // its parts (coefficient, deviator, G, K) and the damping's D, D_0 and D_c formed entry by entry.
@@ -314,27 +314,25 @@ __global__ __launch_bounds__(kPointsPerBlock, 2) void pimy_batch_kernel(PimyBatc
     }
   }
   __syncthreads();
-  if (!live || gp != 0) return;
-  double out[24], fdamp[24];
-  for (int k = 0; k < 24; ++k) out[k] = fdamp[k] = 0.0;
+  if (!live) return;
+  // lane gp of the element sums node gp over the points, in point order
   const PimyParams& p = a.params[a.param[e]];
+  const int j = gp;
+  double out[3] = {0.0, 0.0, 0.0}, fdamp[3] = {0.0, 0.0, 0.0};
   for (int g = 0; g < 8; ++g) {
-    const double* c = part[t + g];
-    const double dvol = c[8 * W];
-    for (int j = 0; j < 8; ++j) {
-      const double Nj = gauss_N(g, j);
-      for (int q = 0; q < 3; ++q) {
-        out[3 * j + q] += c[W * j + q];
-        out[3 * j + q] -= dvol * p.b[q] * Nj;  // body
-        if constexpr (DAMP) fdamp[3 * j + q] += c[W * j + 3 + q];
-      }
+    const double* c = part[t - gp + g];
+    const double dvol = c[8 * W], Nj = gauss_N(g, j);
+    for (int q = 0; q < 3; ++q) {
+      out[q] += c[W * j + q];
+      out[q] -= dvol * p.b[q] * Nj;  // body
+      if constexpr (DAMP) fdamp[q] += c[W * j + 3 + q];
     }
   }
   if constexpr (DAMP)  // fe = resid + fdamp where the element damps
     if (stiffness_damping(p) || p.alphaM != 0.0)
-      for (int k = 0; k < 24; ++k) out[k] += fdamp[k];
+      for (int q = 0; q < 3; ++q) out[q] += fdamp[q];
   const size_t P = static_cast<size_t>(a.padded);
-  for (int k = 0; k < 24; ++k) a.slots[k * P + e] = out[k];
+  for (int q = 0; q < 3; ++q) a.slots[(3 * j + q) * P + e] = out[q];
 }
 
 // diag(B^T D_eff B dvol + cM M) at one point, tied DOFs of the element merged onto the first
@@ -460,30 +458,46 @@ __global__ __launch_bounds__(128) void pimy_operator_kernel(PimyBatchArgs a) {
 
 // The same for small batches, one thread per point (8 lanes per element), so that a batch of a
 // few hundred elements still runs thousands of threads: each point leaves its node terms in
-// LDS and the element's first lane adds them in point order (the same sums as above).
+// LDS and the element's lanes add them in point order, a node each (the same sums as above). The
+// stored tangent is loaded ahead of the chain node -> equation -> x, and D_eff's entries are
+// formed where they are used, as above: 1,024 elements 20.5 -> 9 us, half of it the sums one lane
+// of eight used to walk.
 template <bool DIAG>
 __global__ __launch_bounds__(kPointsPerBlock) void pimy_point_operator_kernel(PimyBatchArgs a) {
-  __shared__ double part[kPointsPerBlock][48];  // per point: 8 nodes x (3 stiffness, 3 mass) or 24 x 2
+  // per point: 8 nodes x (3 stiffness, 3 mass) or the 24 diagonal entries; odd stride: the lanes of
+  // a wave write different banks
+  constexpr int W = DIAG ? 25 : 49;
+  __shared__ double part[kPointsPerBlock][W];
   const int t = threadIdx.x;
   const int e = blockIdx.x * kElemsPerBlock + t / 8, gp = t % 8;
   const bool live = e < a.count;
+  double cK = 0.0, c0 = 0.0, cc = 0.0, cM = 0.0;
   if (live) {
+    double tv[21];
+    if constexpr (!DIAG)
+      for (int w = 0; w < 21; ++w) tv[w] = a.tangent[tangent_at(a, e, gp, w)];
     double X[8], Y[8], Z[8];
     int eq[24];
     element_geometry(a, e, X, Y, Z, eq);
     const PimyParams& p = a.params[a.param[e]];
-    Shape<double> s;
-    gauss_shape(X, Y, Z, gp, s);
+    operator_factors(p, a.k, cK, c0, cc, cM);
     double* mine = part[t];
-    double D[36], cM;
-    effective_D(a, p, e, gp, D, cM);
     if constexpr (!DIAG) {
-      double v[24], eps[6], sig[6];
+      double v[24], eps[6], sig[6], Dc[36];
       for (int k = 0; k < 24; ++k) v[k] = operator_input(a, eq, k);
+      Shape<double> s;
+      gauss_shape(X, Y, Z, gp, s);
       point_strain(s, v, eps);
+      if (cc != 0.0) pimy_committed_tangent(p, a.C + static_cast<int64_t>(e) * 8 + gp, a.npts, Dc);
       for (int r = 0; r < 6; ++r) {
         double sum = 0.0;
-        for (int c = 0; c < 6; ++c) sum += D[6 * r + c] * eps[c];
+        for (int c = 0; c < 6; ++c) {
+          const int lo = r < c ? r : c, hi = r < c ? c : r;
+          double d = cK * tv[lo * 6 - lo * (lo - 1) / 2 + (hi - lo)];
+          if (c0 != 0.0) d += c0 * initial_entry(p, r, c);
+          if (cc != 0.0) d += cc * Dc[6 * r + c];
+          sum += d * eps[c];
+        }
         sig[r] = sum;
       }
       double g[3] = {0, 0, 0};
@@ -500,35 +514,30 @@ __global__ __launch_bounds__(kPointsPerBlock) void pimy_point_operator_kernel(Pi
         }
       }
     } else {
-      double de[24];
-      element_point_diagonal(s, p, D, cM, eq, de);
-      for (int k = 0; k < 24; ++k) {
-        mine[2 * k] = de[k];
-        mine[2 * k + 1] = 0.0;
-      }
+      Shape<double> s;
+      gauss_shape(X, Y, Z, gp, s);
+      double D[36], cMd, de[24];
+      effective_D(a, p, e, gp, D, cMd);
+      element_point_diagonal(s, p, D, cMd, eq, de);
+      for (int k = 0; k < 24; ++k) mine[k] = de[k];
     }
   }
   __syncthreads();
-  if (!live || gp != 0) return;
-  const PimyParams& p = a.params[a.param[e]];
-  double cK, c0, cc, cM;
-  operator_factors(p, a.k, cK, c0, cc, cM);
-  double out[24];
-  for (int k = 0; k < 24; ++k) out[k] = 0.0;
+  if (!live) return;
+  double out[3] = {0.0, 0.0, 0.0};
   for (int g = 0; g < 8; ++g) {
-    const double* c = part[t + g];
-    if constexpr (!DIAG) {
-      for (int j = 0; j < 8; ++j)
-        for (int q = 0; q < 3; ++q) {
-          out[3 * j + q] += c[6 * j + q];
-          if (cM != 0.0) out[3 * j + q] += c[6 * j + 3 + q];
-        }
-    } else {
-      for (int k = 0; k < 24; ++k) out[k] += c[2 * k];
+    const double* c = part[t - gp + g];
+    for (int q = 0; q < 3; ++q) {
+      if constexpr (!DIAG) {
+        out[q] += c[6 * gp + q];
+        if (cM != 0.0) out[q] += c[6 * gp + 3 + q];
+      } else {
+        out[q] += c[3 * gp + q];
+      }
     }
   }
   const size_t P = static_cast<size_t>(a.padded);
-  for (int k = 0; k < 24; ++k) a.slots[k * P + e] = out[k];
+  for (int q = 0; q < 3; ++q) a.slots[(3 * gp + q) * P + e] = out[q];
 }
 
 // The compacted return map (compacted_kernels.hpp:85-202). Predict: one thread per Gauss point,
@@ -591,41 +600,58 @@ __global__ void pimy_clear_count_kernel(int32_t* count) {
   if (threadIdx.x == 0) count[0] = 0;
 }
 
-// y[q] = the sum of equation q's element slots, in (element, DOF) order (assembly.cpp:64-95).
-// An equation with more than kLongGather slots (a tied level of a soil column) is left to
-// long_gather_kernel.
+// y[q] = the sum of equation q's element slots, in (element, DOF) order (assembly.cpp:64-95): one
+// thread per equation, eight list entries and then eight slots in flight (a node of a regular mesh
+// has eight). An equation with more than kLongGather slots (a tied level of a soil column) takes
+// a wave of the workgroups after the first short_blocks: lane l sums slots l, l + 64, ... in
+// order, then a fixed butterfly over the lanes. One launch: 2,400 equations 11.5 + 4.5 -> 5 us.
 constexpr int kLongGather = 64;
 
 template <typename T>
-__global__ void slot_gather_kernel(int32_t neq, const int32_t* __restrict__ start, const int32_t* __restrict__ list,
-                                   const T* __restrict__ slots, T* __restrict__ y, const int32_t* done,
-                                   int accumulate) {
-  if (done && *done) return;
-  const int32_t q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= neq) return;
+__global__ __launch_bounds__(256) void slot_gather_kernel(int32_t neq, const int32_t* __restrict__ start,
+                                                          const int32_t* __restrict__ list, int32_t nlong,
+                                                          const int32_t* __restrict__ long_eqs,
+                                                          const T* __restrict__ slots, T* __restrict__ y,
+                                                          const int32_t* done, int accumulate) {
+  const int stopped = done ? *done : 0;
+  const int short_blocks = (neq + 255) / 256, b = static_cast<int>(blockIdx.x);
+  if (b >= short_blocks) {
+    const int u = (b - short_blocks) * 4 + static_cast<int>(threadIdx.x) / 64, lane = threadIdx.x % 64;
+    if (u >= nlong || stopped) return;  // the whole wave
+    const int32_t q = long_eqs[u], j1 = start[q + 1];
+    T s = T(0);
+    for (int32_t j0 = start[q] + lane; j0 < j1; j0 += 4 * 64) {
+      int32_t at[4];
+      T v[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) at[k] = list[j0 + 64 * k < j1 ? j0 + 64 * k : j0];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[k] = slots[at[k]];
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (j0 + 64 * k < j1) s += v[k];
+    }
+    for (int off = 32; off >= 1; off >>= 1) s += __shfl_xor(s, off, 64);
+    if (lane == 0) y[q] = accumulate ? y[q] + s : s;
+    return;
+  }
+  const int32_t q = b * 256 + static_cast<int32_t>(threadIdx.x);
+  if (q >= neq || stopped) return;
   const int32_t j0 = start[q], j1 = start[q + 1];
   if (j1 - j0 > kLongGather) return;
   T s = T(0);
-  for (int32_t j = j0; j < j1; ++j) s += slots[list[j]];
+  for (int32_t j = j0; j < j1; j += 8) {
+    int32_t at[8];
+    T v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) at[k] = list[j + k < j1 ? j + k : j];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = slots[at[k]];
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      if (j + k < j1) s += v[k];
+  }
   y[q] = accumulate ? y[q] + s : s;
-}
-
-// The long equations: one wave each, lane l summing slots l, l + 64, ... in order, then a fixed
-// butterfly over the lanes.
-template <typename T>
-__global__ __launch_bounds__(256) void long_gather_kernel(int32_t nlong, const int32_t* __restrict__ eqs,
-                                                          const int32_t* __restrict__ start,
-                                                          const int32_t* __restrict__ list,
-                                                          const T* __restrict__ slots, T* __restrict__ y,
-                                                          const int32_t* done, int accumulate) {
-  const int u = static_cast<int>(blockIdx.x) * 4 + static_cast<int>(threadIdx.x) / 64, lane = threadIdx.x % 64;
-  if (u >= nlong) return;  // the whole wave
-  if (done && *done) return;
-  const int32_t q = eqs[u];
-  T s = T(0);
-  for (int32_t j = start[q] + lane; j < start[q + 1]; j += 64) s += slots[list[j]];
-  for (int off = 32; off >= 1; off >>= 1) s += __shfl_xor(s, off, 64);
-  if (lane == 0) y[q] = accumulate ? y[q] + s : s;
 }
 
 __global__ void pimy_batch_init_kernel(int64_t npts, const PimyParams* __restrict__ params,
@@ -671,15 +697,13 @@ PimyBatchArgs batch_args(fx_batch* b, const double* x, const fx_coeffs& k, const
   return a;
 }
 
-// y[q] = the sum of equation q's element slots (slot_gather_kernel, long_gather_kernel)
+// y[q] = the sum of equation q's element slots
 template <typename T>
 int gather(fx_batch* b, const T* slots, T* y, const int32_t* done, int accumulate = 0) {
   if (b->neq > 0)
-    hipLaunchKernelGGL(slot_gather_kernel<T>, dim3((b->neq + 255) / 256), dim3(256), 0, b->ctx->stream, b->neq,
-                       b->gather_start, b->gather_list, slots, y, done, accumulate);
-  if (b->nlong > 0)
-    hipLaunchKernelGGL(long_gather_kernel<T>, dim3((b->nlong + 3) / 4), dim3(256), 0, b->ctx->stream, b->nlong,
-                       b->long_eqs, b->gather_start, b->gather_list, slots, y, done, accumulate);
+    hipLaunchKernelGGL(slot_gather_kernel<T>, dim3((b->neq + 255) / 256 + (b->nlong + 3) / 4), dim3(256), 0,
+                       b->ctx->stream, b->neq, b->gather_start, b->gather_list, b->nlong, b->long_eqs, slots, y, done,
+                       accumulate);
   FX_HIP(b->ctx, hipGetLastError());
   return FX_OK;
 }
