@@ -657,23 +657,77 @@ __global__ __launch_bounds__(64 * WAVES) void column_solve_kernel(PoolArgs a) {
   }
 }
 
-__global__ void column_init_kernel(int64_t cap, int64_t e0, int32_t n, const PimyParams* __restrict__ params,
-                                   const int32_t* __restrict__ elem_param, double* state, int32_t* touched) {
-  const int64_t k = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (k >= n) return;
-  const int64_t i = e0 + k;
-  touched[i] = 0;  // every centre at its initial value in both buffers
-  const PimyParams& p = params[elem_param[i]];
-  const size_t NS = static_cast<size_t>(kPimyNState) * static_cast<size_t>(cap);
-  for (double* S : {state, state + NS}) {
-    for (int f = 0; f < kPimyNState; ++f) S[f * cap + i] = 0.0;
-    S[kPG * cap + i] = p.G;
-    S[kPK * cap + i] = p.K;
-    for (int s = 1; s <= kPimyNS; ++s) {
-      S[(kPSizes + s - 1) * cap + i] = p.size[s];
-      S[(kPModuli + s - 1) * cap + i] = p.modulus[s];
-    }
+// A column's admission, from the pool's pinned staging block (read by the device in place): its
+// parameter sets, the elements' sets and the ground record to their arenas. A column came in
+// through thirteen copies and fills of its own, 100 us of host calls; two launches take 15 us (256
+// short records through a pool of 64 columns: 59 -> 22 ms, with the fetches and removals below).
+struct Staged {
+  const uint64_t* src;  // pinned, then each piece's destination and length in 4-byte words
+  uint32_t* dst[3];
+  int64_t words[3];
+};
+__global__ void column_stage_kernel(Staged st) {
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
+  const uint32_t* src = reinterpret_cast<const uint32_t*>(st.src);
+  for (int k = 0; k < 3; ++k) {
+    for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < st.words[k]; i += stride)
+      st.dst[k][i] = src[i];
+    src += (st.words[k] + 1) / 2 * 2;
   }
+}
+
+// The column's elements at rest (every state zero, the histories initial in both buffers), its
+// slots taken, and its record written. A column has a workgroup or two of elements, so the history
+// fields are spread over blockIdx.y (kInitFields each): one thread that walked all 380 of an
+// element took 23 us (28 -> 22 ms for 256 records).
+constexpr int kInitFields = 10;
+__global__ __launch_bounds__(256) void column_init_kernel(PoolArgs a, ColumnDev cd, int32_t c, int32_t* elem_col) {
+  const int64_t k = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  const bool first = blockIdx.y == 0;
+  if (k == 0 && first) a.cols[c] = cd;
+  if (k >= cd.nelem) return;
+  const int64_t i = cd.e0 + k, cap = a.cap;
+  if (first) {
+    elem_col[i] = c;
+    a.touched[i] = 0;  // every centre at its initial value in both buffers
+    for (double* q : {a.u, a.v, a.a, a.ut, a.vt, a.at, a.du, a.du0})
+      for (int d = 0; d < 3; ++d) q[3 * i + d] = 0.0;
+  }
+  const PimyParams& p = a.params[a.elem_param[i]];
+  const size_t NS = static_cast<size_t>(kPimyNState) * static_cast<size_t>(cap);
+  const int f0 = static_cast<int>(blockIdx.y) * kInitFields;
+  for (int f = f0; f < f0 + kInitFields && f < kPimyNState; ++f) {
+    double x = 0.0;
+    if (f == kPG) x = p.G;
+    else if (f == kPK) x = p.K;
+    else if (f >= kPSizes && f < kPSizes + kPimyNS) x = p.size[f - kPSizes + 1];
+    else if (f >= kPModuli && f < kPModuli + kPimyNS) x = p.modulus[f - kPModuli + 1];
+    a.state[f * cap + i] = x;
+    a.state[NS + f * cap + i] = x;
+  }
+}
+
+// u, v, a of a column (n values each) and its history to pinned memory.
+__global__ void column_fetch_kernel(const double* __restrict__ u, const double* __restrict__ v,
+                                    const double* __restrict__ a, int64_t n, const double* __restrict__ hist, int64_t nh,
+                                    double* out) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i < n) {
+    out[i] = u[i];
+    out[n + i] = v[i];
+    out[2 * n + i] = a[i];
+  }
+  if (i < nh) out[3 * n + i] = hist[i];
+}
+
+// A removed column: idle, its slots nobody's.
+__global__ void column_remove_kernel(ColumnDev* col, int32_t* elem_col, int64_t e0, int32_t n) {
+  const int32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k == 0) {
+    *col = ColumnDev{};
+    col->status = kIdle;
+  }
+  if (k < n) elem_col[e0 + k] = -1;
 }
 
 __global__ void column_count_kernel(const ColumnDev* cols, int32_t n, int32_t* out, int8_t* status) {
@@ -751,6 +805,10 @@ struct fx_column_pool {
   std::vector<fx::HostColumn> host;
   int32_t* count = nullptr;       // device: running columns, then the status byte of each column
   int32_t* count_host = nullptr;  // pinned copy of the same
+  // pinned staging of admissions (queued kernels read them) and of fetched results; reused from its
+  // start once the stream has caught up
+  char* stage = nullptr;
+  size_t stage_at = 0;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   int wpe = 3;                    // the return-map kernels' register budget (waves per SIMD)
@@ -767,6 +825,22 @@ int fail(fx_ctx* ctx, int code, const std::string& msg) {
   if (ctx) ctx->error = msg;
   else set_thread_error(msg);
   return code;
+}
+
+constexpr size_t kStageBytes = size_t(1) << 20;  // over a hundred admissions of short records
+
+// `bytes` (a multiple of 8) of the staging block, the stream waited for when it is used up; null for
+// more than it holds.
+int stage_take(fx_column_pool* p, size_t bytes, char*& out) {
+  out = nullptr;
+  if (bytes > kStageBytes) return FX_OK;
+  if (p->stage_at + bytes > kStageBytes) {
+    FX_HIP(p->ctx, hipStreamSynchronize(p->ctx->stream));
+    p->stage_at = 0;
+  }
+  out = p->stage + p->stage_at;
+  p->stage_at += bytes;
+  return FX_OK;
 }
 
 template <typename T>
@@ -925,6 +999,7 @@ void fx_column_pool_destroy(fx_column_pool* p) {
   if (p->fork) (void)hipEventDestroy(p->fork);
   for (void* q : p->allocs) (void)hipFree(q);
   if (p->count_host) (void)hipHostFree(p->count_host);
+  if (p->stage) (void)hipHostFree(p->stage);
   ctx->used -= std::min<uint64_t>(ctx->used, p->bytes);
   delete p;
 }
@@ -1005,6 +1080,11 @@ int fx_column_pool_create(fx_ctx* ctx, const fx_column_pool_desc* d, fx_column_p
   }
   if (hipHostMalloc(reinterpret_cast<void**>(&p->count_host),
                     sizeof(int32_t) * (1 + (static_cast<size_t>(d->max_columns) + 3) / 4)) != hipSuccess) {
+    fx_column_pool_destroy(p);
+    return fail(ctx, FX_EDEVICE, "hipHostMalloc failed");
+  }
+  if (hipHostMalloc(reinterpret_cast<void**>(&p->stage), kStageBytes, hipHostMallocMapped | hipHostMallocCoherent) !=
+      hipSuccess) {
     fx_column_pool_destroy(p);
     return fail(ctx, FX_EDEVICE, "hipHostMalloc failed");
   }
@@ -1096,7 +1176,7 @@ int fx_column_add(fx_column_pool* p, const fx_column_desc* d, int32_t* id) {
   hc.nsteps = d->nsteps;
   PoolArgs& a = p->args;
   hipStream_t st = ctx->stream;
-  std::vector<int32_t> ecol(N, c), epar(N);
+  std::vector<int32_t> epar(N);
   for (int32_t k = 0; k < N; ++k) epar[k] = static_cast<int32_t>(m0) + d->mat_of[k];
   ColumnDev cd{};
   cd.status = kRunning;
@@ -1110,22 +1190,34 @@ int fx_column_add(fx_column_pool* p, const fx_column_desc* d, int32_t* id) {
   cd.hx = d->hx;
   cd.hy = d->hy;
   cd.hz = d->hz;
-  const size_t n3 = 3 * static_cast<size_t>(N) * sizeof(double);
-  FX_HIP(ctx, hipMemcpyAsync(const_cast<PimyParams*>(a.params) + m0, pp.data(), sizeof(PimyParams) * d->nmat,
-                             hipMemcpyHostToDevice, st));
-  FX_HIP(ctx, hipMemcpyAsync(const_cast<int32_t*>(a.elem_param) + e0, epar.data(), sizeof(int32_t) * N,
-                             hipMemcpyHostToDevice, st));
-  FX_HIP(ctx, hipMemcpyAsync(const_cast<double*>(a.record) + r0, d->ground_accel, sizeof(double) * d->nsteps,
-                             hipMemcpyHostToDevice, st));
-  for (double* q : {a.u, a.v, a.a, a.ut, a.vt, a.at, a.du, a.du0}) FX_HIP(ctx, hipMemsetAsync(q + 3 * e0, 0, n3, st));
-  hipLaunchKernelGGL(column_init_kernel, dim3(static_cast<unsigned>((N + 255) / 256)), dim3(256), 0, st, a.cap, e0, N,
-                     a.params, a.elem_param, a.state, a.touched);
+  const void* src[3] = {pp.data(), epar.data(), d->ground_accel};
+  const size_t len[3] = {sizeof(PimyParams) * static_cast<size_t>(d->nmat), sizeof(int32_t) * static_cast<size_t>(N),
+                         sizeof(double) * static_cast<size_t>(d->nsteps)};
+  void* dst[3] = {const_cast<PimyParams*>(a.params) + m0, const_cast<int32_t*>(a.elem_param) + e0,
+                  const_cast<double*>(a.record) + r0};
+  size_t total = 0;
+  for (size_t n : len) total += (n + 7) / 8 * 8;
+  char* block = nullptr;
+  if (int rc = stage_take(p, total, block)) return rc;
+  if (block) {
+    Staged sg{};
+    sg.src = reinterpret_cast<const uint64_t*>(block);
+    for (int k = 0; k < 3; ++k) {
+      std::memcpy(block, src[k], len[k]);
+      block += (len[k] + 7) / 8 * 8;
+      sg.dst[k] = static_cast<uint32_t*>(dst[k]);
+      sg.words[k] = static_cast<int64_t>(len[k] / 4);
+    }
+    const unsigned blocks = static_cast<unsigned>(std::min<size_t>(64, (total / 4 + 255) / 256));
+    hipLaunchKernelGGL(column_stage_kernel, dim3(blocks), dim3(256), 0, st, sg);
+  } else {  // more than the staging block: plain copies
+    for (int k = 0; k < 3; ++k) FX_HIP(ctx, hipMemcpyAsync(dst[k], src[k], len[k], hipMemcpyHostToDevice, st));
+  }
+  const dim3 init_grid((N + 255) / 256, (kPimyNState + kInitFields - 1) / kInitFields);
+  hipLaunchKernelGGL(column_init_kernel, init_grid, dim3(256), 0, st, a, cd, c,
+                     const_cast<int32_t*>(a.elem_col));
   FX_HIP(ctx, hipGetLastError());
-  // the column joins the running set last: slot ownership, then its status
-  FX_HIP(ctx, hipMemcpyAsync(const_cast<int32_t*>(a.elem_col) + e0, ecol.data(), sizeof(int32_t) * N,
-                             hipMemcpyHostToDevice, st));
-  FX_HIP(ctx, hipMemcpyAsync(a.cols + c, &cd, sizeof cd, hipMemcpyHostToDevice, st));
-  FX_HIP(ctx, hipStreamSynchronize(st));
+  if (total > kStageBytes) FX_HIP(ctx, hipStreamSynchronize(st));  // the caller's record has been read
   *id = c;
   return FX_OK;
 }
@@ -1201,14 +1293,29 @@ int fx_column_fetch(fx_column_pool* p, int32_t id, double* u, double* v, double*
   if (history && hc.hist < 0) return fail(p->ctx, FX_EINVAL, "fx_column_fetch: the column keeps no history");
   fx_ctx* ctx = p->ctx;
   hipStream_t st = ctx->stream;
-  const size_t n3 = 3 * static_cast<size_t>(hc.nelem) * sizeof(double);
-  const double* src[3] = {p->args.u, p->args.v, p->args.a};
+  const size_t n3 = 3 * static_cast<size_t>(hc.nelem), nh = history ? 9 * static_cast<size_t>(hc.nsteps) : 0;
+  const double* src[3] = {p->args.u + 3 * hc.e0, p->args.v + 3 * hc.e0, p->args.a + 3 * hc.e0};
   double* dst[3] = {u, v, a};
+  char* block = nullptr;
+  if (int rc = stage_take(p, sizeof(double) * (3 * n3 + nh), block)) return rc;
+  if (block) {  // one launch and one wait for what were four copies
+    double* out = reinterpret_cast<double*>(block);
+    hipLaunchKernelGGL(column_fetch_kernel, dim3(static_cast<unsigned>((std::max(n3, nh) + 255) / 256)), dim3(256), 0, st,
+                       src[0], src[1], src[2], static_cast<int64_t>(n3),
+                       history ? p->args.record + hc.hist : static_cast<const double*>(nullptr), static_cast<int64_t>(nh),
+                       out);
+    FX_HIP(ctx, hipGetLastError());
+    FX_HIP(ctx, hipStreamSynchronize(st));
+    p->stage_at = 0;  // the stream has caught up
+    for (int k = 0; k < 3; ++k)
+      if (dst[k]) std::memcpy(dst[k], out + k * n3, sizeof(double) * n3);
+    if (history) std::memcpy(history, out + 3 * n3, sizeof(double) * nh);
+    return FX_OK;
+  }
   for (int k = 0; k < 3; ++k)
-    if (dst[k]) FX_HIP(ctx, hipMemcpyAsync(dst[k], src[k] + 3 * hc.e0, n3, hipMemcpyDeviceToHost, st));
+    if (dst[k]) FX_HIP(ctx, hipMemcpyAsync(dst[k], src[k], sizeof(double) * n3, hipMemcpyDeviceToHost, st));
   if (history)
-    FX_HIP(ctx, hipMemcpyAsync(history, p->args.record + hc.hist, sizeof(double) * 9 * hc.nsteps,
-                               hipMemcpyDeviceToHost, st));
+    FX_HIP(ctx, hipMemcpyAsync(history, p->args.record + hc.hist, sizeof(double) * nh, hipMemcpyDeviceToHost, st));
   FX_HIP(ctx, hipStreamSynchronize(st));
   return FX_OK;
 }
@@ -1238,13 +1345,9 @@ int fx_column_remove(fx_column_pool* p, int32_t id) {
   fx_ctx* ctx = p->ctx;
   hipStream_t st = ctx->stream;
   HostColumn& hc = p->host[id];
-  ColumnDev cd{};
-  cd.status = kIdle;
-  std::vector<int32_t> none(hc.nelem, -1);
-  FX_HIP(ctx, hipMemcpyAsync(p->args.cols + id, &cd, sizeof cd, hipMemcpyHostToDevice, st));
-  FX_HIP(ctx, hipMemcpyAsync(const_cast<int32_t*>(p->args.elem_col) + hc.e0, none.data(), sizeof(int32_t) * hc.nelem,
-                             hipMemcpyHostToDevice, st));
-  FX_HIP(ctx, hipStreamSynchronize(st));
+  hipLaunchKernelGGL(column_remove_kernel, dim3(static_cast<unsigned>((hc.nelem + 255) / 256)), dim3(256), 0, st,
+                     p->args.cols + id, const_cast<int32_t*>(p->args.elem_col), hc.e0, hc.nelem);
+  FX_HIP(ctx, hipGetLastError());
   p->elems.give(hc.e0, hc.nelem);
   p->mats.give(hc.m0, hc.nmat);
   p->recs.give(hc.rec, hc.rec_len);
