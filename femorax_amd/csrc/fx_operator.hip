@@ -253,32 +253,49 @@ __device__ __forceinline__ T load_coord(const double* c64, const float* c32, siz
 // gather would fetch them for each of up to eight elements); an element then reads its corners
 // there. Larger blocks gather per element (GATHER: a second launch over the same grid, made
 // only when the batch has such blocks; each launch skips the other's blocks). The values are the
-// same either way, so are the bits. Registers are held to two waves per SIMD for FP64 (the
-// staged FP64 element work fits in 228), four for FP32.
+// same either way, so are the bits. Registers are held to two waves per SIMD for FP64 (the staged
+// element work fits in 226), four for FP32.
+// Bounds, 72^3 distorted elements in FP64: 2,900 vector instructions an element (28 us of issue
+// over the chip) against 85 MB of memory (17 us); the workgroups of a CU run in step, so loads that
+// wait on each other add to it. What a block reads is therefore asked for at its start (its
+// corners, its node lists, its elements' parameters; two nodes a thread in flight), the lists wait
+// in LDS, and the output's words are asked for before the barrier that they stand behind: 60 ->
+// 55 us. Three waves a SIMD (the coordinates' modal coefficients in LDS, 168 registers, 8 spills)
+// took 58 us.
 template <typename T, bool DIAG, bool SSP, bool GATHER = false>
-__global__ __launch_bounds__(kBlockElems, sizeof(T) == 8 ? 2 : 4) void hex8_block_kernel(KernelArgs<T> a,
-                                                                                         T* __restrict__ partial) {
-  extern __shared__ unsigned char smem_raw[];
+__global__ __launch_bounds__(kBlockElems, sizeof(T) == 8 ? 2 : 4) void hex8_block_kernel(
+    KernelArgs<T> a, T* __restrict__ partial) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
   T* slots = reinterpret_cast<T*>(smem_raw);  // [24][kBlockElems]
-  if (a.done && *a.done) return;
+  uint16_t* list = reinterpret_cast<uint16_t*>(slots + 24 * kBlockElems);  // [8 * kBlockElems]
   const int b = blockIdx.x;
   const int t = threadIdx.x;
   const int ln0 = a.ln_start[b], ln1 = a.ln_start[b + 1];
+  if (a.done && *a.done) return;
   if ((ln1 - ln0 > kStageNodes) != GATHER) return;  // the other launch's block (uniform)
   const int e = a.elems[static_cast<size_t>(b) * kBlockElems + t];
+  const uint4 entries = reinterpret_cast<const uint4*>(a.slot_list + static_cast<size_t>(b) * 8 * kBlockElems)[t];
+  const uint16_t* lc = a.lcorner + static_cast<size_t>(b) * 8 * kBlockElems + t;
+  int li[8];
+  if constexpr (!GATHER)
+#pragma unroll
+    for (int k = 0; k < 8; ++k) li[k] = lc[k * kBlockElems];
   const size_t tot = static_cast<size_t>(a.ln_total);
   T X[8], Y[8], Z[8], V[24], out[24];
   int eqe[24];
-  // the element's operator values (or diagonal) from its corners; vl(i) reloads V[i]
-  auto element = [&](auto vl) {
+  double fD = 0.0, cM;
+  ElemCoef<T> c;
+  auto coefficients = [&]() {
     const DevParam& p = a.params[a.param[e]];
-    double fD, cM;
     operator_factors(p, a.k, fD, cM);
-    ElemCoef<T> c;
     c.lam = static_cast<T>(fD * p.lam);
     c.mu = static_cast<T>(fD * p.mu);
     c.rhoM = static_cast<T>(cM * p.rho);
     c.consistent = p.mass_type == 0;
+  };
+  if (!GATHER && e >= 0) coefficients();
+  // the element's operator values (or diagonal) from its corners; vl(i) reloads V[i]
+  auto element = [&](auto vl) {
     if constexpr (SSP) {
       // the constants in block order: coalesced loads
       const size_t at = static_cast<size_t>(b) * kBlockElems + t;
@@ -290,32 +307,48 @@ __global__ __launch_bounds__(kBlockElems, sizeof(T) == 8 ? 2 : 4) void hex8_bloc
     }
   };
   if constexpr (!GATHER) {
-    // staging: x, y, z, then the three x values (or, for the diagonal, equations) per node
+    // staging: x, y, z, then the three x values (or, for the diagonal, equations) per node, two
+    // nodes a thread at a time with their loads in flight together
     T* sxyz = slots;
     T* sv = slots + 3 * kStageNodes;
     int* seq = reinterpret_cast<int*>(sv);
-    for (int i = t; i < ln1 - ln0; i += kBlockElems) {
-      const size_t ln = static_cast<size_t>(ln0) + i;
-      if constexpr (!SSP)
+    for (int i0 = t; i0 < ln1 - ln0; i0 += 2 * kBlockElems) {
+      int q[2][3];
+      T xyz[2][3], v[2][3];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const size_t ln = static_cast<size_t>(ln0) + min(i0 + h * kBlockElems, ln1 - ln0 - 1);
+#pragma unroll
+        for (int d = 0; d < 3; ++d) q[h][d] = a.ln_eq[d * tot + ln];
+        if constexpr (!SSP)
+#pragma unroll
+          for (int d = 0; d < 3; ++d) {
+            if constexpr (sizeof(T) == 8) xyz[h][d] = a.ln_xyz64[d * tot + ln];
+            else xyz[h][d] = a.ln_xyz32[d * tot + ln];
+          }
+      }
+      if constexpr (!DIAG)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int d = 0; d < 3; ++d) v[h][d] = q[h][d] >= 0 ? a.x[q[h][d]] : T(0);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int i = i0 + h * kBlockElems;
+        if (i >= ln1 - ln0) break;
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
-          if constexpr (sizeof(T) == 8) sxyz[d * kStageNodes + i] = a.ln_xyz64[d * tot + ln];
-          else sxyz[d * kStageNodes + i] = a.ln_xyz32[d * tot + ln];
+          if constexpr (!SSP) sxyz[d * kStageNodes + i] = xyz[h][d];
+          if constexpr (DIAG) seq[d * kStageNodes + i] = q[h][d];
+          else sv[d * kStageNodes + i] = v[h][d];
         }
-#pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        const int q = a.ln_eq[d * tot + ln];
-        if constexpr (DIAG) seq[d * kStageNodes + i] = q;
-        else sv[d * kStageNodes + i] = q >= 0 ? a.x[q] : T(0);
       }
     }
+    reinterpret_cast<uint4*>(list)[t] = entries;
     __syncthreads();
     if (e >= 0) {
-      const uint16_t* lc = a.lcorner + static_cast<size_t>(b) * 8 * kBlockElems + t;
-      int li[8];
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
-        li[k] = lc[k * kBlockElems];
         if constexpr (!SSP) {
           X[k] = sxyz[li[k]];
           Y[k] = sxyz[kStageNodes + li[k]];
@@ -330,73 +363,83 @@ __global__ __launch_bounds__(kBlockElems, sizeof(T) == 8 ? 2 : 4) void hex8_bloc
       element([&](int i) { return sv[(i % 3) * kStageNodes + li[i / 3]]; });
     }
     __syncthreads();  // the staging area becomes the slots
-  } else if (e >= 0) {  // per-element gathers
-    const size_t P = static_cast<size_t>(a.padded);
+  } else {  // per-element gathers
+    reinterpret_cast<uint4*>(list)[t] = entries;
+    if (e >= 0) {
+      const size_t P = static_cast<size_t>(a.padded);
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const int n = a.node[k * P + e];
-      if constexpr (!SSP) {
-        X[k] = load_coord<T>(a.coords64, a.coords32, n);
-        Y[k] = load_coord<T>(a.coords64, a.coords32, static_cast<size_t>(a.nnode) + n);
-        Z[k] = load_coord<T>(a.coords64, a.coords32, 2 * static_cast<size_t>(a.nnode) + n);
-      }
+      for (int k = 0; k < 8; ++k) {
+        const int n = a.node[k * P + e];
+        if constexpr (!SSP) {
+          X[k] = load_coord<T>(a.coords64, a.coords32, n);
+          Y[k] = load_coord<T>(a.coords64, a.coords32, static_cast<size_t>(a.nnode) + n);
+          Z[k] = load_coord<T>(a.coords64, a.coords32, 2 * static_cast<size_t>(a.nnode) + n);
+        }
 #pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        const int q = a.node_eq[3 * n + d];
-        eqe[3 * k + d] = q;
-        if constexpr (!DIAG) V[3 * k + d] = q >= 0 ? a.x[q] : T(0);
+        for (int d = 0; d < 3; ++d) {
+          const int q = a.node_eq[3 * n + d];
+          eqe[3 * k + d] = q;
+          if constexpr (!DIAG) V[3 * k + d] = q >= 0 ? a.x[q] : T(0);
+        }
       }
+      coefficients();
+      element([&](int i) { return V[i]; });
     }
-    element([&](int i) { return V[i]; });
   }
   if (e >= 0) {
 #pragma unroll
     for (int k = 0; k < 24; ++k) slots[k * kBlockElems + t] = out[k];
   }
+  // A node's output words: its slots, its partial's place and its equations, two nodes a thread at
+  // a time; the first two are loaded before the barrier.
+  uint32_t sc[2];
+  int part[2], q[2][3];
+  auto words = [&](int at) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int ln = min(at + h * kBlockElems, ln1 - 1);
+      sc[h] = a.ln_slots[ln];
+      part[h] = a.ln_part[ln];
+#pragma unroll
+      for (int d = 0; d < 3; ++d) q[h][d] = a.ln_eq[d * tot + ln];
+    }
+  };
+  if (ln0 + t < ln1) words(ln0 + t);
   __syncthreads();
-  const uint16_t* list = a.slot_list + static_cast<size_t>(b) * 8 * kBlockElems;
-  for (int ln = ln0 + t; ln < ln1; ln += kBlockElems) {
-    const uint32_t sc = a.ln_slots[ln];
-    const int s0 = sc & 0xffff, ns = sc >> 16;
-    T acc0 = 0, acc1 = 0, acc2 = 0;
-    // the node's (element, corner) slots, eight at a time: their list entries are loaded before
-    // the LDS reads use them (one round of memory latency per eight, not one per slot)
-    for (int j0 = 0; j0 < ns; j0 += 8) {
-      int sl[8];
+  for (int at = ln0 + t; at < ln1; at += 2 * kBlockElems) {
+    if (at != ln0 + t) words(at);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) sl[j] = j0 + j < ns ? list[s0 + j0 + j] : -1;
+    for (int h = 0; h < 2; ++h) {
+      const int ln = at + h * kBlockElems;
+      if (ln >= ln1) break;
+      const int s0 = sc[h] & 0xffff, ns = sc[h] >> 16;
+      T acc[3] = {T(0), T(0), T(0)};
+      for (int j = 0; j < ns; ++j) {
+        const int sl = list[s0 + j], el = sl >> 3, corner = sl & 7;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        if (sl[j] < 0) break;
-        const int el = sl[j] >> 3, corner = sl[j] & 7;
-        acc0 += slots[(3 * corner) * kBlockElems + el];
-        acc1 += slots[(3 * corner + 1) * kBlockElems + el];
-        acc2 += slots[(3 * corner + 2) * kBlockElems + el];
+        for (int d = 0; d < 3; ++d) acc[d] += slots[(3 * corner + d) * kBlockElems + el];
       }
-    }
-    const T acc[3] = {acc0, acc1, acc2};
-    const int part = a.ln_part[ln];
-    if (part >= 0) {  // a node other blocks touch too: this block's partial sum
+      if (part[h] >= 0) {  // a node other blocks touch too: this block's partial sum
 #pragma unroll
-      for (int d = 0; d < 3; ++d) partial[3 * static_cast<size_t>(part) + d] = acc[d];
-      continue;
-    }
-    if (a.ynode) {  // tied mesh: node space, contracted afterwards
-      const int n = static_cast<int>(a.lnode[ln]);
+        for (int d = 0; d < 3; ++d) partial[3 * static_cast<size_t>(part[h]) + d] = acc[d];
+      } else if (a.ynode) {  // tied mesh: node space, contracted afterwards
+        const int n = static_cast<int>(a.lnode[ln]);
 #pragma unroll
-      for (int d = 0; d < 3; ++d) a.ynode[3 * static_cast<size_t>(n) + d] = acc[d];
-    } else {
+        for (int d = 0; d < 3; ++d) a.ynode[3 * static_cast<size_t>(n) + d] = acc[d];
+      } else {
 #pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        const int q = a.ln_eq[d * tot + ln];
-        if (q < 0) continue;
-        a.y[q] = a.accumulate ? a.y[q] + acc[d] : acc[d];
+        for (int d = 0; d < 3; ++d) {
+          const int r = q[h][d];
+          if (r < 0) continue;
+          a.y[r] = a.accumulate ? a.y[r] + acc[d] : acc[d];
+        }
       }
     }
   }
 }
 
-// The nodes several blocks touch: their blocks' partial sums added in block order.
+// The nodes several blocks touch: their blocks' partial sums added in block order, four loads of
+// each component in flight (202,000 nodes: 7.4 -> 6.8 us).
 template <typename T>
 __global__ void block_shared_sum_kernel(int32_t nshared, const int32_t* __restrict__ sh_node,
                                         const int32_t* __restrict__ sh_start, const T* __restrict__ partial,
@@ -405,20 +448,30 @@ __global__ void block_shared_sum_kernel(int32_t nshared, const int32_t* __restri
   if (done && *done) return;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= nshared) return;
-  const int n = sh_node[i];
+  const int n = sh_node[i], s0 = sh_start[i], s1 = sh_start[i + 1];
   T acc[3] = {T(0), T(0), T(0)};
-  for (int s = sh_start[i]; s < sh_start[i + 1]; ++s)
+  int q[3];
 #pragma unroll
-    for (int d = 0; d < 3; ++d) acc[d] += partial[3 * static_cast<size_t>(s) + d];
+  for (int d = 0; d < 3; ++d) q[d] = node_eq[3 * n + d];
+  for (int s = s0; s < s1; s += 4) {  // four partials' loads in flight, added in block order
+    T p[4][3];
+#pragma unroll
+    for (int h = 0; h < 4; ++h)
+#pragma unroll
+      for (int d = 0; d < 3; ++d) p[h][d] = partial[3 * static_cast<size_t>(min(s + h, s1 - 1)) + d];
+#pragma unroll
+    for (int h = 0; h < 4; ++h)
+#pragma unroll
+      for (int d = 0; d < 3; ++d) acc[d] = s + h < s1 ? acc[d] + p[h][d] : acc[d];
+  }
   if (ynode) {
 #pragma unroll
     for (int d = 0; d < 3; ++d) ynode[3 * static_cast<size_t>(n) + d] = acc[d];
   } else {
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-      const int q = node_eq[3 * n + d];
-      if (q < 0) continue;
-      y[q] = accumulate ? y[q] + acc[d] : acc[d];
+      if (q[d] < 0) continue;
+      y[q[d]] = accumulate ? y[q[d]] + acc[d] : acc[d];
     }
   }
 }
@@ -484,7 +537,7 @@ __global__ void contract_kernel(int32_t neq, const int32_t* __restrict__ start, 
 template <typename T, bool DIAG>
 int launch_operator(fx_batch* b, const KernelArgs<T>& args) {
   hipStream_t st = b->ctx->stream;
-  const size_t smem = sizeof(T) * 24 * kBlockElems;
+  const size_t smem = (sizeof(T) * 24 + sizeof(uint16_t) * 8) * kBlockElems;
   T* partial;
   if constexpr (sizeof(T) == 8) partial = b->partial64;
   else partial = b->partial32;
