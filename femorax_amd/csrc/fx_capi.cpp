@@ -271,7 +271,7 @@ void fx_batch_destroy(fx_batch* b) {
                   b->tiles, b->words, b->tile_slots, b->cell_param, b->orphans, b->shared_word, b->shared_start,
                   b->shared_meta, b->tied_word, b->tied_start, b->tie_idx, b->tie_val, b->partial64, b->partial32, b->perm, b->lumped_m, b->lumped_am, b->body, b->pimy_params,
                   b->state_c, b->state_t, b->tangent, b->tangent32, b->slots, b->gather_start, b->gather_list, b->long_eqs, b->pimy_touched, b->dyn, b->gm,
-                  b->cres, b->clist, b->ccount, b->nodal_m, b->nodal_am, b->nodal_m32, b->nodal_am32, b->eq_dir_dev,
+                  b->ceps, b->pimy_fail, b->clist, b->ccount, b->nodal_m, b->nodal_am, b->nodal_m32, b->nodal_am32, b->eq_dir_dev,
                   b->words_ref, b->shared_word_ref, b->tied_word_ref, b->orphans_ref, b->ssp_elem, b->ssp_box,
                   b->kx, b->ky, b->kz, b->cg_state, b->cg_red, b->internal_of_dev,
                   b->shared_at};
@@ -1389,7 +1389,7 @@ int fx_pimy_batch_create(fx_ctx* ctx, const fx_pimy_batch_desc* d, uint32_t flag
   ok(dev_upload(ctx, b->pimy_params, pp.data(), pp.size(), by)) &&
       ok(dev_zeros(ctx, b->state_c, np * fx::kPimyNState, by)) && ok(dev_zeros(ctx, b->state_t, np * fx::kPimyNState, by)) &&
       ok(dev_zeros(ctx, b->pimy_touched, np, by)) &&
-      ok(dev_zeros(ctx, b->tangent, np * 21, by)) &&
+      ok(dev_zeros(ctx, b->tangent, np * 21, by)) && ok(dev_zeros(ctx, b->pimy_fail, np, by)) &&
       // FX_BATCH_FP32: the FP32 operator (an FP32 copy of the tangents) and the mixed CG's FP32 vectors
       ok((flags & FX_BATCH_FP32) ? dev_zeros(ctx, b->tangent32, np * 21, by) : FX_OK) &&
       ok((flags & FX_BATCH_FP32) ? dev_zeros(ctx, b->work32, static_cast<size_t>(9) * std::max(1, d->neq), by) : FX_OK) &&
@@ -1400,7 +1400,7 @@ int fx_pimy_batch_create(fx_ctx* ctx, const fx_pimy_batch_desc* d, uint32_t flag
       ok(long_eqs.empty() ? FX_OK : dev_upload(ctx, b->long_eqs, long_eqs.data(), long_eqs.size(), by)) &&
       ok((b->nlong = static_cast<int32_t>(long_eqs.size()), FX_OK)) &&
       (!(flags & FX_BATCH_COMPACT) ||
-       (ok(dev_zeros(ctx, b->cres, np * 33, by)) && ok(dev_zeros(ctx, b->clist, np, by)) &&
+       (ok(dev_zeros(ctx, b->ceps, np * 6, by)) && ok(dev_zeros(ctx, b->clist, np, by)) &&
         ok(dev_zeros(ctx, b->ccount, static_cast<size_t>(1), by)))) &&
       ok(fx::pimy_batch_init(b));
   if (rc == FX_OK) {

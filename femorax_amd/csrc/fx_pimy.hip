@@ -81,7 +81,8 @@ struct PimyBatchArgs {
   int32_t* touched; // per point: the highest surface whose centre an update has written
   double* slots;    // [24 * padded]
   fx_coeffs k;
-  double* cres;     // compacted return map: [33 * npts] stress, tangent (upper), strain
+  int8_t* fail;     // per point: its last update failed (the force then has NaN stress)
+  double* ceps;     // compacted return map: [6 * npts] the plastic points' strains
   int32_t* clist;
   int32_t* ccount;
   int32_t unit_dir;  // operator: >= 0 replaces x by the rigid unit translation in that direction
@@ -214,18 +215,41 @@ __device__ __forceinline__ double gauss_N(int gp, int k) {
   return cxy * fz;
 }
 
-// The internal force: the update at u at every point (STORE also keeps the tangents; REPLAY takes
-// each point's stress and tangent from the compacted pass instead of updating; DAMP adds the
-// Rayleigh damping force at the velocities a.v, std_brick.hpp:409-464). One thread per point.
-// A point leaves in LDS its node forces (and damping terms) and its dvol, 25 (49) values; the
-// element's eight lanes then sum a node each and form its body terms. The registers are held to 256, two waves per
-// SIMD (the return map's history loads then overlap another wave's arithmetic): the element's
-// geometry is formed again after the return map instead of held through it, the tangent kept as
-// its parts (coefficient, deviator, G, K) and the damping's D, D_0 and D_c formed entry by entry.
-// DAMP blocks hold half the points.
-template <int MODE, bool STORE, bool REPLAY = false, bool DAMP = false>
-__global__ __launch_bounds__(kPointsPerBlock, 2) void pimy_batch_kernel(PimyBatchArgs a) {
-  static_assert(MODE == 0, "the operator and its diagonal run in pimy_operator_kernel");
+// The strain at u (a.x) of element e's Gauss point gp.
+__device__ inline void trial_strain(const PimyBatchArgs& a, int e, int gp, double (&eps)[6]) {
+  double X[8], Y[8], Z[8], u[24];
+  int eq[24];
+  element_geometry(a, e, X, Y, Z, eq);
+  Shape<double> s;
+  gauss_shape(X, Y, Z, gp, s);
+  for (int k = 0; k < 24; ++k) u[k] = eq[k] >= 0 ? a.x[eq[k]] : 0.0;
+  point_strain(s, u, eps);
+}
+
+// The internal force in two launches. First the return map at u, one thread per Gauss point: the
+// strain, the update, the trial history (and whether it failed). It is a serial chain of FP64
+// divides, square roots and dependent reads of the surfaces' centres, so what it needs is waves:
+// without the element's force beside it it fits three per SIMD (168 registers), where one kernel
+// for both held two. 40^3 column, points yielding: 1,270 and 1,620 (damped) us for both in one
+// kernel, now 1,130 and a force of 59 and 78; held to two waves (no spills) 1,270, four 1,180.
+__global__ __launch_bounds__(kPointsPerBlock, 3) void pimy_trial_kernel(PimyBatchArgs a) {
+  const int t = threadIdx.x;
+  const int e = blockIdx.x * kElemsPerBlock + t / 8, gp = t % 8;
+  if (e >= a.count) return;
+  const int64_t pt = static_cast<int64_t>(e) * 8 + gp;
+  double eps[6];
+  trial_strain(a, e, gp, eps);
+  a.fail[pt] = pimy_trial(a.params[a.param[e]], a.C + pt, a.T + pt, a.npts, eps, a.touched + pt) ? 0 : 1;
+}
+
+// Then the element's force from the trial history: the point's stress is its trial stress (NaN where
+// the update failed), its tangent (STORE keeps it) and the Rayleigh damping force at the
+// velocities a.v (DAMP, std_brick.hpp:409-464) come from its trial moduli, deviator and active
+// surface. One thread per point leaves its node forces (and damping terms) and its dvol in LDS;
+// the element's eight lanes then sum a node each and form its body terms. DAMP blocks hold half
+// the points.
+template <bool STORE, bool DAMP>
+__global__ __launch_bounds__(kPointsPerBlock, 2) void pimy_force_kernel(PimyBatchArgs a) {
   constexpr int PTS = DAMP ? kPointsPerBlock / 2 : kPointsPerBlock, W = DAMP ? 6 : 3;
   // per point: 8 nodes x (3 force terms [, 3 damping terms]), then dvol
   __shared__ double part[PTS][8 * W + 1];
@@ -236,80 +260,62 @@ __global__ __launch_bounds__(kPointsPerBlock, 2) void pimy_batch_kernel(PimyBatc
     const PimyParams& p = a.params[a.param[e]];
     const int64_t pt = static_cast<int64_t>(e) * 8 + gp;
     double* mine = part[t];
-    if constexpr (MODE == 0) {
-      // the point's tangent as its parts (entries formed where they are used, the same values)
-      double sig[6];
-      PimyTangentParts Dt{};
-      if constexpr (REPLAY) {
-        for (int c = 0; c < 6; ++c) sig[c] = a.cres[c * a.npts + pt];
-        if constexpr (STORE)
-          for (int w = 0; w < 21; ++w) a.tangent[tangent_at(a, e, gp, w)] = a.cres[(6 + w) * a.npts + pt];
-      } else {
-        // the strain in a scope of its own: the geometry is formed again after the return map
-        // rather than held through it (the same operations, so the same values)
-        double eps[6];
-        {
-          double X[8], Y[8], Z[8], u[24];
-          int eq[24];
-          element_geometry(a, e, X, Y, Z, eq);
-          Shape<double> s;
-          gauss_shape(X, Y, Z, gp, s);
-          for (int k = 0; k < 24; ++k) u[k] = eq[k] >= 0 ? a.x[eq[k]] : 0.0;
-          point_strain(s, u, eps);
-        }
-        pimy_update_parts(p, a.C + pt, a.T + pt, a.npts, eps, sig, Dt, a.touched + pt);
-        if constexpr (STORE) {
-          int w = 0;
-          for (int i = 0; i < 6; ++i)
-            for (int j = i; j < 6; ++j, ++w) a.tangent[tangent_at(a, e, gp, w)] = Dt.entry(p.load_stage, i, j);
+    double sig[6];
+    for (int c = 0; c < 6; ++c) sig[c] = a.T[(kPStress + c) * a.npts + pt];
+    if (a.fail[pt])
+      for (int c = 0; c < 6; ++c) sig[c] = NAN;
+    PimyTangentParts Dt{};
+    if constexpr (STORE || DAMP) Dt = pimy_committed_tangent_parts(p, a.T + pt, a.npts);  // of the trial history
+    if constexpr (STORE) {
+      int w = 0;
+      for (int i = 0; i < 6; ++i)
+        for (int j = i; j < 6; ++j, ++w) a.tangent[tangent_at(a, e, gp, w)] = Dt.entry(p.load_stage, i, j);
+    }
+    double X[8], Y[8], Z[8];
+    int eq[24];
+    element_geometry(a, e, X, Y, Z, eq);
+    Shape<double> s;
+    gauss_shape(X, Y, Z, gp, s);
+    for (int j = 0; j < 8; ++j) {
+      double rj[3];
+      node_force(s, sig, j, rj);
+      for (int q = 0; q < 3; ++q) mine[W * j + q] = rj[q];
+    }
+    mine[8 * W] = s.dvol;  // the body terms s.dvol b N_j are formed by the summing lane
+    if constexpr (DAMP) {
+      // sigma_d = (betaK D + betaKinit D_0 + betaKcomm D_c) B v; the node terms B_j^T sigma_d dvol
+      // + alphaM N_j dvol rho v (point_update_shape :420-442, point_node_contribution :448-464)
+      const bool stiff = stiffness_damping(p);
+      double vel[24], dsig[6] = {0, 0, 0, 0, 0, 0}, vgp[3] = {0, 0, 0};
+      for (int k = 0; k < 24; ++k) vel[k] = eq[k] >= 0 ? a.v[eq[k]] : 0.0;
+      if (stiff) {
+        // D_0 and D_c entry by entry (the same values as the matrices, without holding them)
+        double rate[6];
+        PimyTangentParts Dc{};
+        if (p.betaKcomm != 0.0) Dc = pimy_committed_tangent_parts(p, a.C + pt, a.npts);
+        point_strain(s, vel, rate);
+        for (int r = 0; r < 6; ++r) {
+          double sum = 0.0;
+          for (int c = 0; c < 6; ++c) {
+            double Drc = p.betaK * Dt.entry(p.load_stage, r, c);
+            if (p.betaKinit != 0.0) Drc += p.betaKinit * initial_entry(p, r, c);
+            if (p.betaKcomm != 0.0) Drc += p.betaKcomm * Dc.entry(p.load_stage, r, c);
+            sum += Drc * rate[c];
+          }
+          dsig[r] = sum;
         }
       }
-      double X[8], Y[8], Z[8];
-      int eq[24];
-      element_geometry(a, e, X, Y, Z, eq);
-      Shape<double> s;
-      gauss_shape(X, Y, Z, gp, s);
+      if (p.alphaM != 0.0 && p.mass_type == 0)
+        for (int j = 0; j < 8; ++j)
+          for (int q = 0; q < 3; ++q) vgp[q] += s.N[j] * vel[3 * j + q];
       for (int j = 0; j < 8; ++j) {
-        double rj[3];
-        node_force(s, sig, j, rj);
-        for (int q = 0; q < 3; ++q) mine[W * j + q] = rj[q];
-      }
-      mine[8 * W] = s.dvol;  // the body terms s.dvol b N_j are formed by the summing lane
-      if constexpr (DAMP) {
-        // sigma_d = (betaK D + betaKinit D_0 + betaKcomm D_c) B v; the node terms B_j^T sigma_d dvol
-        // + alphaM N_j dvol rho v (point_update_shape :420-442, point_node_contribution :448-464)
-        const bool stiff = stiffness_damping(p);
-        double vel[24], dsig[6] = {0, 0, 0, 0, 0, 0}, vgp[3] = {0, 0, 0};
-        for (int k = 0; k < 24; ++k) vel[k] = eq[k] >= 0 ? a.v[eq[k]] : 0.0;
-        if (stiff) {
-          // D_0 and D_c entry by entry (the same values as the matrices, without holding them)
-          double rate[6];
-          PimyTangentParts Dc{};
-          if (p.betaKcomm != 0.0) Dc = pimy_committed_tangent_parts(p, a.C + pt, a.npts);
-          point_strain(s, vel, rate);
-          for (int r = 0; r < 6; ++r) {
-            double sum = 0.0;
-            for (int c = 0; c < 6; ++c) {
-              double Drc = p.betaK * Dt.entry(p.load_stage, r, c);
-              if (p.betaKinit != 0.0) Drc += p.betaKinit * initial_entry(p, r, c);
-              if (p.betaKcomm != 0.0) Drc += p.betaKcomm * Dc.entry(p.load_stage, r, c);
-              sum += Drc * rate[c];
-            }
-            dsig[r] = sum;
-          }
+        double dj[3] = {0, 0, 0};
+        if (stiff) node_force(s, dsig, j, dj);
+        if (p.alphaM != 0.0) {
+          const double temp = s.N[j] * s.dvol * p.rho;
+          for (int q = 0; q < 3; ++q) dj[q] += p.alphaM * temp * (p.mass_type == 0 ? vgp[q] : vel[3 * j + q]);
         }
-        if (p.alphaM != 0.0 && p.mass_type == 0)
-          for (int j = 0; j < 8; ++j)
-            for (int q = 0; q < 3; ++q) vgp[q] += s.N[j] * vel[3 * j + q];
-        for (int j = 0; j < 8; ++j) {
-          double dj[3] = {0, 0, 0};
-          if (stiff) node_force(s, dsig, j, dj);
-          if (p.alphaM != 0.0) {
-            const double temp = s.N[j] * s.dvol * p.rho;
-            for (int q = 0; q < 3; ++q) dj[q] += p.alphaM * temp * (p.mass_type == 0 ? vgp[q] : vel[3 * j + q]);
-          }
-          for (int q = 0; q < 3; ++q) mine[W * j + 3 + q] = dj[q];
-        }
+        for (int q = 0; q < 3; ++q) mine[W * j + 3 + q] = dj[q];
       }
     }
   }
@@ -540,36 +546,24 @@ __global__ __launch_bounds__(kPointsPerBlock) void pimy_point_operator_kernel(Pi
   for (int q = 0; q < 3; ++q) a.slots[(3 * gp + q) * P + e] = out[q];
 }
 
-// The compacted return map (compacted_kernels.hpp:85-202). Predict: one thread per Gauss point,
-// the strain as the fused kernel forms it, the elastic predictor; an elastic point is finished
-// (stress and tangent stored), a plastic one keeps its strain and joins the list (one atomic per
+// The compacted return map (compacted_kernels.hpp:85-202), in place of pimy_trial_kernel. Predict:
+// one thread per Gauss point, the strain as the fused kernel forms it, the elastic predictor; an
+// elastic point is finished, a plastic one keeps its strain and joins the list (one atomic per
 // wave). Correct: a fixed grid walks the list, one full update per listed point (the same
-// function as the fused kernel, so the same bits). The force kernel then replays the stored
-// results.
+// function as the fused kernel, so the same bits).
 __global__ __launch_bounds__(kPointsPerBlock) void pimy_predict_kernel(PimyBatchArgs a) {
   const int t = threadIdx.x;
   const int e = blockIdx.x * kElemsPerBlock + t / 8, gp = t % 8;
   bool plastic = false;
   const int64_t pt = static_cast<int64_t>(e) * 8 + gp;
   if (e < a.count) {
-    double X[8], Y[8], Z[8];
-    int eq[24];
-    element_geometry(a, e, X, Y, Z, eq);
-    const PimyParams& p = a.params[a.param[e]];
-    Shape<double> s;
-    gauss_shape(X, Y, Z, gp, s);
-    double u[24], eps[6], sig[6], D[36];
-    for (int k = 0; k < 24; ++k) u[k] = eq[k] >= 0 ? a.x[eq[k]] : 0.0;
-    point_strain(s, u, eps);
-    plastic = pimy_predict(p, a.C + pt, a.T + pt, a.npts, eps, sig, D, a.touched + pt);
-    if (plastic) {
-      for (int c = 0; c < 6; ++c) a.cres[(27 + c) * a.npts + pt] = eps[c];
-    } else {
-      for (int c = 0; c < 6; ++c) a.cres[c * a.npts + pt] = sig[c];
-      int w = 0;
-      for (int i = 0; i < 6; ++i)
-        for (int j = i; j < 6; ++j, ++w) a.cres[(6 + w) * a.npts + pt] = D[6 * i + j];
-    }
+    double eps[6], sig[6], D[36];
+    trial_strain(a, e, gp, eps);
+    plastic = pimy_predict(a.params[a.param[e]], a.C + pt, a.T + pt, a.npts, eps, sig, D, a.touched + pt);
+    if (plastic)
+      for (int c = 0; c < 6; ++c) a.ceps[c * a.npts + pt] = eps[c];
+    else
+      a.fail[pt] = sig[0] == sig[0] ? 0 : 1;
   }
   const uint64_t mask = __ballot(plastic);
   if (mask == 0) return;
@@ -585,14 +579,9 @@ __global__ __launch_bounds__(128) void pimy_correct_kernel(PimyBatchArgs a) {
   const int32_t n = *a.ccount;
   for (int32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
     const int64_t pt = a.clist[k];
-    const PimyParams& p = a.params[a.param[pt / 8]];
-    double eps[6], sig[6], D[36];
-    for (int c = 0; c < 6; ++c) eps[c] = a.cres[(27 + c) * a.npts + pt];
-    pimy_update(p, a.C + pt, a.T + pt, a.npts, eps, sig, D, a.touched + pt);
-    for (int c = 0; c < 6; ++c) a.cres[c * a.npts + pt] = sig[c];
-    int w = 0;
-    for (int i = 0; i < 6; ++i)
-      for (int j = i; j < 6; ++j, ++w) a.cres[(6 + w) * a.npts + pt] = D[6 * i + j];
+    double eps[6];
+    for (int c = 0; c < 6; ++c) eps[c] = a.ceps[c * a.npts + pt];
+    a.fail[pt] = pimy_trial(a.params[a.param[pt / 8]], a.C + pt, a.T + pt, a.npts, eps, a.touched + pt) ? 0 : 1;
   }
 }
 
@@ -687,7 +676,8 @@ PimyBatchArgs batch_args(fx_batch* b, const double* x, const fx_coeffs& k, const
   a.touched = b->pimy_touched;
   a.slots = b->slots;
   a.k = k;
-  a.cres = b->cres;
+  a.fail = b->pimy_fail;
+  a.ceps = b->ceps;
   a.clist = b->clist;
   a.ccount = b->ccount;
   a.unit_dir = -1;
@@ -1108,17 +1098,21 @@ int run_pimy(fx_batch* b, const PimyBatchArgs& a, double* y, const int32_t* done
     if (b->ssp) {  // SSPbrick: one thread per element, its one point
       if (b->count > 0)
         hipLaunchKernelGGL(pimy_ssp_kernel<STORE>, dim3((b->count + 127) / 128), dim3(128), 0, st, a);
-    } else if (b->count > 0 && a.v) {  // the damping force: the fused return map, half blocks
-      const dim3 g2((b->count + kElemsPerBlock / 2 - 1) / (kElemsPerBlock / 2));
-      hipLaunchKernelGGL((pimy_batch_kernel<0, STORE, false, true>), g2, dim3(kPointsPerBlock / 2), 0, st, a);
-    } else if (b->count > 0 && b->cres) {  // compacted: predict, correct, replay
-      hipLaunchKernelGGL(pimy_predict_kernel, grid, dim3(kPointsPerBlock), 0, st, a);
-      const unsigned cgrid = static_cast<unsigned>(std::min<int64_t>((b->npts + 127) / 128, 2048));
-      hipLaunchKernelGGL(pimy_correct_kernel, dim3(cgrid), dim3(128), 0, st, a);
-      hipLaunchKernelGGL(pimy_clear_count_kernel, dim3(1), dim3(64), 0, st, a.ccount);
-      hipLaunchKernelGGL((pimy_batch_kernel<0, STORE, true>), grid, dim3(kPointsPerBlock), 0, st, a);
     } else if (b->count > 0) {
-      hipLaunchKernelGGL((pimy_batch_kernel<0, STORE>), grid, dim3(kPointsPerBlock), 0, st, a);
+      if (b->ceps) {  // compacted: predict, correct
+        hipLaunchKernelGGL(pimy_predict_kernel, grid, dim3(kPointsPerBlock), 0, st, a);
+        const unsigned cgrid = static_cast<unsigned>(std::min<int64_t>((b->npts + 127) / 128, 2048));
+        hipLaunchKernelGGL(pimy_correct_kernel, dim3(cgrid), dim3(128), 0, st, a);
+        hipLaunchKernelGGL(pimy_clear_count_kernel, dim3(1), dim3(64), 0, st, a.ccount);
+      } else {
+        hipLaunchKernelGGL(pimy_trial_kernel, grid, dim3(kPointsPerBlock), 0, st, a);
+      }
+      if (a.v) {  // with the damping force: half blocks
+        const dim3 g2((b->count + kElemsPerBlock / 2 - 1) / (kElemsPerBlock / 2));
+        hipLaunchKernelGGL((pimy_force_kernel<STORE, true>), g2, dim3(kPointsPerBlock / 2), 0, st, a);
+      } else {
+        hipLaunchKernelGGL((pimy_force_kernel<STORE, false>), grid, dim3(kPointsPerBlock), 0, st, a);
+      }
     }
   } else {
     launch_operator_slots<MODE == 2>(b, a);

@@ -551,12 +551,12 @@ struct Point {
     finish(sig, D);
   }
 
-  // the same with the tangent as its parts (coeff, devia, G, K; entries by tangent_entry)
-  __device__ void update_parts(const double (&eps)[6], double (&sig)[6], double& coeff, V6& devia) {
+  // the trial history alone; whether the update succeeded
+  __device__ bool update_trial(const double (&eps)[6]) {
     get_stress(eps, false);
-    tangent_parts(coeff, devia);
-    double D[36];  // finish's tangent, unused (its stores fold away)
+    double sig[6], D[36];  // finish's outputs, unused (their stores fold away)
     finish(sig, D);
+    return ok;
   }
 
   // The compacted path's predictor (pressure_independ_multi_yield.hpp:247-255): a point that
@@ -582,11 +582,16 @@ __device__ inline void pimy_update(const PimyParams& p, const double* C, double*
   if (touched && pt.moved > copy) *touched = pt.moved;
 }
 
-// pimy_update with the tangent as its parts (PimyTangentParts below, load_stage p.load_stage)
-struct PimyTangentParts;
-__device__ inline void pimy_update_parts(const PimyParams& p, const double* C, double* T, int64_t stride,
-                                         const double (&eps)[6], double (&sig)[6], PimyTangentParts& parts,
-                                         int32_t* touched = nullptr);
+// The update into the trial history alone (its stress and tangent are read from there); false where
+// it failed.
+__device__ inline bool pimy_trial(const PimyParams& p, const double* C, double* T, int64_t stride,
+                                  const double (&eps)[6], int32_t* touched) {
+  const int copy = *touched;
+  pimy::Point pt(p, C, T, stride, copy);
+  const bool ok = pt.update_trial(eps);
+  if (pt.moved > copy) *touched = pt.moved;
+  return ok;
+}
 
 // committed_tangent (:162-168): getTangent with the committed stress, active surface, surfaces
 // and moduli (the surfaces are read from C; nothing is written).
@@ -600,7 +605,7 @@ __device__ inline void pimy_committed_tangent(const PimyParams& p, const double*
   pt.tangent(D);
 }
 
-// The committed tangent's parts (entries by pimy::Point::tangent_entry with p.load_stage, G, K):
+// A history's tangent as its parts (entries by pimy::Point::tangent_entry with p.load_stage, G, K):
 // the damping force forms sigma_d entry by entry without holding the 6 x 6 matrix.
 struct PimyTangentParts {
   double coeff, G, K;
@@ -609,17 +614,6 @@ struct PimyTangentParts {
     return pimy::Point::tangent_entry(load_stage, coeff, devia, G, K, i, j);
   }
 };
-__device__ inline void pimy_update_parts(const PimyParams& p, const double* C, double* T, int64_t stride,
-                                         const double (&eps)[6], double (&sig)[6], PimyTangentParts& parts,
-                                         int32_t* touched) {
-  const int copy = touched ? *touched : -1;
-  pimy::Point pt(p, C, T, stride, copy);
-  pt.update_parts(eps, sig, parts.coeff, parts.devia);
-  parts.G = pt.G;
-  parts.K = pt.K;
-  if (touched && pt.moved > copy) *touched = pt.moved;
-}
-
 __device__ inline PimyTangentParts pimy_committed_tangent_parts(const PimyParams& p, const double* C, int64_t stride) {
   pimy::Point pt(p, C, const_cast<double*>(C), stride);
   pt.trial = pt.load_t2(kPStress);
