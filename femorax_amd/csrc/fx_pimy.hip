@@ -227,12 +227,13 @@ __device__ inline void trial_strain(const PimyBatchArgs& a, int e, int gp, doubl
 }
 
 // The internal force in two launches. First the return map at u, one thread per Gauss point: the
-// strain, the update, the trial history (and whether it failed). It is a serial chain of FP64
-// divides, square roots and dependent reads of the surfaces' centres, so what it needs is waves:
-// without the element's force beside it it fits three per SIMD (168 registers), where one kernel
-// for both held two. 40^3 column, points yielding: 1,270 and 1,620 (damped) us for both in one
-// kernel, now 1,130 and a force of 59 and 78; held to two waves (no spills) 1,270, four 1,180.
-__global__ __launch_bounds__(kPointsPerBlock, 3) void pimy_trial_kernel(PimyBatchArgs a) {
+// strain, the update, the trial history (and whether it failed). Its walk over the surfaces is a
+// serial chain of FP64 arithmetic, about 30,000 instructions a point: the 40^3 column's points yielding
+// took 1,270 (1,620 damped) us with the force beside it in one kernel, 1,130 by itself, and 700 since
+// the walk holds its surfaces in registers (450 us of that is issue of vector instructions, the
+// history's 1.3 GB would take 270). Two waves a SIMD hold it without spills (224 registers); three
+// spill 66 and took 4 % longer.
+__global__ __launch_bounds__(kPointsPerBlock, 2) void pimy_trial_kernel(PimyBatchArgs a) {
   const int t = threadIdx.x;
   const int e = blockIdx.x * kElemsPerBlock + t / 8, gp = t % 8;
   if (e >= a.count) return;

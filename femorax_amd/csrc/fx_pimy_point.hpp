@@ -29,36 +29,27 @@ __device__ inline double dd(const V6& a, const V6& b) {
   for (int i = 0; i < 3; ++i) r += a.v[i] * b.v[i] + 2 * a.v[i + 3] * b.v[i + 3];
   return r;
 }
-// a = s * a + f * o with OpenSees Vector::addVector's special cases (t2_vector.hpp:40-75)
+// a = s * a + f * o with OpenSees Vector::addVector's special case f = 0 (t2_vector.hpp:40-75; its
+// others, f = 1 and -1, s = 0 and 1, give the general form's values)
 __device__ inline void axpby(V6& a, double s, const V6& o, double f) {
-  if (f == 0.0) {
-    if (s == 1.0) return;
-    if (s == 0.0) {
-      a = zero6();
-      return;
-    }
-    for (int i = 0; i < 6; ++i) a.v[i] *= s;
-    return;
-  }
-  for (int i = 0; i < 6; ++i) {
-    if (s == 1.0) {
-      if (f == 1.0) a.v[i] += o.v[i];
-      else if (f == -1.0) a.v[i] -= o.v[i];
-      else a.v[i] += o.v[i] * f;
-    } else if (s == 0.0) {
-      if (f == 1.0) a.v[i] = o.v[i];
-      else if (f == -1.0) a.v[i] = -(o.v[i]);
-      else a.v[i] = o.v[i] * f;
-    } else {
-      if (f == 1.0) a.v[i] = a.v[i] * s + o.v[i];
-      else if (f == -1.0) a.v[i] = a.v[i] * s - o.v[i];
-      else a.v[i] = a.v[i] * s + o.v[i] * f;
-    }
-  }
+  if (s != 1.0)
+    for (int i = 0; i < 6; ++i) a.v[i] = s == 0.0 ? 0.0 : a.v[i] * s;
+  if (f != 0.0)
+    for (int i = 0; i < 6; ++i) a.v[i] = s == 0.0 ? o.v[i] * f : a.v[i] + o.v[i] * f;
 }
+// x / f where r is 1 / f correctly rounded: the quotient's residual, exact in one FMA, corrects x r
+// (Markstein, "Computation of elementary functions on the IBM RISC System/6000 processor", 1990; the
+// same value as the division in 10^9 random pairs), then the hardware's cases of zeros, infinities
+// and NaN. Four operations for what a division takes eleven.
+__device__ inline double over(double x, double f, double r) {
+  const double q = x * r;
+  return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-f, q, x), r, q), f, x);
+}
+__device__ inline double third(double x) { return over(x, 3.0, 1.0 / 3.0); }
 // a /= f, with the 1e200 fill of a division by zero (t2_vector.hpp:86-92)
 __device__ inline void divide(V6& a, double f) {
-  for (int i = 0; i < 6; ++i) a.v[i] = f == 0.0 ? kBig : a.v[i] / f;
+  const double r = 1.0 / f;
+  for (int i = 0; i < 6; ++i) a.v[i] = f == 0.0 ? kBig : over(a.v[i], f, r);
 }
 
 // a symmetric tensor with its deviator and mean (soil::T2)
@@ -67,7 +58,7 @@ struct T2 {
   double vol;
   __device__ void set(const V6& x, bool engineering) {
     t2 = x;
-    vol = (t2.v[0] + t2.v[1] + t2.v[2]) / 3.0;
+    vol = third(t2.v[0] + t2.v[1] + t2.v[2]);
     for (int i = 0; i < 3; ++i) {
       dev.v[i] = t2.v[i] - vol;
       dev.v[i + 3] = t2.v[i + 3];
@@ -79,7 +70,7 @@ struct T2 {
   }
   __device__ void set_dev(const V6& d, double volume) {
     vol = volume;
-    const double dv = (d.v[0] + d.v[1] + d.v[2]) / 3.;
+    const double dv = third(d.v[0] + d.v[1] + d.v[2]);
     for (int i = 0; i < 3; ++i) {
       dev.v[i] = d.v[i] - dv;
       dev.v[i + 3] = d.v[i + 3];
@@ -141,15 +132,33 @@ __device__ inline int to_int(double x) {
   return static_cast<int>(x);
 }
 
+// A yield surface: its centre, size and plastic modulus (surface 0: all zero).
+struct Surface {
+  V6 c;
+  double sz, mod;
+};
+
 // One material point: committed history C, trial history T (strided views into the SoA state).
+// The return map walks outwards from the active surface: the active surface and the next one are
+// held in registers, a surface is read once when it becomes the next (from `from`: C, until
+// this update has written centres into T) and the active one's centre is written once when it is
+// left. Read again at each use, after stores that might alias, they were 2,100 memory
+// instructions a wave and half of its time waiting; now 680.
 struct Point {
   const PimyParams& p;
   const double* C;
   double* T;
   int64_t s;  // stride between fields
-  bool ok = true;
-  T2 cur_stress, cur_strain, trial, rate, sub_rate;
+  const double* from;
+  bool ok = true, dirty = false;
+  // With phi = 0 the surfaces' sizes and moduli never change (paramScaling is a no-op,
+  // :633-639): they are read from the parameter set and their history fields are left as
+  // initialised (same values), so an update moves 40 doubles less per point.
+  const bool fixed;
+  T2 cur_stress, trial, rate, sub_rate;
   int committed_active = 0, active = 0, e2p = 0;
+  Surface act, nxt;     // surfaces active and active + 1 (the latter while active < nsurf)
+  double inner_mod = 0;  // the modulus of surface active - 1, once a correction has crossed
   double G = 0, K = 0;
   // The surfaces whose centres get_stress copies from C into T: a batch keeps per point the
   // highest surface whose centre any update has written, and every centre above it holds its
@@ -159,29 +168,47 @@ struct Point {
   mutable int moved = 0;
 
   __device__ Point(const PimyParams& pp, const double* c, double* t, int64_t stride, int copy = -1)
-      : p(pp), C(c), T(t), s(stride), ncopy(copy < 0 || copy > pp.nsurf ? pp.nsurf : copy) {}
+      : p(pp), C(c), T(t), s(stride), from(c), fixed(pp.phi == 0.), ncopy(copy < 0 || copy > pp.nsurf ? pp.nsurf : copy) {}
 
   __device__ double c(int k) const { return C[k * s]; }
   __device__ double& t(int k) const { return T[k * s]; }
-  // With phi = 0 the surfaces' sizes and moduli never change (paramScaling is a no-op,
-  // :633-639): they are read from the parameter set and their history fields are left as
-  // initialised (same values), so an update moves 40 doubles less per point.
-  __device__ bool fixed_surfaces() const { return p.phi == 0.; }
-  __device__ double size(int i) const {
-    return i == 0 ? 0. : fixed_surfaces() ? p.size[i] : t(kPSizes + i - 1);
+  __device__ double size(int i) const { return fixed ? p.size[i] : from[(kPSizes + i - 1) * s]; }  // i >= 1
+  __device__ double modulus(int i) const { return fixed ? p.modulus[i] : from[(kPModuli + i - 1) * s]; }
+  __device__ Surface surface(int i) const {
+    Surface x{zero6(), 0., 0.};
+    if (i == 0) return x;
+    const double* q = from + (kPCenters + 6 * (i - 1)) * s;
+    for (int k = 0; k < 6; ++k) x.c.v[k] = q[k * s];
+    x.sz = size(i);
+    x.mod = modulus(i);
+    return x;
   }
-  __device__ double modulus(int i) const {
-    return i == 0 ? 0. : fixed_surfaces() ? p.modulus[i] : t(kPModuli + i - 1);
+  // a centre into the trial history; from then on surfaces are read there
+  __device__ void set_center(int i, const V6& o) {
+    from = T;
+    store_center(i, o);
   }
-  __device__ V6 center(int i) const {
-    V6 o = zero6();
-    if (i == 0) return o;
-    for (int k = 0; k < 6; ++k) o.v[k] = t(kPCenters + 6 * (i - 1) + k);
-    return o;
-  }
-  __device__ void set_center(int i, const V6& o) const {
+  __device__ void store_center(int i, const V6& o) const {
     moved = i > moved ? i : moved;
-    for (int k = 0; k < 6; ++k) t(kPCenters + 6 * (i - 1) + k) = o.v[k];
+    double* q = T + (kPCenters + 6 * (i - 1)) * s;
+    for (int k = 0; k < 6; ++k) q[k * s] = o.v[k];
+  }
+  // the active surface's centre, if this update has moved it
+  __device__ void leave() {
+    if (dirty) store_center(active, act.c);
+    dirty = false;
+  }
+  __device__ void enter(int i) {
+    active = i;
+    act = surface(i);
+    if (i < p.nsurf) nxt = surface(i + 1);
+  }
+  __device__ void outward() {  // to the next surface
+    leave();
+    inner_mod = act.mod;
+    act = nxt;
+    ++active;
+    if (active < p.nsurf) nxt = surface(active + 1);
   }
   __device__ T2 load_t2(int k) const {
     T2 x;
@@ -196,34 +223,29 @@ struct Point {
     t(k + 12) = x.vol;
   }
 
-  __device__ double yield(const T2& x, int i) const {
+  __device__ static double yield(const T2& x, const Surface& f) {
     V6 d = x.dev;
-    const V6 cc = center(i);
-    for (int k = 0; k < 6; ++k) d.v[k] -= cc.v[k];
-    const double sz = size(i);
-    return 3. / 2. * dd(d, d) - sz * sz;
+    for (int k = 0; k < 6; ++k) d.v[k] -= f.c.v[k];
+    return 3. / 2. * dd(d, d) - f.sz * f.sz;
   }
 
-  __device__ void deviator_scaling(T2& x, int i) {
-    const int n = p.nsurf;
+  // x scaled back to surface f (outermost: whether it is the last)
+  __device__ void deviator_scaling(T2& x, const Surface& f, bool outermost) {
     for (int iter = 0; iter < 100000; ++iter) {
-      const double diff = yield(x, i);
-      if (i < n && diff < 0.) {
-        const double sz = size(i);
-        const double dsz = sqrt(sz * sz + diff);
+      const double diff = yield(x, f);
+      if (!outermost && diff < 0.) {
+        const double dsz = sqrt(f.sz * f.sz + diff);
         V6 devia = x.dev, tmp;
-        const V6 cc = center(i);
-        for (int k = 0; k < 6; ++k) tmp.v[k] = devia.v[k] - cc.v[k];
-        double coeff = (sz - dsz) / dsz;
+        for (int k = 0; k < 6; ++k) tmp.v[k] = devia.v[k] - f.c.v[k];
+        double coeff = (f.sz - dsz) / dsz;
         if (coeff < 1.e-13) coeff = 1.e-13;
         axpby(devia, 1.0, tmp, coeff);
         x.set_dev(devia, x.vol);
         continue;
       }
-      if (i == n && fabs(diff) > kLow) {
-        const double sz = size(i);
+      if (outermost && fabs(diff) > kLow) {
         V6 nd = zero6();
-        axpby(nd, 0.0, x.dev, sz / sqrt(diff + sz * sz));
+        axpby(nd, 0.0, x.dev, f.sz / sqrt(diff + f.sz * f.sz));
         x.set_dev(nd, x.vol);
       }
       return;
@@ -256,6 +278,7 @@ struct Point {
     scale = pow(scale, p.pdc);
     G *= scale;
     K *= scale;
+    from = T;
     for (int i = 1; i <= p.nsurf; ++i) {
       const double pm = modulus(i) * scale;
       const double sz = size(i) * con;
@@ -274,9 +297,9 @@ struct Point {
     }
     param_scaling();
     if (cur_stress.dev_len() == 0.) return;
-    while (yield(cur_stress, ++committed_active) > 0) {
+    while (yield(cur_stress, surface(++committed_active)) > 0) {
       if (committed_active == p.nsurf) {
-        deviator_scaling(cur_stress, p.nsurf);
+        deviator_scaling(cur_stress, surface(p.nsurf), true);
         init_surface_update();
         return;
       }
@@ -298,7 +321,7 @@ struct Point {
     if (active == 0) {
       epm = 2 * G;
     } else {
-      const double pm = modulus(active);
+      const double pm = act.mod;
       epm = 2 * G * pm / (2 * G + pm);
     }
     V6 inc = zero6();
@@ -317,8 +340,7 @@ struct Point {
 
   __device__ V6 normal(const T2& x) const {
     V6 nrm = x.dev;
-    const V6 cc = center(active);
-    for (int k = 0; k < 6; ++k) nrm.v[k] -= cc.v[k];
+    for (int k = 0; k < 6; ++k) nrm.v[k] -= act.c.v[k];
     divide(nrm, sqrt(dd(nrm, nrm)));
     return nrm;
   }
@@ -332,26 +354,25 @@ struct Point {
   }
 
   __device__ T2 contact_stress() const {
-    const V6 cc = center(active);
     V6 devia = trial.dev;
-    for (int k = 0; k < 6; ++k) devia.v[k] -= cc.v[k];
+    for (int k = 0; k < 6; ++k) devia.v[k] -= act.c.v[k];
     const double Ms = sqrt(3. / 2. * dd(devia, devia));
-    const double f = size(active) / Ms;
+    const double f = act.sz / Ms;
     for (int k = 0; k < 6; ++k) devia.v[k] *= f;
-    for (int k = 0; k < 6; ++k) devia.v[k] += cc.v[k];
+    for (int k = 0; k < 6; ++k) devia.v[k] += act.c.v[k];
     T2 x;
     x.set_dev(devia, trial.vol);
     return x;
   }
 
   __device__ double loading(const T2& cs, const V6& nrm, bool crossed) const {
-    const double t1 = 2. * G, t2 = modulus(active);
+    const double t1 = 2. * G, t2 = act.mod;
     const double tt = t1 + t2;
     V6 tmp = trial.dev;
     for (int k = 0; k < 6; ++k) tmp.v[k] -= cs.dev.v[k];
     double lf = dd(nrm, tmp) / tt;
     if (crossed) {
-      const double t3 = modulus(active - 1);
+      const double t3 = inner_mod;
       lf *= (t3 - t2) / t3;
     }
     return lf;
@@ -359,7 +380,7 @@ struct Point {
 
   __device__ bool crossing_next() const {
     if (active == p.nsurf) return false;
-    return yield(trial, active + 1) > 0;
+    return yield(trial, nxt) > 0;
   }
 
   __device__ void stress_correction(bool crossed) {
@@ -371,9 +392,9 @@ struct Point {
       axpby(devia, 0.0, nrm, -2 * G * lf);
       for (int k = 0; k < 6; ++k) devia.v[k] += trial.dev.v[k];
       trial.set_dev(devia, trial.vol);
-      deviator_scaling(trial, active);
+      deviator_scaling(trial, act, active == p.nsurf);
       if (crossing_next()) {
-        active++;
+        outward();
         crossed = true;
         continue;
       }
@@ -382,12 +403,11 @@ struct Point {
   }
 
   __device__ void update_active_surface() {
-    const int n = p.nsurf;
-    if (active == n) return;
-    V6 cen = center(active);
-    const double sz = size(active);
-    const V6 outc = center(active + 1);
-    const double outsz = size(active + 1);
+    if (active == p.nsurf) return;
+    V6 cen = act.c;
+    const double sz = act.sz;
+    const V6 outc = nxt.c;
+    const double outsz = nxt.sz;
     V6 t1, t2, tmp;
     for (int k = 0; k < 6; ++k) {
       t1.v[k] = trial.dev.v[k] - cen.v[k];
@@ -404,10 +424,11 @@ struct Point {
     }
     tmp = cen;
     axpby(tmp, 1.0, t1, X);
-    const double f = 1.0 - sz / outsz;
+    const double ratio = sz / outsz;
+    const double f = 1.0 - ratio;
     for (int k = 0; k < 6; ++k) tmp.v[k] *= f;
     t2 = cen;
-    axpby(t2, 1.0, outc, -sz / outsz);
+    axpby(t2, 1.0, outc, -ratio);
     for (int k = 0; k < 6; ++k) tmp.v[k] -= t2.v[k];
     T2 dir;
     dir.set(tmp, false);
@@ -425,18 +446,17 @@ struct Point {
     }
     X = quad_root(A, B, Cc, ok);
     axpby(cen, 1.0, tmp, X);
-    set_center(active, cen);
+    act.c = cen;
+    dirty = true;
   }
 
   __device__ void update_inner_surface() {
     if (active <= 1) return;
     const V6 devia = cur_stress.dev;
-    const V6 cen = center(active);
-    const double sz = size(active);
     for (int i = 1; i < active; ++i) {
       V6 nc;
-      const double f = size(i) / sz;
-      for (int k = 0; k < 6; ++k) nc.v[k] = (cen.v[k] - devia.v[k]) * f + devia.v[k];
+      const double f = size(i) / act.sz;
+      for (int k = 0; k < 6; ++k) nc.v[k] = (act.c.v[k] - devia.v[k]) * f + devia.v[k];
       set_center(i, nc);
     }
   }
@@ -447,11 +467,9 @@ struct Point {
     coeff = 0.;
     devia = zero6();
     if (p.load_stage == 1 && active > 0) {
-      const V6 cc = center(active);
       devia = trial.dev;
-      for (int k = 0; k < 6; ++k) devia.v[k] -= cc.v[k];
-      const double sz = size(active), pm = modulus(active);
-      coeff = 6. * G * G / (2. * G + pm) / sz / sz;
+      for (int k = 0; k < 6; ++k) devia.v[k] -= act.c.v[k];
+      coeff = 6. * G * G / (2. * G + act.mod) / act.sz / act.sz;
     }
   }
 
@@ -474,27 +492,46 @@ struct Point {
       for (int j = 0; j < 6; ++j) D[6 * i + j] = tangent_entry(p.load_stage, coeff, devia, G, K, i, j);
   }
 
+  // fields k .. k + N - 1 from C into T, their loads in flight together (T may alias C to the compiler)
+  template <int N>
+  __device__ void copy_fields(int k) const {
+    const double* from = C + k * s;
+    double* to = T + k * s;
+    double w[N];
+    for (int j = 0; j < N; ++j) w[j] = from[j * s];
+    for (int j = 0; j < N; ++j) to[j * s] = w[j];
+  }
+
   // getStress (:455-509). With stop_at_correction (the compacted path's predictor) it returns
   // true, and stops, where the first stress correction would run; otherwise it sets the trial
   // stress and returns false.
   __device__ bool get_stress(const double (&eps)[6], bool stop_at_correction) {
     cur_stress = load_t2(kPStress);
-    cur_strain = load_t2(kPStrain);
     committed_active = static_cast<int>(c(kPActive));
     active = committed_active;
     e2p = static_cast<int>(c(kPE2P));
     G = c(kPG);
     K = c(kPK);
     {
-      V6 d, cs = cur_strain.engineering();
-      for (int k = 0; k < 6; ++k) d.v[k] = eps[k] - cs.v[k];
+      V6 d, sc;
+      for (int k = 0; k < 6; ++k) sc.v[k] = c(kPStrain + k);
+      for (int k = 0; k < 6; ++k) d.v[k] = eps[k] - (k < 3 ? sc.v[k] : sc.v[k] * 2.);
       rate.set(d, true);
+      for (int k = 0; k < 6; ++k) sc.v[k] += rate.t2.v[k];
+      T2 strain_commit;  // stored now, so that it is not held through the walk
+      strain_commit.set(sc, false);
+      store_t2(strain_commit, kPStrain);
     }
     // committed surfaces into the trial buffer (centres of the nsurf surfaces in use)
-    if (!fixed_surfaces())
-      for (int k = kPSizes; k < kPCenters; ++k) t(k) = c(k);
-    for (int k = kPCenters; k < kPCenters + 6 * ncopy; ++k) t(k) = c(k);
+    if (!fixed)
+      for (int k = kPSizes; k < kPCenters; k += 10) copy_fields<10>(k);
+    int k = kPCenters;
+    for (int i = 0; i + 1 < ncopy; i += 2, k += 12) copy_fields<12>(k);
+    if (ncopy & 1) copy_fields<6>(k);
     if (p.load_stage == 1 && e2p == 0) elastic_to_plastic();
+    t(kPE2P) = e2p;
+    t(kPG) = G;
+    t(kPK) = K;
     if (p.load_stage != 1) {
       double De[36];
       tangent(De);
@@ -504,23 +541,24 @@ struct Point {
         for (int j = 0; j < 6; ++j) a.v[j] += De[6 * j + i] * r.v[i];
       trial.set(a, false);
     } else {
-      active = committed_active;
+      enter(committed_active);
       sub_rate = rate;
       set_trial_stress(cur_stress);
       if (load_reversal()) {
         update_inner_surface();
-        active = 0;
+        enter(0);
       }
       const int nsub = set_sub_strain_rate();
+      if (nsub > 0) trial = cur_stress;
       for (int i = 0; i < nsub; ++i) {
-        if (i == 0) set_trial_stress(cur_stress);
-        else set_trial_stress(trial);
+        set_trial_stress(trial);
         if (active == 0 && !crossing_next()) continue;
         if (stop_at_correction) return true;
-        if (active == 0) active++;
+        if (active == 0) outward();
         stress_correction(false);
         update_active_surface();
       }
+      leave();
       double vol = K * (rate.vol * 3.);
       vol += cur_stress.vol;
       const V6 d = trial.dev;
@@ -533,15 +571,7 @@ struct Point {
   __device__ void finish(double (&sig)[6], double (&D)[36]) {
     tangent(D);
     for (int i = 0; i < 6; ++i) sig[i] = ok ? trial.t2.v[i] : NAN;
-    V6 sc = cur_strain.t2;
-    for (int k = 0; k < 6; ++k) sc.v[k] += rate.t2.v[k];
-    T2 strain_commit;
-    strain_commit.set(sc, false);
     store_t2(trial, kPStress);
-    store_t2(strain_commit, kPStrain);
-    t(kPE2P) = e2p;
-    t(kPG) = G;
-    t(kPK) = K;
     t(kPActive) = p.load_stage == 1 ? active : committed_active;
   }
 
@@ -600,6 +630,7 @@ __device__ inline void pimy_committed_tangent(const PimyParams& p, const double*
   pimy::Point pt(p, C, const_cast<double*>(C), stride);
   pt.trial = pt.load_t2(kPStress);
   pt.active = static_cast<int>(pt.c(kPActive));
+  pt.act = pt.surface(pt.active);
   pt.G = pt.c(kPG);
   pt.K = pt.c(kPK);
   pt.tangent(D);
@@ -618,6 +649,7 @@ __device__ inline PimyTangentParts pimy_committed_tangent_parts(const PimyParams
   pimy::Point pt(p, C, const_cast<double*>(C), stride);
   pt.trial = pt.load_t2(kPStress);
   pt.active = static_cast<int>(pt.c(kPActive));
+  pt.act = pt.surface(pt.active);
   pt.G = pt.c(kPG);
   pt.K = pt.c(kPK);
   PimyTangentParts t;
