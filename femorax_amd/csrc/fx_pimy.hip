@@ -60,9 +60,6 @@ __global__ void pimy_init_kernel(int64_t npts, const PimyParams* __restrict__ pa
 namespace {
 
 constexpr int kPointsPerBlock = 128;  // 16 elements
-// batches below this many elements run the operator one thread per point (enough threads to
-// fill the device), larger ones one thread per element (no LDS, sums in registers)
-constexpr int kPointOperatorBelow = 32768;
 constexpr int kElemsPerBlock = kPointsPerBlock / 8;
 
 struct PimyBatchArgs {
@@ -396,84 +393,20 @@ __device__ inline void element_point_diagonal(const Shape<double>& s, const Pimy
           }
 }
 
-// The operator (DIAG false) and its diagonal on the stored tangents: one thread per element, its
-// 8 points in order, each point's node terms added to the element's 24 values as they come
-// (element_operator_apply / _diagonal, element_operator.hpp:82-209). Registers only. COMM: some
-// parameter set has a committed-tangent term (betaKcomm with damping in the coefficients).
-template <bool DIAG, bool COMM>
-__global__ __launch_bounds__(128) void pimy_operator_kernel(PimyBatchArgs a) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= a.count) return;
-  double X[8], Y[8], Z[8];
-  int eq[24];
-  element_geometry(a, e, X, Y, Z, eq);
-  const PimyParams& p = a.params[a.param[e]];
-  double v[24];
-  if constexpr (!DIAG)
-    for (int k = 0; k < 24; ++k) v[k] = operator_input(a, eq, k);
-  double out[24];
-  for (int k = 0; k < 24; ++k) out[k] = 0.0;
-  double cK, c0, cc, cM;
-  operator_factors(p, a.k, cK, c0, cc, cM);
-#pragma unroll 1
-  for (int gp = 0; gp < 8; ++gp) {
-    Shape<double> s;
-    gauss_shape(X, Y, Z, gp, s);
-    if constexpr (!DIAG) {
-      // sigma = D_eff eps with D_eff's entries formed one at a time as effective_D forms them
-      double eps[6], sig[6], Dc[36];
-      if constexpr (COMM)
-        if (cc != 0.0) pimy_committed_tangent(p, a.C + static_cast<int64_t>(e) * 8 + gp, a.npts, Dc);
-      point_strain(s, v, eps);
-      for (int r = 0; r < 6; ++r) {
-        double sum = 0.0;
-        for (int c = 0; c < 6; ++c) {
-          const int lo = r < c ? r : c, hi = r < c ? c : r;
-          const int w = lo * 6 - lo * (lo - 1) / 2 + (hi - lo);  // packed upper triangle, row-major
-          double d = cK * a.tangent[tangent_at(a, e, gp, w)];
-          if (c0 != 0.0) d += c0 * initial_entry(p, r, c);
-          if constexpr (COMM)
-            if (cc != 0.0) d += cc * Dc[6 * r + c];
-          sum += d * eps[c];
-        }
-        sig[r] = sum;
-      }
-      double g[3] = {0, 0, 0};
-      if (cM != 0.0 && p.mass_type == 0)
-        for (int kk = 0; kk < 8; ++kk)
-          for (int q = 0; q < 3; ++q) g[q] += s.N[kk] * v[3 * kk + q];
-      for (int j = 0; j < 8; ++j) {
-        double fj[3];
-        node_force(s, sig, j, fj);
-        const double temp = s.N[j] * s.dvol * p.rho;
-        for (int q = 0; q < 3; ++q) {
-          out[3 * j + q] += fj[q];
-          if (cM != 0.0) out[3 * j + q] += cM * (temp * (p.mass_type == 0 ? g[q] : v[3 * j + q]));
-        }
-      }
-    } else {
-      double D[36], cMd;
-      effective_D(a, p, e, gp, D, cMd);
-      double de[24];
-      element_point_diagonal(s, p, D, cMd, eq, de);
-      for (int k = 0; k < 24; ++k) out[k] += de[k];
-    }
-  }
-  const size_t P = static_cast<size_t>(a.padded);
-  for (int k = 0; k < 24; ++k) a.slots[k * P + e] = out[k];
-}
-
-// The same for small batches, one thread per point (8 lanes per element), so that a batch of a
-// few hundred elements still runs thousands of threads: each point leaves its node terms in
-// LDS and the element's lanes add them in point order, a node each (the same sums as above). The
-// stored tangent is loaded ahead of the chain node -> equation -> x, and D_eff's entries are
-// formed where they are used, as above: 1,024 elements 20.5 -> 9 us, half of it the sums one lane
-// of eight used to walk.
-template <bool DIAG>
+// The operator (DIAG false) and its diagonal on the stored tangents (element_operator_apply /
+// _diagonal, element_operator.hpp:82-209), one thread per Gauss point (8 lanes per element), so that
+// a batch of a few hundred elements still runs thousands of threads and a large one has eight
+// times the loads in flight: each point leaves its node terms in LDS (MASS: the mass terms beside
+// them) and the element's lanes add them in point order, a node each. The stored tangent is loaded
+// ahead of the chain node -> equation -> x, and D_eff's entries are formed where they are used.
+// 512 elements with mass 10.8 -> 9.5 us since the terms a call does not have are left out; 64,000
+// elements 86 us, one element per thread with its points in turn 114. Registers are the
+// compiler's choice: held to two waves a SIMD it spills, 13 and 140 us.
+template <bool DIAG, bool MASS>
 __global__ __launch_bounds__(kPointsPerBlock) void pimy_point_operator_kernel(PimyBatchArgs a) {
   // per point: 8 nodes x (3 stiffness, 3 mass) or the 24 diagonal entries; odd stride: the lanes of
   // a wave write different banks
-  constexpr int W = DIAG ? 25 : 49;
+  constexpr int W = DIAG || !MASS ? 25 : 49, N = MASS ? 6 : 3;
   __shared__ double part[kPointsPerBlock][W];
   const int t = threadIdx.x;
   const int e = blockIdx.x * kElemsPerBlock + t / 8, gp = t % 8;
@@ -508,7 +441,7 @@ __global__ __launch_bounds__(kPointsPerBlock) void pimy_point_operator_kernel(Pi
         sig[r] = sum;
       }
       double g[3] = {0, 0, 0};
-      if (cM != 0.0 && p.mass_type == 0)
+      if (MASS && p.mass_type == 0)
         for (int kk = 0; kk < 8; ++kk)
           for (int q = 0; q < 3; ++q) g[q] += s.N[kk] * v[3 * kk + q];
       for (int j = 0; j < 8; ++j) {
@@ -516,8 +449,8 @@ __global__ __launch_bounds__(kPointsPerBlock) void pimy_point_operator_kernel(Pi
         node_force(s, sig, j, fj);
         const double temp = s.N[j] * s.dvol * p.rho;
         for (int q = 0; q < 3; ++q) {
-          mine[6 * j + q] = fj[q];
-          mine[6 * j + 3 + q] = cM != 0.0 ? cM * (temp * (p.mass_type == 0 ? g[q] : v[3 * j + q])) : 0.0;
+          mine[N * j + q] = fj[q];
+          if constexpr (MASS) mine[N * j + 3 + q] = cM != 0.0 ? cM * (temp * (p.mass_type == 0 ? g[q] : v[3 * j + q])) : 0.0;
         }
       }
     } else {
@@ -536,8 +469,9 @@ __global__ __launch_bounds__(kPointsPerBlock) void pimy_point_operator_kernel(Pi
     const double* c = part[t - gp + g];
     for (int q = 0; q < 3; ++q) {
       if constexpr (!DIAG) {
-        out[q] += c[6 * gp + q];
-        if (cM != 0.0) out[q] += c[6 * gp + 3 + q];
+        out[q] += c[N * gp + q];
+        if constexpr (MASS)
+          if (cM != 0.0) out[q] += c[N * gp + 3 + q];
       } else {
         out[q] += c[3 * gp + q];
       }
@@ -706,7 +640,7 @@ __global__ void tangent_to_f32_kernel(int64_t n, const double* __restrict__ t, f
 }
 
 // The FP32 operator on the stored tangents, for the inner solves of mixed-precision CG: one
-// thread per element as pimy_operator_kernel, its terms in the same order, with x, the
+// thread per element, its points in turn, its terms in the order above, with x, the
 // tangents, strains, stresses and sums in FP32. The geometry (Jacobian, shape derivatives,
 // dvol), the operator factors and the committed tangent are formed in FP64 and rounded once.
 template <bool COMM>
@@ -1068,24 +1002,22 @@ __global__ __launch_bounds__(128) void pimy_ssp_operator_kernel(PimyBatchArgs a)
 }
 
 // The operator (DIAG false) or its diagonal on the stored tangents into a.slots, element values
-// a * padded + e: one thread per point below kPointOperatorBelow elements, one per element above.
+// a * padded + e.
 template <bool DIAG>
 void launch_operator_slots(fx_batch* b, const PimyBatchArgs& a) {
   hipStream_t st = b->ctx->stream;
   if (b->ssp) {
     if (b->count > 0)
       hipLaunchKernelGGL(pimy_ssp_operator_kernel<DIAG>, dim3((b->count + 127) / 128), dim3(128), 0, st, a);
-  } else if (b->count > 0 && b->count < kPointOperatorBelow) {  // small: one thread per point
+  } else if (b->count > 0) {
+    // each set's cM is k.mass + k.damping alphaM
+    bool mass = a.k.mass != 0.0;
+    for (const PimyParams& q : b->host_pimy) mass |= a.k.damping * q.alphaM != 0.0;
     const dim3 grid((b->count + kElemsPerBlock - 1) / kElemsPerBlock);
-    hipLaunchKernelGGL((pimy_point_operator_kernel<DIAG>), grid, dim3(kPointsPerBlock), 0, st, a);
-  } else if (b->count > 0) {  // one element per thread
-    bool comm = false;
-    for (const PimyParams& q : b->host_pimy) comm |= a.k.damping * q.betaKcomm != 0.0;
-    const dim3 g((b->count + 127) / 128);
-    if (comm)
-      hipLaunchKernelGGL((pimy_operator_kernel<DIAG, true>), g, dim3(128), 0, st, a);
+    if (mass && !DIAG)
+      hipLaunchKernelGGL((pimy_point_operator_kernel<DIAG, !DIAG>), grid, dim3(kPointsPerBlock), 0, st, a);
     else
-      hipLaunchKernelGGL((pimy_operator_kernel<DIAG, false>), g, dim3(128), 0, st, a);
+      hipLaunchKernelGGL((pimy_point_operator_kernel<DIAG, false>), grid, dim3(kPointsPerBlock), 0, st, a);
   }
 }
 
