@@ -36,7 +36,7 @@ def box(nx, ny, nz, layers=1):
 CASES = {
     "one_element": lambda: box(1, 1, 1),                # 12 equations: one partial chunk
     "one_tile_and_a_cell": lambda: box(9, 8, 4, 2),     # one shared plane, a cut tile
-    "chunk_less_3": lambda: box(10, 2, 62),             # 2046 equations: no tile ends a chunk
+    "chunk_less_3": lambda: box(10, 2, 62),             # 6138 equations: six short of three chunks
     "chunk_plus": lambda: box(13, 9, 13, 3),            # 5460: the last chunk partly shared equations
     "tied": lambda: meshes.column(10),                  # tied sets behind the shared equations
     "general": lambda: meshes.distorted_box(6),
