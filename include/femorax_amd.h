@@ -185,7 +185,7 @@ typedef struct fx_batch_desc {
 #define FX_BATCH_COMPACT 128u /* stdBrick<PressureIndependMultiYield> batches: the compacted return map
                                  (compacted_kernels.hpp:85-202): an elastic predictor per Gauss point, the
                                  plastic points listed, one full update per listed point, the element
-                                 forces replayed from the stored results (same bits as the fused kernel) */
+                                 forces from the trial history they leave (same bits as one update per point) */
 
 int fx_batch_create(fx_ctx* ctx, const fx_batch_desc* desc, uint32_t flags, fx_batch** out);
 void fx_batch_destroy(fx_batch* b);
@@ -537,7 +537,7 @@ int fx_newmark(fx_batch* b, const fx_newmark_desc* d, double* u, double* v, doub
 #define FX_COLUMN_MIXED 1u    /* inner CG in FP32 on FP32 blocks, inside FP64 iterative refinement */
 #define FX_COLUMN_NO_GRAPH 2u /* launch the iteration kernels one by one instead of replaying a hipGraph */
 #define FX_COLUMN_WAVES(n) ((uint32_t)(n) << 8) /* register budget of the return-map kernels: at least n
-                                 waves per SIMD (3 or 4; 1: the compiler's choice); default 3 */
+                                 waves per SIMD (3 or 4; 1: the compiler's choice, the default) */
 #define FX_COLUMN_ONE_STREAM 8u /* the four solve sizes one after another on the pool's stream (default:
                                  forked onto four side streams so they overlap; one stream leaves the
                                  other hardware queues to co-running work) */
