@@ -15,6 +15,7 @@
 #include <cmath>
 #include <vector>
 
+#include "fx_cg_watch.hpp"
 #include "fx_internal.hpp"
 #include "fx_kernels.hpp"
 #include "fx_vecops.hpp"
@@ -271,8 +272,8 @@ int gmres64_solver(fx_batch* b, const fx_coeffs& k, const fx_solve_options& o, c
   };
   // until the device has written `cols` columns
   auto wait = [&](int cols) -> int {
-    for (uint64_t spins = 1; __atomic_load_n(ready, __ATOMIC_ACQUIRE) < cols; ++spins) {
-      if (spins % 4096) continue;
+    for (DeviceWait look; __atomic_load_n(ready, __ATOMIC_ACQUIRE) < cols;) {
+      if (!look.pause()) continue;
       const hipError_t q = hipStreamQuery(st);
       if (q == hipErrorNotReady) continue;
       FX_HIP(ctx, q);

@@ -3,8 +3,8 @@
 // ConjugateGradient::solve with Jacobi (src/solvers/cg.cpp:24-72, jacobi.cpp:10-26) with its
 // scalars kept on the device: each kernel reads a `done` flag and becomes a no-op once the
 // stop rule ||r|| <= max(rtol ||b||, atol) (cg.cpp:34, 60) or p.Ap <= 0 (cg.cpp:49-53) has
-// fired, so the host only polls every few iterations and the iterate is exactly the one the
-// reference stops at. Dot products follow VectorOps' order (vector_ops.cpp:19-64): chunks of
+// fired, so the host may queue iterations ahead of the progress the device reports
+// (fx_cg_watch.hpp) and the iterate is exactly the one the reference stops at. Dot products follow VectorOps' order (vector_ops.cpp:19-64): chunks of
 // 2048 entries, 64 lanes, lane l summing entries l, l+64, ...; lane sums in lane order; chunk
 // sums reduced level by level. They accumulate in FP64 whatever the vector type.
 //
@@ -18,6 +18,7 @@
 #include <mutex>
 #include <string>
 
+#include "fx_cg_watch.hpp"
 #include "fx_internal.hpp"
 #include "fx_kernels.hpp"
 #include "fx_vecops.hpp"
@@ -525,11 +526,6 @@ hipGraphExec_t cg_solve_graph(fx_ctx* ctx, int64_t n, const CgVectors<T>& v, dou
   return cg_graph(ctx, key, [&](int i) -> int { return cg_iteration<T>(ctx, n, op, v, i, i + 1 == kGraphIters); });
 }
 
-// Iterations queued beyond the last one the device has reported: enough to hide the host's launch
-// times, and the only iterations that run as no-ops after the stop (four launches each; polling
-// by copies in groups of up to 64 iterations ran 30 of them on average).
-constexpr int kQueueAhead = 8;
-
 // The CG iterations on the device after cg_setup: the host launches them while it watches the
 // solve's mirror. With graphs on, each group replays a captured graph of kGraphIters iterations
 // (the same kernels and arguments, so the same bits as launching them).
@@ -537,7 +533,6 @@ template <typename T>
 int cg_device(fx_ctx* ctx, int64_t n, const BatchOp<T>& op, const T* inv, const T* b, T* x, T* r, T* z, T* p, T* p2,
               T* ap, CgState* st, double rtol, double atol, int max_it, const int32_t* zeros, CgMirror& host) {
   if (int rc = ensure_red(ctx, n)) return rc;
-  hipStream_t s = ctx->stream;
   // the mirror sits behind the dots' result in the context's pinned block
   CgMirror* mirror = reinterpret_cast<CgMirror*>(static_cast<char*>(ctx->host_pinned) + 256);
   __atomic_store_n(&mirror->it, 0, __ATOMIC_RELAXED);
@@ -545,31 +540,37 @@ int cg_device(fx_ctx* ctx, int64_t n, const BatchOp<T>& op, const T* inv, const 
   const CgVectors<T> v{inv, b, x, r, z, p, p2, ap, st, ctx->red, mirror};
   if (int rc = cg_setup<T>(ctx, n, op, v, rtol, atol, max_it, zeros)) return rc;
   hipGraphExec_t exec = cg_solve_graph<T>(ctx, n, v, rtol, atol, max_it, op);
-  const int group = exec ? kGraphIters : 1;
-  int launched = 0;
-  for (uint64_t spins = 0; !__atomic_load_n(&mirror->done, __ATOMIC_ACQUIRE);) {
-    if (launched < max_it && launched - __atomic_load_n(&mirror->it, __ATOMIC_RELAXED) < kQueueAhead + group - 1) {
+  struct Device {  // cg_watch's device: this solve
+    fx_ctx* ctx;
+    CgMirror* mirror;
+    hipGraphExec_t exec;
+    const CgVectors<T>& v;
+    const BatchOp<T>& op;
+    int64_t n;
+    int max_it;
+    int it() const { return __atomic_load_n(&mirror->it, __ATOMIC_RELAXED); }
+    bool done() const { return __atomic_load_n(&mirror->done, __ATOMIC_ACQUIRE) != 0; }
+    int launch(int i) {
       if (exec) {
-        FX_HIP(ctx, hipGraphLaunch(exec, s));
-      } else {
-        if (int rc = cg_iteration<T>(ctx, n, op, v, launched, launched + 1 == max_it)) return rc;
-        FX_HIP(ctx, hipGetLastError());
+        FX_HIP(ctx, hipGraphLaunch(exec, ctx->stream));
+        return FX_OK;
       }
-      launched += group;
-      spins = 0;
-      continue;
+      if (int rc = cg_iteration<T>(ctx, n, op, v, i, i + 1 == max_it)) return rc;
+      FX_HIP(ctx, hipGetLastError());
+      return FX_OK;
     }
-    if (++spins % 4096 == 0) {  // the queued work has ended without a stop: a device error
-      const hipError_t q = hipStreamQuery(s);
-      if (q == hipErrorNotReady) continue;
-      FX_HIP(ctx, q);
-      if (__atomic_load_n(&mirror->done, __ATOMIC_ACQUIRE)) break;
-      if (launched >= max_it || __atomic_load_n(&mirror->it, __ATOMIC_RELAXED) < launched) {
-        ctx->error = "CG: the device did not report the queued iterations";
-        return FX_EDEVICE;
-      }
+    int idle(bool& is) {
+      const hipError_t q = hipStreamQuery(ctx->stream);
+      is = q == hipSuccess;
+      if (q != hipErrorNotReady) FX_HIP(ctx, q);
+      return FX_OK;
     }
-  }
+    int stalled() {
+      ctx->error = "CG: the device did not report the queued iterations";
+      return FX_EDEVICE;
+    }
+  } dev{ctx, mirror, exec, v, op, n, max_it};
+  if (int rc = cg_watch(dev, max_it, exec ? kGraphIters : 1)) return rc;
   host = *mirror;
   return FX_OK;
 }

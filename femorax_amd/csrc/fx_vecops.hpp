@@ -99,8 +99,9 @@ struct CgState {
   int32_t it, done, converged, indefinite, max_it, zeros;
 };
 
-// The host's copy of a solve's progress, in pinned memory: the device writes `it` after each
-// iteration and, last of all, `done`, so the host neither copies nor synchronises to poll.
+// The host's copy of a solve's progress, in pinned memory: the kernel that takes the stop test after
+// an iteration writes `it` (direction_kernel, or the next iteration's tiles where they form the
+// direction) and, last of all, `done`, so the host neither copies nor synchronises to poll.
 struct CgMirror {
   double rhs_norm, init_res, final_res;
   int32_t it, converged, indefinite, zeros, done, pad;
