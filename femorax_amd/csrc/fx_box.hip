@@ -632,9 +632,11 @@ __global__ __launch_bounds__(kTileThreads) void hex8_box_cg_kernel(BoxArgs<T> a,
   __shared__ T top[3 * G::kRing * kPlane];
   __shared__ double row[2][kLanes];
   __shared__ double tot[2];
+  __shared__ int32_t stopped;  // one thread reads the flag: another workgroup may be setting it (cg_decide)
   const int t = threadIdx.x, wave = t / kLanes, l = t % kLanes;
   const int tile = blockIdx.x;
-  const int stopped = d.st->done, it = d.st->it, max_it = d.st->max_it;
+  const int it = d.st->it, max_it = d.st->max_it;
+  const int done = t == 0 ? d.st->done : 0;
   const double rz = d.st->rz, tol = d.st->tol;
   TileFetch<T, TZ> f;
   T q[G::kRounds][3];
@@ -656,9 +658,10 @@ __global__ __launch_bounds__(kTileThreads) void hex8_box_cg_kernel(BoxArgs<T> a,
   if (wave < 2) {
     const double s = wave_total(d.part, 2, wave, d.npart, l, row[wave]);
     if (l == 0) tot[wave] = s;
+    if (t == 0) stopped = done;
   }
-  if (stopped) return;
   __syncthreads();
+  if (stopped) return;
   double beta;
   if (!cg_decide(d.st, d.mirror, it, max_it, tol, rz, tot[0], tot[1], tile == 0 && t == 0, beta)) return;
   const T bt = static_cast<T>(beta);

@@ -244,10 +244,12 @@ template <typename T>
 __global__ __launch_bounds__(kVecThreads) void direction_kernel(int64_t n, CgDirection<T> d) {
   __shared__ double row[2][kLanes];
   __shared__ double tot[2];
+  __shared__ int32_t stopped;  // one thread reads the flag: another workgroup may be setting it (cg_decide)
   const int64_t begin = static_cast<int64_t>(blockIdx.x) * kChunk;
   const int len = static_cast<int>(n - begin < kChunk ? n - begin : kChunk);
   const int t = threadIdx.x, w = t / kLanes, l = t % kLanes;
-  const int stopped = d.st->done, it = d.st->it, max_it = d.st->max_it;
+  const int it = d.st->it, max_it = d.st->max_it;
+  const int done = t == 0 ? d.st->done : 0;
   const double rz = d.st->rz, tol = d.st->tol;
   T zv[kPerThread], pv[kPerThread];
 #pragma unroll
@@ -260,9 +262,10 @@ __global__ __launch_bounds__(kVecThreads) void direction_kernel(int64_t n, CgDir
   if (w < 2) {
     const double s = wave_total(d.part, 2, w, d.npart, l, row[w]);
     if (l == 0) tot[w] = s;
+    if (t == 0) stopped = done;
   }
-  if (stopped) return;
   __syncthreads();
+  if (stopped) return;
   double beta;
   if (!cg_decide(d.st, d.mirror, it, max_it, tol, rz, tot[0], tot[1], blockIdx.x == 0 && t == 0, beta)) return;
 #pragma unroll
