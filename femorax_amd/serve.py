@@ -162,7 +162,7 @@ class BlockWorker(threading.Thread):
                     self.inbox.put(None)
             t = time.perf_counter()
             for q in batch:
-                q.start = t
+                q.start, q.result = t, None
             try:
                 if ctx is None:
                     raise RuntimeError(f"no device context: {self.error!r}")
@@ -173,7 +173,8 @@ class BlockWorker(threading.Thread):
             except Exception as e:  # noqa: BLE001 - the requests fail, the worker goes on
                 self.error = e
                 for q in batch:
-                    q.result = {"error": repr(e)}
+                    if q.result is None:  # a round's earlier parts have their results
+                        q.result = {"error": repr(e)}
             t = time.perf_counter()
             for q in batch:
                 q.end = t
@@ -224,9 +225,7 @@ class BlockWorker(threading.Thread):
                 x.zero()
             res = core.cg_many(ctx, [g[0] for g in got], [g[1] for g in got], [g[2] for g in got], rtol=self.rtol)
             for r, g, rr in zip(now, got, res):
-                r.result = dict(rr)
-                if self.keep_x:
-                    r.result["x"] = g[2].get()
+                r.result = dict(rr, x=g[2].get()) if self.keep_x else dict(rr)
             rs = later
 
     def _solve(self, ctx, resident, r):
@@ -236,9 +235,7 @@ class BlockWorker(threading.Thread):
             res = batch.cg_mixed(b, x, rtol=self.rtol, inner_rtol=self.inner_rtol)
         else:
             res = batch.cg(b, x, rtol=self.rtol)
-        r.result = dict(res)
-        if self.keep_x:
-            r.result["x"] = x.get()
+        r.result = dict(res, x=x.get()) if self.keep_x else dict(res)
 
 
 def _block_bytes(neq, mixed):

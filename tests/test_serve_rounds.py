@@ -1,6 +1,7 @@
 """Block admission rounds under a small budget (host logic only): a round's own batches stay
 resident until its solves have run; blocks that do not fit beside them follow."""
 import collections
+import queue
 
 from femorax_amd import serve
 
@@ -65,3 +66,41 @@ def test_a_round_does_not_evict_its_own_blocks(monkeypatch):
         w._solve_round(None, resident, rs)
         assert calls == groups
         assert [r.result["iterations"] for r in rs] == [4, 5, 6, 7]
+
+
+def test_a_failed_part_leaves_the_solved_results(monkeypatch):
+    """A round of two parts whose second solve fails: the first part's requests keep their results."""
+    def cg_many(ctx, batches, bs, xs, rtol):
+        if any(b.n >= 6 for b in batches):
+            raise RuntimeError("no room")
+        return [dict(converged=1, iterations=b.n) for b in batches]
+
+    class Array(Handle):
+        def __init__(self, ctx, n):
+            super().__init__(n)
+
+        @classmethod
+        def from_host(cls, ctx, a):
+            return cls(ctx, a)
+
+    class Problems:
+        def get(self, n):
+            return {}, Mesh(n), n
+
+    class Request:
+        def __init__(self, n):
+            self.n, self.result, self.start, self.end = n, {"of": "an earlier run"}, None, None
+
+    monkeypatch.setattr(serve.core, "Context", lambda device: Handle(device))
+    monkeypatch.setattr(serve.core, "Batch", lambda ctx, mesh, params, **kw: Handle(mesh.neq))
+    monkeypatch.setattr(serve.core, "DeviceArray", Array)
+    monkeypatch.setattr(serve.core, "cg_many", cg_many)
+    monkeypatch.setattr(serve, "_block_bytes", lambda neq, mixed: 10)
+    inbox, done = queue.Queue(), queue.Queue()
+    rs = [Request(n) for n in (4, 5, 6, 7)]
+    for r in (*rs, None):
+        inbox.put(r)
+    serve.BlockWorker(0, Problems(), inbox, done, budget=25, mixed=False, rounds=True).run()
+    assert [done.get_nowait() for _ in rs] == rs
+    assert [r.result.get("iterations") for r in rs] == [4, 5, None, None]
+    assert ["error" in r.result for r in rs] == [False, False, True, True]
