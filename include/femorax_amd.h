@@ -595,7 +595,9 @@ int fx_column_pool_create(fx_ctx* ctx, const fx_column_pool_desc* d, fx_column_p
 void fx_column_pool_destroy(fx_column_pool* p);
 /* Admits a column at rest (u = v = a = 0, histories at their initial state) and starts its
  * first step; *id names it until fx_column_remove. FX_EFULL when the pool lacks element slots,
- * materials, record space or a column slot now. */
+ * materials, record space or a column slot now. The caller's arrays have been read on return; the
+ * device's part is queued on the context's stream, so that a device failure in it is reported by
+ * the next call that waits (fx_column_run, fx_column_status, fx_column_fetch). */
 int fx_column_add(fx_column_pool* p, const fx_column_desc* d, int32_t* id);
 /* Runs `iterations` Newton iterations of every running column (asynchronous columns: a column
  * that converges commits, records and predicts its next step within the same iteration);
@@ -610,7 +612,8 @@ int fx_column_finished(fx_column_pool* p, int32_t* ids, int32_t cap, int32_t* co
 int fx_column_fetch(fx_column_pool* p, int32_t id, double* u, double* v, double* a, double* history);
 /* The column's committed histories [FX_PIMY_NSTATE * nelem], field-major (host). */
 int fx_column_state(fx_column_pool* p, int32_t id, double* state);
-/* Frees the column's slots (a running column is stopped). */
+/* Frees the column's slots (a running column is stopped); queued on the context's stream, as
+ * fx_column_add. */
 int fx_column_remove(fx_column_pool* p, int32_t id);
 
 /* Node recorders (exec/recorders.hpp:5-20; recorders.cpp:193-240, 272-298): OpenSees'
