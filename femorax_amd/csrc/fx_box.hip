@@ -1146,7 +1146,8 @@ int resident_tiles(fx_ctx* ctx, const void* kernel) {
 
 // Up to this many tiles (one launch's worth of resident workgroups) the words of a tile's interior
 // nodes are loaded, not computed from the header's base: the header is one more round of memory
-// latency before the gathers, and the bytes it saves do not matter there.
+// latency before the gathers, and the bytes it saves do not matter there. It is the CG's tiles that
+// gain; the plain product is the same either way (GMRES at 16^3 to 96^3, within 0.5 %).
 constexpr int kFewTiles = 1024;
 
 template <typename T>
@@ -1317,8 +1318,14 @@ int launch_box_force(fx_batch* b, const double* u, const double* v, double vscal
 bool box_sums_with_dot(const fx_batch* b) {
   return b->lattice && !b->pimy && b->norphans == 0 && !b->nodal_m && !b->nodal_am;
 }
+// 25 iterations, us each, formed by the tiles against the pass of its own (8-deep tiles, as the
+// autotune chooses here): 16^3 22.2 / 23.5, 48^3 29.0 / 29.9, 64^3 (397 chunks) 38.8 / 38.8, 72^3 (563)
+// 48.8 / 50.0, 76^3 (661) 57.4 / 55.1, 88^3 (1,022) 76.1 / 74.1; FP32 crosses at the same place.
+// Past kFewTiles a tile waits for its header before both gathers: 4-deep tiles at 68^3 (1,377 of
+// them) 45.9 / 43.8, FP32 37.5 / 34.7.
+constexpr int64_t kDirectionChunks = 600;
 bool box_forms_direction(const fx_batch* b) {
-  return box_sums_with_dot(b) && b->tile_z != 16 && chunks(b->neq) <= kInlineParts;
+  return box_sums_with_dot(b) && b->tile_z != 16 && chunks(b->neq) <= kDirectionChunks && b->ntiles <= kFewTiles;
 }
 
 template <typename T>

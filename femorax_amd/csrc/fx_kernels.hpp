@@ -65,10 +65,8 @@ bool elements_damp(const fx_batch* b);
 // tile launch and one that adds the shared nodes' partial sums (solver numbering); and in front
 // of it, where d.z is given, the stop test and the direction p = z + beta p_old, formed as the
 // tiles fetch it. box_sums_with_dot: the batches it takes (the product is the elements' alone).
-// box_forms_direction: those whose direction it forms: 4- and 8-deep tiles, few enough equations
-// that every tile adds up r.r and r.z itself. At 13,872 equations that saves a launch (3.7 us of
-// 24 us an iteration); at 6.4 M the second gather costs more than the pass it saves (75 + 32
-// against 21 + 52 + 28 us).
+// box_forms_direction: those whose direction it forms: few enough equations that the launch it saves
+// is worth the tiles' second gather, and every tile adds up r.r and r.z itself.
 template <typename T>
 struct CgDirection;
 bool box_sums_with_dot(const fx_batch* b);
