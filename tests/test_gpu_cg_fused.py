@@ -133,3 +133,92 @@ def test_gmres_steps_match_oracle(ctx, name):
     _, ro = om.gmres(op, b, rtol=0.3)
     assert r["converged"] and r["iterations"] == ro["iterations"]
     batch.close()
+
+
+def graded(model):
+    """The planes in z moved apart towards the top: a rectilinear lattice."""
+    z = model["xyz"][:, 2]
+    model["xyz"][:, 2] = z * (1.0 + 0.4 * z / z.max())
+    return model
+
+
+def form_of(form, model):
+    """Three layers with stiffness and mass damping, the second with lumped mass, and the element."""
+    model = graded(model) if form == "graded" else model
+    model["region"] = model["group"].copy()
+    model["rayleigh"] = [(0.6 + 0.1 * g, 5.8e-4, 1e-4 * (g % 2), 2e-5) for g in range(3)]
+    for g, p in enumerate(model["params"]):
+        p["mass_type"] = g % 2
+    pm = core.Mesh(model)
+    element = "SSPbrick" if form == "ssp" else "stdBrick"
+    return model, pm, [dict(p, element=element) for p in pm.params_for(model)], element
+
+
+# every group of the product's instantiations: uniform stdBrick (16-deep tiles take the direction
+# given), SSPbrick and rectilinear, at each tile depth; 19 x 10 x 21 cells cut the last tiles of
+# every axis and depth
+FORMS = [("box", 4), ("box", 8), ("box", 16), ("ssp", 4), ("ssp", 8), ("graded", 4), ("graded", 8)]
+OPERATORS = {"K": (1.0, 0.0, 0.0), "KCM": (1.0, 20.0, 4e4)}
+
+
+@pytest.mark.parametrize("op_name", sorted(OPERATORS))
+@pytest.mark.parametrize("form,depth", FORMS)
+def test_every_form_matches_oracle(ctx, form, depth, op_name):
+    model, pm, params, element = form_of(form, box(19, 10, 21, 3))
+    batch = core.Batch(ctx, pm, params, element=element, tile_depth=depth, tune=False)
+    assert batch.info()["lattice"] == 1 and batch.info()["tiles"] == 6 * -(-21 // depth)
+    om, op = fxo.OracleMesh(model), fxo.elastic_params(params)
+    k = OPERATORS[op_name]
+    b = meshes.random_vector(pm.neq, 5)
+    db, dx = core.DeviceArray.from_host(ctx, b), core.DeviceArray(ctx, pm.neq)
+    for its in (1, 2, 12):
+        dx.zero()
+        r = batch.cg(db, dx, rtol=0.0, max_it=its, k=core.coeffs(*k))
+        xo, ro = om.cg(op, b, rtol=0.0, max_it=its, lanes=64, k=fxo.coeffs(*k))
+        assert r["iterations"] == ro["iterations"] == its
+        assert np.max(np.abs(dx.get() - xo)) <= 1e-11 * np.max(np.abs(xo)), its
+    batch.close()
+
+
+@pytest.mark.parametrize("op_name", sorted(OPERATORS))
+@pytest.mark.parametrize("form,depth", FORMS)
+def test_every_form_in_fp32(ctx, form, depth, op_name):
+    """The inner solve of the mixed CG stopped after a few iterations, before it can correct itself: an
+    FP32 product is within 2e-6 of its largest entry (the operator tests' bound), carried on with the
+    iteration count squared. A wrong direction entry is of the order of x."""
+    model, pm, params, element = form_of(form, box(19, 10, 21, 3))
+    batch = core.Batch(ctx, pm, params, element=element, tile_depth=depth, tune=False, fp32=True)
+    om, op = fxo.OracleMesh(model), fxo.elastic_params(params)
+    k = OPERATORS[op_name]
+    b = meshes.random_vector(pm.neq, 5)
+    db, dx = core.DeviceArray.from_host(ctx, b), core.DeviceArray(ctx, pm.neq)
+    for its in (1, 2, 5):
+        dx.zero()
+        r = batch.cg_mixed(db, dx, rtol=1e-30, inner_rtol=1e-20, max_it=its, k=core.coeffs(*k))
+        assert r["iterations"] == its and r["outer_iterations"] == 1
+        xo, _ = om.cg(op, b, rtol=0.0, max_it=its, lanes=64, k=fxo.coeffs(*k))
+        assert np.max(np.abs(dx.get() - xo)) <= 2e-6 * its * its * np.max(np.abs(xo)), its
+    batch.close()
+
+
+@pytest.mark.parametrize("fp32", [False, True], ids=["fp64", "fp32"])
+def test_direction_by_its_own_pass(ctx, fp32):
+    """More chunks than the tiles form the direction for (600), few enough that the pass adds their
+    partials up itself."""
+    model = box(70, 70, 90)
+    pm = core.Mesh(model)
+    assert 600 * 2048 < pm.neq < 1024 * 2048
+    params = pm.params_for(model)
+    batch = core.Batch(ctx, pm, params, tune=False, fp32=fp32)
+    om, op = fxo.OracleMesh(model, coloring=False), fxo.elastic_params(params)
+    b = np.resize(meshes.random_vector(10007, 3), pm.neq)
+    db, dx = core.DeviceArray.from_host(ctx, b), core.DeviceArray(ctx, pm.neq)
+    dx.zero()
+    if fp32:
+        r = batch.cg_mixed(db, dx, rtol=1e-30, inner_rtol=1e-20, max_it=3)
+    else:
+        r = batch.cg(db, dx, rtol=0.0, max_it=3)
+    xo, _ = om.cg(op, b, rtol=0.0, max_it=3, lanes=64, nthreads=8)
+    assert r["iterations"] == 3
+    assert np.max(np.abs(dx.get() - xo)) <= (2e-6 * 9 if fp32 else 1e-12) * np.max(np.abs(xo))
+    batch.close()
