@@ -1322,7 +1322,8 @@ bool box_sums_with_dot(const fx_batch* b) {
 // autotune chooses here): 16^3 22.2 / 23.5, 48^3 29.0 / 29.9, 64^3 (397 chunks) 38.8 / 38.8, 72^3 (563)
 // 48.8 / 50.0, 76^3 (661) 57.4 / 55.1, 88^3 (1,022) 76.1 / 74.1; FP32 crosses at the same place.
 // Past kFewTiles a tile waits for its header before both gathers: 4-deep tiles at 68^3 (1,377 of
-// them) 45.9 / 43.8, FP32 37.5 / 34.7.
+// them) 45.9 / 43.8, FP32 37.5 / 34.7, with mass terms 48.7 / 50.7 (SSPbrick and graded 49.0 / 48.0,
+// 52.3 / 51.4).
 constexpr int64_t kDirectionChunks = 600;
 bool box_forms_direction(const fx_batch* b) {
   return box_sums_with_dot(b) && b->tile_z != 16 && chunks(b->neq) <= kDirectionChunks && b->ntiles <= kFewTiles;

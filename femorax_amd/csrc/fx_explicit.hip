@@ -2,14 +2,16 @@
 // ExplicitDifference loops.
 //
 // For ElasticIsotropic the element force is linear: f = K u + C v - F_body (std_brick.hpp:
-// 493-543 with element_operator's Factors), so the force runs on the operator kernels (K u,
-// and C v with the operator coefficients (0, 1, 0)) plus a combine kernel; F_body is a vector
-// built once per batch. The CentralDifference step (explicit_analysis.cpp:87-117, 712-722)
-// is one device-resident loop: per step the garbage velocity v_e = -c2 u(n-1) (only when the
-// elements damp), the force, the point loads, and one fused update per equation that forms
-// R = -f - M a_g + P, solves the diagonal system (c3 M + c2 C) U = R and writes U, the recorded
-// velocity and acceleration. U goes into u(n-1)'s buffer and the two buffers swap roles, so the
-// update writes 3 vectors, not 4. ExplicitDifference (explicit_analysis.cpp:60-85) runs its
+// 493-543 with element_operator's Factors). stdBrick lattices of 4- and 8-deep tiles form it in one
+// tile pass (launch_box_force); the others run the operator kernels (K u, and C v with the operator
+// coefficients (0, 1, 0)) plus a combine kernel, with F_body a vector built once per batch. The
+// CentralDifference step (explicit_analysis.cpp:87-117, 712-722) is one device-resident loop:
+// per step the force at the garbage velocity v_e = -c2 u(n-1) (where the elements damp), the
+// point loads, and one update per equation that forms R = -f - M a_g + P, solves the diagonal
+// system (c3 M + c2 C) U = R and writes U and, where they are asked for, the recorded velocity
+// and acceleration: inside the tile pass on a lattice (up to kStepLoads point loads, no nodal
+// damping), else in kernels of their own. U goes into u(n-1)'s buffer and the two buffers swap
+// roles, so the update writes 3 vectors, not 4. ExplicitDifference (explicit_analysis.cpp:60-85) runs its
 // predictor, the force at the predicted velocity and one fused update (a = R / m, the recorded
 // velocity). Both add the ground-motion load of a uniform excitation (:48-58).
 #include <hip/hip_runtime.h>

@@ -3,7 +3,8 @@
     python femorax_amd/profile_kernels.py general N REPS   general-geometry operator (hex8_block_kernel) on a
                                                              distorted N^3 layered box, FP64 and FP32 applies
     python femorax_amd/profile_kernels.py pimy SIDE REPS   stdBrick<PressureIndependMultiYield> force at a yielding
-                                                             state (pimy_batch_kernel) on the SIDE^3 reference column
+                                                             state (pimy_trial_kernel, pimy_force_kernel) on the
+                                                             SIDE^3 reference column
     python femorax_amd/profile_kernels.py pimy_time SIDE REPS   wall time per force call (every kernel of the call) on
                                                              the same column, elastic and yielding, fused and compacted
                                                              (pimy_time_damped: with the column's Rayleigh damping at
